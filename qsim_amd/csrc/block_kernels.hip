@@ -100,7 +100,7 @@ GateBlockKernel(float2* __restrict__ s, BlockGeom g, BlockProgram p,
   for (int w = 0; w < kRingQuads; ++w) {
     ring4[threadIdx.x + NT * w] = gfrag[threadIdx.x + NT * w];
   }
-  TileIo<PER, NT> io;
+  TileIo<PER, NT, false> io;
   io.Init(g);
   unsigned k = 0;  // ops run so far: the current op's slot is k % 2
   // Op `op` on the tile in LDS; `extra` runs once op nxt's record loads are
@@ -187,16 +187,18 @@ GateBlockKernel(float2* __restrict__ s, BlockGeom g, BlockProgram p,
   }
 }
 
-// The FP16-with-scaling pass (block_tile.h).  Every op record of the pass
-// is copied to LDS once per workgroup, so the ops issue no global loads:
+// The FP16-with-scaling pass (block_tile.h) over tiles of up to 13 qubits
+// (14: GateBlockF16IoKernel).  Every op record of the pass is copied to LDS
+// once per workgroup, so the ops issue no global loads:
 // the only vector memory operations are the tile's loads and stores, and
 // the wait for the next tile's loads (issued in full at the start of the
 // current tile's ops) never stands behind a record fetch issued after the
 // previous tile's stores.  The stores of a tile drain while the next
 // tile's ops run.  Measured on MI355X, an op costs about 2 ms per 32-qubit
 // pass whatever the HBM traffic: rewriting the tile in LDS (8-byte LDS
-// writes run at half the read rate) bounds it, not the MFMA or VALU work.  The tile is scaled by 2^e when staged and by 2^-e when
-// stored (TileScale, exact); one more barrier per tile for the maximum.
+// writes run at half the read rate) bounds it, not the MFMA or VALU work.  The tile is scaled by 2^e when
+// staged and by 2^-e when stored (TileScale, exact); one more barrier per
+// tile for the maximum.
 template <int TB, bool FULL>
 __global__ void __launch_bounds__(BlockShape<TB>::NT)
 __attribute__((amdgpu_waves_per_eu(2)))
@@ -220,7 +222,7 @@ GateBlockF16Kernel(float2* __restrict__ s, BlockGeom g, BlockProgram p,
     uint4* dst = reinterpret_cast<uint4*>(rec);
     for (unsigned q = threadIdx.x; q < nq; q += NT) dst[q] = src[q];
   }
-  TileIo<PER, NT> io;
+  TileIo<PER, NT, true> io;
   io.Init(g);
   float2 buf[PER];
   uint64_t tile = PairedTile(blockIdx.x, gridDim.x);
@@ -244,16 +246,9 @@ GateBlockF16Kernel(float2* __restrict__ s, BlockGeom g, BlockProgram p,
     const uint64_t nb = InsertZeros(next << g.Lc, g.outer, g.nouter);
     io.template Fetch<FULL, 3u>(s, nb, g, buf);
     for (unsigned op = 0; op < p.nops; ++op) {
-      const uint32_t* r = rec + op * unsigned(kF16RecWords);
-      v8h f[4];
-      LoadFragF16(r, l, f);
-      const uint32_t* tab = r + kF16TabOff + 16 * (l >> 5);
-      const uint32_t sj = r[kF16TabOff + kTableWords + (l & 31)];
-      uint32_t mo[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) mo[q] = tab[q] ^ sj;
-      ApplyTileOpF16(reinterpret_cast<const uint8_t*>(r + kF16BposOff), f,
-                     mo, nbatch, wave, NW);
+      F16Op o;
+      o.Load(rec + op * unsigned(kF16RecWords), l);
+      ApplyTileOpF16(o, nbatch, wave, NW);
       __syncthreads();
       if (op == 1) io.template Fetch<FULL, 12u>(s, nb, g, buf);
     }
@@ -265,8 +260,240 @@ GateBlockF16Kernel(float2* __restrict__ s, BlockGeom g, BlockProgram p,
   }
 }
 
+// The FP16 pass over 14-qubit tiles.  One 128 KiB tile fills a CU's LDS, so
+// no second workgroup can hide its HBM phases; the workgroup hides them
+// itself: 8 waves run the ops and 4 waves (one per SIMD) do nothing but move
+// tiles.  The IO waves hold a whole tile in registers (32 16-byte pairs a
+// thread).  While the ops of a tile run they issue, share by share, the
+// stores of the previous tile and, into the registers each store frees, the
+// loads of the next one; a wave that stalls on a full memory queue holds up
+// no op until the barrier that ends it.  Between two tiles they exchange the
+// tile in LDS for the one in registers.  Shares go out with all ops but the
+// last, whose time covers the last loads' latency.
+//
+// The tile is scaled as in GateBlockF16Kernel, but by the first op as it
+// reads (the maximum is known only once the loads have arrived, and the
+// exchange, which nothing overlaps, moves bits unchanged) and on the way out
+// by the stores.
+//
+// Bound by the HBM stream up to 5 ops, then by the ops (about 2.1 ms each:
+// LDS reads and writes of the whole tile, the fp16 split and the MFMA chain
+// in sequence).  32 qubits, tiles of 4 low and 10 random higher qubits, 1 / 3
+// / 5 / 7 ops: 15.4-16.0 / 15.4-15.9 / 16.0-16.2 / 20.3-20.4 ms, against
+// 16.3 / 16.0-17.5 / 18.7-20.1 / 23.2-24.2 with every wave doing both.  The
+// 64 KiB shape has two workgroups a CU, which hide each other's phases, and
+// keeps that structure.  The grid is one workgroup a CU: two or four in
+// turn measured the same, and cost a small state its overlap.
+constexpr unsigned kIoNT = 256;                       // 4 IO waves
+constexpr unsigned kIoThreads = BlockShape<14>::NT + kIoNT;
+
+// Pair i of IO thread t: tile-local amplitudes 2 t + 512 i and its
+// successor.  Positions 9 and up are never in the low run (PrepareGateBlock),
+// so i's bits are the tile's five highest qubits, h[0..4].
+struct TileIoPairs {
+  static constexpr int PER = (1 << 14) / (2 * kIoNT);  // 32 pairs a thread
+  uint64_t tofs;  // t's part of the offset in the state, amplitudes
+  uint64_t h[5];  // wave-uniform
+  unsigned unit;  // t's part of the 16-byte LDS unit
+
+  __device__ __forceinline__ void Init(const BlockGeom& g, unsigned t) {
+    const unsigned a = 2 * t;
+    tofs = (a & ((1u << g.Lc) - 1)) + DepositHigh(a >> g.Lc, g);
+#pragma unroll
+    for (int b = 0; b < 5; ++b) h[b] = g.hbit[9 - g.Lc + b];
+    unit = F16Swz(a) >> 1;
+  }
+  // Addresses of the four pairs 4 C .. 4 C + 3 of the tile at `base`.  The
+  // thread's part is hidden from the optimiser so that the 32 addresses are
+  // not kept in registers across the tile loop, where the pairs are.
+  template <int C>
+  __device__ __forceinline__ void At(float2* s, uint64_t base,
+                                     v4f* (&q)[4]) const {
+    uint64_t o = tofs;
+    asm volatile("" : "+v"(o));
+    uint64_t b = base;
+    if (C & 1) b += h[2];
+    if (C & 2) b += h[3];
+    if (C & 4) b += h[4];
+    float2* p = s + o;
+    q[0] = reinterpret_cast<v4f*>(p + b);
+    q[1] = reinterpret_cast<v4f*>(p + (b + h[0]));
+    q[2] = reinterpret_cast<v4f*>(p + (b + h[1]));
+    q[3] = reinterpret_cast<v4f*>(p + (b + h[0] + h[1]));
+  }
+  __device__ __forceinline__ unsigned Unit(int i) const {
+    unsigned u = unit;
+    asm volatile("" : "+v"(u));
+    return (u ^ ((F16Swz(512u * unsigned(i)) & 15u) >> 1)) +
+           256u * unsigned(i);
+  }
+};
+
+// Maximum of a non-negative value over the wave, in lane 63.
+__device__ __forceinline__ float WaveMaxTo63(float m) {
+  auto step = [&](auto ctrl) {
+    m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                     0, __builtin_bit_cast(int, m), decltype(ctrl)::value, 0xf,
+                     0xf, false)));
+  };
+  step(std::integral_constant<int, 0x111>{});  // row_shr:1, :2, :4, :8
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});  // row_bcast:15, :31
+  step(std::integral_constant<int, 0x143>{});
+  return m;
+}
+
+template <int N, typename F>
+__device__ __forceinline__ void Unrolled(F&& f) {
+  if constexpr (N > 0) {
+    Unrolled<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+__global__ void __launch_bounds__(kIoThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3)))
+GateBlockF16IoKernel(float2* __restrict__ s, BlockGeom g, BlockProgram p,
+                     const uint32_t* __restrict__ recs) {
+  constexpr int NW = BlockShape<14>::kWaves;
+  constexpr int PER = TileIoPairs::PER;
+  constexpr int kShares = PER / 4;
+  extern __shared__ char lds_raw[];
+  v4f* lds4 = reinterpret_cast<v4f*>(lds_raw);
+  float* slots = reinterpret_cast<float*>(lds_raw + F16Lds<14>::kMaxOff);
+  uint32_t* rec = reinterpret_cast<uint32_t*>(lds_raw + F16Lds<14>::kRecOff);
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint64_t first = PairedTile(blockIdx.x, gridDim.x);
+  // The scale exponent of the tile whose wave maxima are in slots 4 par ...
+  auto scale_of = [&](unsigned par) {
+    const float* m = slots + 4 * par;
+    return __builtin_amdgcn_readfirstlane(ScaleExponent(
+        fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), p.headroom));
+  };
+  if (wave < unsigned(NW)) {
+    const int l = threadIdx.x & 63;
+    const unsigned nq = p.nops * unsigned(kF16RecWords / 4);
+    const uint4* src = reinterpret_cast<const uint4*>(recs);
+    uint4* dst = reinterpret_cast<uint4*>(rec);
+    for (unsigned q = threadIdx.x; q < nq; q += 64 * NW) dst[q] = src[q];
+    __syncthreads();
+    unsigned par = 0;
+    // An op's record is read while the op before it finishes.
+    F16Op o;
+    o.Load(rec, l);
+    auto run_op = [&](unsigned op, auto scale, int e) {
+      ApplyTileOpF16<decltype(scale)::value>(o, 32u, wave, NW, e);
+      o.Load(rec + (op + 1 < p.nops ? op + 1 : 0) * unsigned(kF16RecWords), l);
+      __syncthreads();
+    };
+    for (uint64_t tile = first; tile < g.ntiles; tile += gridDim.x) {
+      run_op(0, std::true_type{}, scale_of(par));
+      for (unsigned op = 1; op < p.nops; ++op) run_op(op, std::false_type{}, 0);
+      __syncthreads();
+      par ^= 1u;
+    }
+    return;
+  }
+  const unsigned t = threadIdx.x - 64u * NW;
+  TileIoPairs io;
+  io.Init(g, t);
+  v4f buf[PER];
+  auto load = [&](auto c, uint64_t base) {
+    constexpr int C = decltype(c)::value;
+    v4f* q[4];
+    io.At<C>(s, base, q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) buf[4 * C + i] = *q[i];
+  };
+  auto store = [&](auto c, uint64_t base, int e) {
+    constexpr int C = decltype(c)::value;
+    v4f* q[4];
+    io.At<C>(s, base, q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const v4f v = buf[4 * C + i];
+      *q[i] = v4f{ldexpf(v.x, -e), ldexpf(v.y, -e), ldexpf(v.z, -e),
+                  ldexpf(v.w, -e)};
+    }
+  };
+  // Waits for the loads; the maximum of this wave's values to its slot.
+  auto arrive = [&](unsigned par) {
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const v4f v = buf[i];
+      m = fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y));
+      m = fmaxf(fmaxf(m, fabsf(v.z)), fabsf(v.w));
+    }
+    m = WaveMaxTo63(m);
+    if ((t & 63u) == 63u) slots[4 * par + (t >> 6)] = m;
+  };
+  // At least one tile (the grid is no larger than the tiles).
+  uint64_t tile = first;
+  uint64_t base = InsertZeros(tile << g.Lc, g.outer, g.nouter);
+  Unrolled<kShares>([&](auto c) { load(c, base); });
+  arrive(0);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) lds4[io.Unit(i)] = buf[i];
+  __syncthreads();
+  unsigned par = 0;
+  uint64_t obase = 0;  // the finished tile in buf
+  int oe = 0;
+  const unsigned spread = p.nops > 1 ? p.nops - 1 : 1;
+  for (bool out = false;; out = true) {
+    const int e = scale_of(par);
+    const bool more = tile + gridDim.x < g.ntiles;
+    tile += gridDim.x;
+    const uint64_t nb =
+        more ? InsertZeros(tile << g.Lc, g.outer, g.nouter) : 0;
+    unsigned op = 0;
+    Unrolled<kShares>([&](auto c) {
+      constexpr unsigned C = decltype(c)::value;
+      // Share C goes out with op C spread / 8.
+      for (const unsigned due = C * spread / kShares; op < due; ++op)
+        __syncthreads();
+      if (out) store(c, obase, oe);
+      if (more) load(c, nb);
+    });
+    for (; op + 1 < p.nops; ++op) __syncthreads();
+    par ^= 1u;
+    if (more) arrive(par);
+    __syncthreads();
+    // The exchange: every slot of the tile belongs to one thread here.  The
+    // reads of one step are in flight while the step before is written.
+    constexpr int ST = 2;
+    v4f old[2][ST];
+    auto take = [&](auto c) {
+      constexpr int C = decltype(c)::value;
+#pragma unroll
+      for (int i = 0; i < ST; ++i) old[C & 1][i] = lds4[io.Unit(ST * C + i)];
+    };
+    take(std::integral_constant<int, 0>{});
+    Unrolled<PER / ST>([&](auto c) {
+      constexpr int C = decltype(c)::value;
+      if constexpr (C + 1 < PER / ST) take(std::integral_constant<int, C + 1>{});
+#pragma unroll
+      for (int i = 0; i < ST; ++i) {
+        if (more) lds4[io.Unit(ST * C + i)] = buf[ST * C + i];
+        buf[ST * C + i] = old[C & 1][i];
+      }
+    });
+    __syncthreads();
+    obase = base;
+    oe = e;
+    if (!more) break;
+    base = nb;
+  }
+  Unrolled<kShares>([&](auto c) { store(c, obase, oe); });
+}
+
 // TileSwz on the host (the slot of tile-local amplitude a).
 unsigned HostTileSwz(unsigned a) { return a ^ (((a >> 4) ^ (a >> 8)) & 15u); }
+unsigned HostSwz(unsigned a, bool f16) {
+  return f16 ? F16Swz(a) : HostTileSwz(a);
+}
 
 // x's low k bits placed at positions pos[0..k).
 unsigned Deposit(unsigned x, const unsigned* pos, unsigned k) {
@@ -283,8 +510,11 @@ unsigned Deposit(unsigned x, const unsigned* pos, unsigned k) {
 // over 32 four-byte banks), then the same over the half-wave (slot mod 32),
 // so that the op's LDS reads and writes are conflict-free where the
 // targets allow it.
-void ChooseLanePositions(const unsigned* pad, unsigned tb, unsigned* lane,
-                         unsigned* batch) {
+// An FP16 op with position 0 among its targets reads 16-byte units: the
+// same over units, 8 columns for 8 lanes and 16 for 16.
+void ChooseLanePositions(const unsigned* pad, unsigned tb, bool f16,
+                         unsigned* lane, unsigned* batch) {
+  const unsigned unit = f16 && pad[0] == 0 ? 1u : 0u;
   unsigned np = 0, nonk[kBlockMaxBits];
   for (unsigned q = 0; q < tb; ++q) {
     if (q != pad[0] && q != pad[1] && q != pad[2] && q != pad[3]) nonk[np++] = q;
@@ -310,10 +540,15 @@ void ChooseLanePositions(const unsigned* pad, unsigned tb, unsigned* lane,
             cand[3] = nonk[d];
             cand[4] = nonk[e];
             unsigned sl[32];
-            for (unsigned j = 0; j < 32; ++j) sl[j] = HostTileSwz(Deposit(j, cand, 5));
-            const unsigned score =
-                ((std::max(worst(sl, 16, 16), worst(sl + 16, 16, 16)) - 1) << 8) |
-                (worst(sl, 32, 32) - 1);
+            for (unsigned j = 0; j < 32; ++j)
+              sl[j] = HostSwz(Deposit(j, cand, 5), f16) >> unit;
+            const unsigned w = 16u >> unit;
+            unsigned quarter = 0, half = 0;
+            for (unsigned j = 0; j < 32; j += w)
+              quarter = std::max(quarter, worst(sl + j, w, w));
+            for (unsigned j = 0; j < 32; j += 2 * w)
+              half = std::max(half, worst(sl + j, 2 * w, 2 * w));
+            const unsigned score = ((quarter - 1) << 8) | (half - 1);
             if (score < best) {
               best = score;
               std::copy(cand, cand + 5, lane);
@@ -326,16 +561,17 @@ void ChooseLanePositions(const unsigned* pad, unsigned tb, unsigned* lane,
   for (; nb < kBlockMaxBits - 9; ++nb) batch[nb] = 0;
 }
 
-// ChooseLanePositions depends on the padded targets and tb alone (all below
-// 16), and a batch of trajectories repeats the same few thousand
+// ChooseLanePositions depends on the padded targets, tb (all below 16) and
+// the swizzle alone, and a batch of trajectories repeats the same few thousand
 // combinations across its passes: the choice is memoised per process.
-void LanePositions(const unsigned* pad, unsigned tb, unsigned* lane,
+void LanePositions(const unsigned* pad, unsigned tb, bool f16, unsigned* lane,
                    unsigned* batch) {
   constexpr unsigned kNb = kBlockMaxBits - 9;
   static std::mutex mu;
   static std::unordered_map<uint32_t, std::array<uint8_t, 5 + kNb>> memo;
   const uint32_t key =
-      pad[0] | (pad[1] << 4) | (pad[2] << 8) | (pad[3] << 12) | (tb << 16);
+      pad[0] | (pad[1] << 4) | (pad[2] << 8) | (pad[3] << 12) | (tb << 16) |
+      (f16 ? 1u << 24 : 0u);
   {
     std::lock_guard<std::mutex> lock(mu);
     auto it = memo.find(key);
@@ -345,7 +581,7 @@ void LanePositions(const unsigned* pad, unsigned tb, unsigned* lane,
       return;
     }
   }
-  ChooseLanePositions(pad, tb, lane, batch);
+  ChooseLanePositions(pad, tb, f16, lane, batch);
   std::array<uint8_t, 5 + kNb> v{};
   for (unsigned b = 0; b < 5; ++b) v[b] = uint8_t(lane[b]);
   for (unsigned b = 0; b < kNb; ++b) v[5 + b] = uint8_t(batch[b]);
@@ -520,6 +756,7 @@ int PrepareGateBlock(unsigned n, const unsigned* tile, unsigned nt,
   p = BlockProgram{};
   p.nops = nops;
   p.arith = unsigned(arith);
+  const bool f16 = arith == kBlockArithF16;
   const size_t kOpElems =  // uint16 per op record
       2 * size_t(arith == kBlockArithF16 ? kF16RecWords : kOpWords);
   fb.assign(std::max<size_t>(nops, 1) * kOpElems, 0);
@@ -580,17 +817,17 @@ int PrepareGateBlock(unsigned n, const unsigned* tile, unsigned nt,
         const unsigned rm = arith == kBlockArithF16
                                 ? F16Col(4 * h + 8 * (q >> 2) + (q & 3))
                                 : 4 * h + 8 * (q >> 2) + (q & 3);
-        tab[16 * h + q] = uint32_t(sizeof(float2)) * HostTileSwz(toff(rm));
+        tab[16 * h + q] = uint32_t(sizeof(float2)) * HostSwz(toff(rm), f16);
         tab[16 * h + 8 + q] = uint32_t(sizeof(float2)) *
-                              HostTileSwz(toff(2 * h + 4 * (q >> 1) + (q & 1)));
+                              HostSwz(toff(2 * h + 4 * (q >> 1) + (q & 1)), f16);
       }
     }
     // Group table: lane j's group has j's bits at the lane positions.
     unsigned lane[5], batch[kBlockMaxBits - 9];
-    LanePositions(pad, nt, lane, batch);
+    LanePositions(pad, nt, f16, lane, batch);
     for (unsigned j = 0; j < 32; ++j) {
       tab[kTableWords + j] =
-          uint32_t(sizeof(float2)) * HostTileSwz(Deposit(j, lane, 5));
+          uint32_t(sizeof(float2)) * HostSwz(Deposit(j, lane, 5), f16);
     }
     for (unsigned b = 0; b < kBlockMaxBits - 9; ++b) p.bpos[i][b] = uint8_t(batch[b]);
     uint32_t bw[2] = {0, 0};
@@ -599,7 +836,8 @@ int PrepareGateBlock(unsigned n, const unsigned* tile, unsigned nt,
       uint32_t r32[kF16RecWords];
       BuildRecF16(u16.data(), tab, r32);
       r32[kF16BposOff] = bw[0];
-      r32[kF16BposOff + 1] = bw[1];
+      // Position 0 a target: 16-byte accesses (F16Op).
+      r32[kF16BposOff + 1] = bw[1] | (pad[0] == 0 ? 256u : 0u);
       r32[kF16BposOff + 2] = 0;
       r32[kF16BposOff + 3] = 0;
       std::memcpy(rec, r32, sizeof(r32));
@@ -669,9 +907,9 @@ void LaunchF16(float2* s, const BlockGeom& g, const BlockProgram& p,
     const uint32_t* r = drec + size_t(c0) * kF16RecWords;
     if (g.tb == 14) {
       const uint64_t blocks =
-          std::min<uint64_t>(g.ntiles, uint64_t(NumCUs()) * 4);
-      hipLaunchKernelGGL((GateBlockF16Kernel<14, true>), dim3(unsigned(blocks)),
-                         dim3(BlockShape<14>::NT), F16Lds<14>::Bytes(q.nops),
+          std::min<uint64_t>(g.ntiles, uint64_t(NumCUs()));
+      hipLaunchKernelGGL(GateBlockF16IoKernel, dim3(unsigned(blocks)),
+                         dim3(kIoThreads), F16Lds<14>::Bytes(q.nops),
                          Stream(), s, g, q, r);
     } else {
       const uint64_t blocks =
@@ -718,7 +956,7 @@ int RunGateBlock(float2* s, const BlockGeom& g, const BlockProgram& p,
          F16Lds<13>::Bytes(F16Lds<13>::kMaxOps)},
         {reinterpret_cast<const void*>(&GateBlockF16Kernel<13, false>),
          F16Lds<13>::Bytes(F16Lds<13>::kMaxOps)},
-        {reinterpret_cast<const void*>(&GateBlockF16Kernel<14, true>),
+        {reinterpret_cast<const void*>(&GateBlockF16IoKernel),
          F16Lds<14>::Bytes(F16Lds<14>::kMaxOps)}};
     for (const auto& f : fns) {
       hipFuncAttributes fa{};

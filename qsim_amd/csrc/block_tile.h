@@ -70,6 +70,23 @@ __device__ __forceinline__ LdsV2f* LdsAt(unsigned b) {
   return reinterpret_cast<LdsV2f*>(size_t{b});
 }
 
+// Slot of amplitude a in the LDS tile of an FP16 pass: the 16-byte unit
+// a / 2 with the bits of a from position 4 up folded into its low three.
+// Position 0 stays where it is, so the two amplitudes of a pair are one
+// aligned 16-byte LDS access: an op with position 0 among its targets reads
+// and writes pairs (on MI355X 16-byte LDS reads run at ~192 B/clock per CU
+// against ~118 for 8-byte ones, writes at ~75 against ~64), and so does the
+// staging.  Each unit bit hashes four positions, so every other op finds
+// lane positions free of bank conflicts unless its targets are one whole
+// class.  Linear over GF(2).
+__host__ __device__ constexpr unsigned F16Swz(unsigned a) {
+  return a ^ ((((a >> 4) ^ (a >> 7) ^ (a >> 10) ^ (a >> 13)) & 7u) << 1);
+}
+template <bool F16>
+__device__ __forceinline__ unsigned BlockSwz(unsigned a) {
+  return F16 ? F16Swz(a) : TileSwz(a);
+}
+
 // One 4-qubit op over the LDS tile.  A group (the 16 amplitudes the op
 // mixes) is fixed by its bits at the tile's non-target positions; the host
 // splits those positions into 5 lane positions (chosen so that the 32
@@ -82,12 +99,13 @@ __device__ __forceinline__ LdsV2f* LdsAt(unsigned b) {
 // and member offsets occupy disjoint bits, so a member's slot is the XOR of
 // the three parts' swizzled slots: the batch part is scalar work and an
 // address is one XOR (the tile sits at LDS offset 0).
+template <bool F16 = false>
 __device__ __forceinline__ unsigned BatchSlot(unsigned bt,
                                               const unsigned (&b)[5]) {
   unsigned pb = 0;
 #pragma unroll
   for (int i = 0; i < 5; ++i) pb |= ((bt >> i) & 1u) << b[i];
-  return TileSwz(pb) * unsigned(sizeof(float2));
+  return BlockSwz<F16>(pb) * unsigned(sizeof(float2));
 }
 
 // Lane half h's 8 members of its group as bf16 (hi, lo) pairs.
@@ -344,67 +362,126 @@ __device__ __forceinline__ v16f MfmaChainF16(const v8h (&f)[4],
   return c;
 }
 
-// Results of a batch back to the slots its inputs came from: C registers
-// (4 q + 2 u, 4 q + 2 u + 1) are member index 2 q + u of the lane's list.
-__device__ __forceinline__ void WriteBack(const uint32_t (&a)[8],
-                                          const v16f& c) {
+// A lane's part of an FP16 op: its A fragments, its member offsets (record
+// column order, so that reads and writes share them) XOR its group's slot,
+// the batch-bit positions, and whether members 2 q and 2 q + 1 are the two
+// amplitudes of a 16-byte unit (position 0 is a target).
+struct F16Op {
+  v8h f[4];
+  uint32_t mo[8];
+  uint32_t bw[2];
+  bool pair;
+
+  __device__ __forceinline__ void Load(const uint32_t* r, int l) {
+    LoadFragF16(r, l, f);
+    const uint32_t* tab = r + kF16TabOff + 16 * (l >> 5);
+    const uint32_t sj = r[kF16TabOff + kTableWords + (l & 31)];
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 8; ++q) mo[q] = tab[q] ^ sj;
+    bw[0] = r[kF16BposOff];
+    bw[1] = r[kF16BposOff + 1];
+  }
+  // The wave-uniform part, in scalar registers.
+  __device__ __forceinline__ void Uniform(unsigned (&b)[5]) {
+    const unsigned w0 = unsigned(__builtin_amdgcn_readfirstlane(int(bw[0])));
+    const unsigned w1 = unsigned(__builtin_amdgcn_readfirstlane(int(bw[1])));
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      *LdsAt(a[2 * q + u]) = v2f{c[4 * q + 2 * u], c[4 * q + 2 * u + 1]};
-    }
+    for (int i = 0; i < 4; ++i) b[i] = (w0 >> (8 * i)) & 255u;
+    b[4] = w1 & 255u;
+    pair = (w1 >> 8) & 1u;
+  }
+};
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4f LdsV4f;
+__device__ __forceinline__ LdsV4f* LdsAt16(unsigned b) {
+  return reinterpret_cast<LdsV4f*>(size_t{b});
 }
 
-// One FP16 op over the (scaled) LDS tile; batches as in ApplyTileOp, two
-// at a time.  mo: the lane's member offsets (record column order, so that
-// reads and writes share them) XOR its group's slot.
-__device__ __forceinline__ void ApplyTileOpF16(const uint8_t* bp,
-                                               const v8h (&f)[4],
-                                               const uint32_t (&mo)[8],
-                                               unsigned nbatch, unsigned wave,
-                                               unsigned nwaves) {
-  unsigned b[5];
+template <bool PAIR>
+__device__ __forceinline__ void ReadBatch(unsigned sp, const uint32_t (&mo)[8],
+                                          v2f (&v)[8]) {
+  if (PAIR) {
 #pragma unroll
-  for (int i = 0; i < 5; ++i)
-    b[i] = unsigned(__builtin_amdgcn_readfirstlane(int(bp[i])));
+    for (int q = 0; q < 4; ++q) {
+      const v4f x = *LdsAt16(sp ^ mo[2 * q]);
+      v[2 * q] = v2f{x[0], x[1]};
+      v[2 * q + 1] = v2f{x[2], x[3]};
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = *LdsAt(sp ^ mo[q]);
+  }
+}
+
+// Results of a batch back to the slots its inputs came from: C registers
+// (2 q, 2 q + 1) are the q-th member of the lane's list.
+template <bool PAIR>
+__device__ __forceinline__ void WriteBack(unsigned sp, const uint32_t (&mo)[8],
+                                          const v16f& c) {
+  if (PAIR) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *LdsAt16(sp ^ mo[2 * q]) =
+          v4f{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      *LdsAt(sp ^ mo[q]) = v2f{c[2 * q], c[2 * q + 1]};
+  }
+}
+
+// One FP16 op over the LDS tile; batches as in ApplyTileOp, two at a time.
+// SCALE: the tile in LDS is not scaled yet; what is read is multiplied by
+// 2^e.
+template <bool PAIR, bool SCALE>
+__device__ __forceinline__ void RunOpF16(const F16Op& o,
+                                         const unsigned (&b)[5],
+                                         unsigned nbatch, unsigned wave,
+                                         unsigned nwaves, int e) {
+  auto read = [&](unsigned sp, v2f (&v)[8]) {
+    ReadBatch<PAIR>(sp, o.mo, v);
+    if (SCALE) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        v[q] = v2f{ldexpf(v[q][0], e), ldexpf(v[q][1], e)};
+    }
+  };
   unsigned bt = wave;
   for (; bt + nwaves < nbatch; bt += 2 * nwaves) {
-    const unsigned sp0 = BatchSlot(bt, b);
-    const unsigned sp1 = BatchSlot(bt + nwaves, b);
-    uint32_t a0[8], a1[8];
+    const unsigned sp0 = BatchSlot<true>(bt, b);
+    const unsigned sp1 = BatchSlot<true>(bt + nwaves, b);
     v2f v0[8], v1[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      a0[q] = sp0 ^ mo[q];
-      v0[q] = *LdsAt(a0[q]);
-    }
+    read(sp0, v0);
     v8h bh0[2], bl0[2], bh1[2], bl1[2];
     SplitF16(v0, bh0, bl0);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      a1[q] = sp1 ^ mo[q];
-      v1[q] = *LdsAt(a1[q]);
-    }
-    const v16f c0 = MfmaChainF16(f, bh0, bl0);
+    read(sp1, v1);
+    const v16f c0 = MfmaChainF16(o.f, bh0, bl0);
     SplitF16(v1, bh1, bl1);
-    const v16f c1 = MfmaChainF16(f, bh1, bl1);
-    WriteBack(a0, c0);
-    WriteBack(a1, c1);
+    const v16f c1 = MfmaChainF16(o.f, bh1, bl1);
+    WriteBack<PAIR>(sp0, o.mo, c0);
+    WriteBack<PAIR>(sp1, o.mo, c1);
   }
   if (bt < nbatch) {
-    const unsigned sp0 = BatchSlot(bt, b);
-    uint32_t a0[8];
+    const unsigned sp0 = BatchSlot<true>(bt, b);
     v2f v0[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      a0[q] = sp0 ^ mo[q];
-      v0[q] = *LdsAt(a0[q]);
-    }
+    read(sp0, v0);
     v8h bh0[2], bl0[2];
     SplitF16(v0, bh0, bl0);
-    WriteBack(a0, MfmaChainF16(f, bh0, bl0));
+    WriteBack<PAIR>(sp0, o.mo, MfmaChainF16(o.f, bh0, bl0));
   }
+}
+
+template <bool SCALE = false>
+__device__ __forceinline__ void ApplyTileOpF16(F16Op& o, unsigned nbatch,
+                                               unsigned wave, unsigned nwaves,
+                                               int e = 0) {
+  unsigned b[5];
+  o.Uniform(b);
+  if (o.pair)
+    RunOpF16<true, SCALE>(o, b, nbatch, wave, nwaves, e);
+  else
+    RunOpF16<false, SCALE>(o, b, nbatch, wave, nwaves, e);
 }
 
 // Largest |re| or |im| over the first `nper` of a thread's PER elements
@@ -422,10 +499,18 @@ __device__ __forceinline__ float LocalMax(const float2 (&v)[PER],
   return m;
 }
 
+// The scale exponent of a tile whose largest |re| or |im| is t: t goes to
+// [2^5, 2^6) / 2^headroom; 0 for an all-zero (or non-finite) tile.
+__device__ __forceinline__ int ScaleExponent(float t, unsigned headroom) {
+  if (!(t > 0.0f) || !(t <= 3.0e38f)) return 0;
+  int e;
+  (void)frexpf(t, &e);  // t in [2^(e-1), 2^e)
+  return 6 - int(headroom) - e;  // |e| <= 149: ldexpf takes any such shift
+}
+
 // Workgroup maximum of `m` through `slots` (one float per wave), then the
-// tile's scale exponent: the largest value to [2^5, 2^6) / 2^headroom, or
-// 0 for an all-zero (or non-finite) tile.  Ends with a barrier before the
-// slots are read; the slots are written again only after a later barrier.
+// tile's scale exponent.  Ends with a barrier before the slots are read;
+// the slots are written again only after a later barrier.
 template <int NWAVES>
 __device__ __forceinline__ int TileScale(float m, float* slots,
                                          unsigned headroom) {
@@ -436,10 +521,7 @@ __device__ __forceinline__ int TileScale(float m, float* slots,
   float t = 0.0f;
 #pragma unroll
   for (int w = 0; w < NWAVES; ++w) t = fmaxf(t, slots[w]);
-  if (!(t > 0.0f) || !(t <= 3.0e38f)) return 0;
-  int e;
-  (void)frexpf(t, &e);  // t in [2^(e-1), 2^e)
-  return 6 - int(headroom) - e;  // |e| <= 149: ldexpf takes any such shift
+  return ScaleExponent(t, headroom);
 }
 
 // Offset (in amplitudes) of tile-local high index x: x's bits deposited at
@@ -447,6 +529,20 @@ __device__ __forceinline__ int TileScale(float m, float* slots,
 __device__ __forceinline__ uint64_t DepositHigh(unsigned x, const BlockGeom& g) {
   uint64_t o = 0;
   for (unsigned b = 0; b < g.h; ++b) o += ((x >> b) & 1u) ? g.hbit[b] : 0;
+  return o;
+}
+
+// The same for x's bits at tile positions first, first + 1, ... (a
+// compile-time x < 2^NB, none of them in the low run), in units of 2^Lc
+// amplitudes; hbit is zero past the tile's last position.
+template <int NB>
+__device__ __forceinline__ uint32_t HighOffset(unsigned x, unsigned first,
+                                               const BlockGeom& g) {
+  uint32_t o = 0;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if ((x >> b) & 1u) o += uint32_t(g.hbit[first - g.Lc + b] >> g.Lc);
+  }
   return o;
 }
 
@@ -459,19 +555,21 @@ __device__ __forceinline__ uint64_t DepositHigh(unsigned x, const BlockGeom& g) 
 // element instead of a deposit loop.  The element parts are wave-uniform
 // and kept in units of 2^Lc amplitudes (32 bits: no tile qubit is 32 above
 // the low run).
-template <int PER, int NT>
+template <int PER, int NT, bool F16>
 struct TileIo {
   static_assert(NT == 256 || NT == 512, "thread bits");
+  static_assert(PER <= 32, "element bits");
   static constexpr unsigned kLogNT = NT == 256 ? 8 : 9;
   uint64_t tofs;       // this thread's part
   uint32_t eofs[PER];  // the element parts >> Lc
 
-  // LDS slot of element i: TileSwz is linear and changes only the low four
-  // bits, so TileSwz(t + NT i) = (TileSwz(t) ^ (TileSwz(NT i) & 15)) + NT i
-  // with TileSwz(t) < NT: the NT i part is an instruction offset and the
+  // LDS slot of element i: the swizzle S is linear and changes only the low
+  // four bits, so S(t + NT i) = (S(t) ^ (S(NT i) & 15)) + NT i with
+  // S(t) < NT: the NT i part is an instruction offset and the
   // rest takes one XOR with a constant.
   __device__ __forceinline__ unsigned Slot(int i) const {
-    return (TileSwz(threadIdx.x) ^ (TileSwz(NT * unsigned(i)) & 15u)) +
+    return (BlockSwz<F16>(threadIdx.x) ^
+            (BlockSwz<F16>(NT * unsigned(i)) & 15u)) +
            NT * unsigned(i);
   }
 
@@ -480,7 +578,7 @@ struct TileIo {
     tofs = (t & ((1u << g.Lc) - 1)) + DepositHigh(t >> g.Lc, g);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      eofs[i] = uint32_t(DepositHigh(unsigned(i) << (kLogNT - g.Lc), g) >> g.Lc);
+      eofs[i] = HighOffset<5>(unsigned(i), kLogNT, g);
     }
   }
 

@@ -460,7 +460,7 @@ __device__ __forceinline__ void TrajTileRun(float2* __restrict__ s,
     uint4* dst = reinterpret_cast<uint4*>(rec);
     for (unsigned q = threadIdx.x; q < nq; q += NT) dst[q] = src[q];
   }
-  TileIo<PER, NT> io;
+  TileIo<PER, NT, true> io;
   io.Init(g);
   float2 buf[PER];
   io.template Fetch<FULL, 15u>(s, 0, g, buf);  // tile 0 starts at amplitude 0
@@ -475,16 +475,9 @@ __device__ __forceinline__ void TrajTileRun(float2* __restrict__ s,
     const uint64_t nb = InsertZeros(next << g.Lc, g.outer, g.nouter);
     io.template Fetch<FULL, 3u>(s, nb, g, buf);
     for (unsigned op = 0; op < nops; ++op) {
-      const uint32_t* r = rec + op * unsigned(kF16RecWords);
-      v8h f[4];
-      LoadFragF16(r, l, f);
-      const uint32_t* tab = r + kF16TabOff + 16 * (l >> 5);
-      const uint32_t sj = r[kF16TabOff + kTableWords + (l & 31)];
-      uint32_t mo[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) mo[q] = tab[q] ^ sj;
-      ApplyTileOpF16(reinterpret_cast<const uint8_t*>(r + kF16BposOff), f,
-                     mo, nbatch, wave, NW);
+      F16Op o;
+      o.Load(rec + op * unsigned(kF16RecWords), l);
+      ApplyTileOpF16(o, nbatch, wave, NW);
       __syncthreads();
       if (op == 1) io.template Fetch<FULL, 12u>(s, nb, g, buf);
     }

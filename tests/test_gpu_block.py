@@ -87,6 +87,25 @@ def test_block_random_programs(sim, n, lc, tb, arith):
         assert fid > 1 - fbar
 
 
+@pytest.mark.parametrize("nops", [1, 2, 3, 9, 14])
+def test_f16_many_14_qubit_tiles_per_workgroup(sim, nops):
+    # 2 and 4 tiles a workgroup (one workgroup a CU, 256 CUs): the tile
+    # exchange with every share schedule (1, 2, ... ops) and both LDS access
+    # widths (position 0 a target or not).  Bar: 2^-22 per op.
+    rng = np.random.default_rng(40 + nops)
+    for n in (23, 24):
+        tile = random_tile(n, 4, 14, rng)
+        gates = []
+        for i in range(nops):
+            low = [0] if i % 2 else []
+            qs = low + [int(q) for q in rng.choice(tile[1:], 4 - len(low),
+                                                   replace=False)]
+            gates.append((sorted(qs), to_interleaved(random_matrix(4, rng),
+                                                     np.float64)))
+        err, fid = run_case(sim, n, tile, gates, rng)
+        assert err < 2.0 ** -22 * (nops + 1), (n, tile, err)
+
+
 @pytest.mark.parametrize("arith", ["f16", "bf16"])
 def test_block_max_program_and_single_gates(sim, arith):
     rng = np.random.default_rng(5)
