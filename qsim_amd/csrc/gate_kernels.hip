@@ -1,17 +1,19 @@
 // gate_kernels.hip -- k-qubit gate passes and <psi|U|psi> on gfx950.
 //
-// Two kernel families apply psi <- U psi on every 2^k-amplitude group
+// Three kernel families apply psi <- U psi on every 2^k-amplitude group
 // (the operation of SimulatorCUDA::ApplyGate / ApplyControlledGate,
 // lib/simulator_cuda.h:70-207; arithmetic as lib/simulator_basic.h:167-275):
 //
-//  * GateRegKernel  -- all targets and controls at qubit >= 5.  One group per
-//    work item, held in registers; the 64 lanes of a wave read 64 consecutive
-//    float2/double2 for every group member, so each member load is one
-//    contiguous 512 B (complex64) stream.  No LDS, no barriers.
-//  * GateTileKernel -- some target or control below qubit 5.  A workgroup
-//    stages a tile of 2^tb amplitudes (the Lc lowest qubits, contiguous in
-//    memory, times the high targets) in LDS with coalesced loads, applies the
-//    groups from LDS and streams the tile back.
+//  * GateLaneKernel -- k <= 4, any targets and controls, states of at least
+//    2^(6+k) amplitudes per control pattern.  A wave loads 2^k runs of 64
+//    consecutive amplitudes; targets among the lane qubits move to register
+//    bits by swaps across lanes.  No LDS, no barriers.
+//  * GateRegKernel  -- k = 5, 6 with all targets and controls at qubit >= 5:
+//    one group per work item, held in registers.
+//  * GateTileKernel -- the rest (k = 5, 6 with a qubit below 5, and small
+//    states).  A workgroup stages a tile of 2^tb amplitudes (the Lc lowest
+//    qubits, contiguous in memory, times the high targets) in LDS with
+//    coalesced loads, applies the groups from LDS and streams the tile back.
 //
 // The gate matrix (row-major, row/column bit j <-> qs[j]) travels by value in
 // the kernel arguments when it fits in 2 KiB (scalar loads, uniform across the
@@ -163,6 +165,118 @@ GateTileKernel(typename Cplx<FP>::T* __restrict__ s, TileGeom g, M m) {
   }
 }
 
+// Geometry of the lane kernel.  A wave's chunk is 2^(6+K) amplitudes.  Lane
+// bit i is qubit lane[i]: the six lowest qubits, passing over controls that
+// can be skipped.  Register bit j is the amplitude offset roff[j]: first,
+// one per target among the lane qubits, the lowest qubits that are neither
+// lane, target nor control; then the other targets, ascending.  Chunk c
+// starts at c << low (the lane qubits 0 .. low - 1) with zero bits inserted
+// at ins[0..nins) (every other lane qubit, register bit and control,
+// ascending) OR cbits.
+struct LaneGeom {
+  uint64_t nchunks;
+  uint64_t cbits;
+  uint64_t roff[6];
+  unsigned low;
+  unsigned nins;
+  unsigned ins[kMaxInserted];
+  unsigned lane[6];
+  unsigned nlow;        // targets among the lane qubits: bits lbit[0..nlow)
+  unsigned lbit[6];
+  unsigned cmask;       // controls among the lane bits
+  unsigned cvals;
+};
+
+__device__ __forceinline__ float PullLane(unsigned addr, float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(
+                                       int(addr), __builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double PullLane(unsigned addr, double v) {
+  const uint2 w = __builtin_bit_cast(uint2, v);
+  const uint2 r{unsigned(__builtin_amdgcn_ds_bpermute(int(addr), int(w.x))),
+                unsigned(__builtin_amdgcn_ds_bpermute(int(addr), int(w.y)))};
+  return __builtin_bit_cast(double, r);
+}
+
+// Swaps lane bit b with register bit I of the D values a lane holds (its own
+// inverse): of each register pair a lane keeps the value whose register bit
+// equals its lane bit and trades the other with its partner lane ^ 2^b.
+template <int K, int I, typename C>
+__device__ __forceinline__ void SwapLaneBit(C (&v)[1 << K], unsigned b) {
+  const unsigned lane = threadIdx.x & 63;
+  const bool hi = (lane >> b) & 1u;
+  const unsigned addr = (lane ^ (1u << b)) * 4;
+#pragma unroll
+  for (int j = 0; j < (1 << K); ++j) {
+    if ((j >> I) & 1) continue;
+    C& lo = v[j];
+    C& up = v[j | (1 << I)];
+    const auto x = PullLane(addr, hi ? lo.x : up.x);
+    const auto y = PullLane(addr, hi ? lo.y : up.y);
+    lo.x = hi ? x : lo.x;
+    lo.y = hi ? y : lo.y;
+    up.x = hi ? up.x : x;
+    up.y = hi ? up.y : y;
+  }
+}
+
+template <int K, int I, typename C>
+__device__ __forceinline__ void SwapLowTargets(C (&v)[1 << K],
+                                               const LaneGeom& g) {
+  if constexpr (I < K) {
+    if (I < int(g.nlow)) {
+      SwapLaneBit<K, I>(v, g.lbit[I]);
+      SwapLowTargets<K, I + 1>(v, g);
+    }
+  }
+}
+
+// Any targets and controls, K <= 4, on states with 2^(6+K) amplitudes in the
+// subspace of the skipped controls.  A wave's loads and stores are runs of
+// consecutive amplitudes (64 of them unless a control is skipped below
+// qubit 6); targets among the lane qubits are brought from lane bits into
+// register bits, and back, by swaps across lanes, so that each lane holds
+// whole groups in matrix order.  No LDS, no barriers.
+//
+// Bound by the HBM stream.  Complex128, 27 qubits, targets below qubit 6:
+// k = 1..3 0.77-0.83 ms, k = 4 0.81-1.0 ms (the LDS tile kernel, half of
+// whose threads have no group at these sizes: 1.8 and 2.3-2.5 ms); complex64,
+// 28 qubits: k = 1..3 0.72-0.83 ms (0.78-0.87); 2^12 .. 2^20 amplitudes:
+// 1-5 us less per pass, many short waves instead of a few large tiles.
+//
+// A control below kLineQubit (8 complex64 or 4 complex128 to a 64-byte
+// half line) cannot skip memory: its lanes load and store too and keep
+// their values; masked partial lines measured 7 % slower (28 qubits,
+// control 0).  Controls above are skipped as any other high qubit.
+template <typename FP, int K, typename M>
+__global__ void __launch_bounds__(256)
+GateLaneKernel(typename Cplx<FP>::T* __restrict__ s, LaneGeom g, M m) {
+  using C = typename Cplx<FP>::T;
+  constexpr int D = 1 << K;
+  const unsigned lane = threadIdx.x & 63;
+  const bool active = (lane & g.cmask) == g.cvals;
+  uint64_t loff = 0;
+#pragma unroll
+  for (int b = 0; b < 6; ++b) loff += uint64_t((lane >> b) & 1u) << g.lane[b];
+  const uint64_t stride = uint64_t(gridDim.x) * 4;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (uint64_t c = uint64_t(blockIdx.x) * 4 + wave; c < g.nchunks;
+       c += stride) {
+    C* p = s + (InsertZeros(c << g.low, g.ins, g.nins) | g.cbits);
+    C v[D], u[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) v[j] = p[MemberOffset<K>(j, g.roff) + loff];
+    SwapLowTargets<K, 0>(v, g);
+    MatVec<FP, K>(v, m, [&](int r, C val) {
+      u[r].x = active ? val.x : v[r].x;
+      u[r].y = active ? val.y : v[r].y;
+    });
+    SwapLowTargets<K, 0>(u, g);
+#pragma unroll
+    for (int j = 0; j < D; ++j) p[MemberOffset<K>(j, g.roff) + loff] = u[j];
+  }
+}
+
 // <psi|U|psi> partial sums; any target positions (reads through the cache
 // hierarchy, like the gate kernels' register path).
 template <typename FP, int K, typename M>
@@ -265,6 +379,69 @@ int LaunchTile(typename Cplx<FP>::T* s, const TileGeom& g, const M& m) {
 }
 
 
+// The lane kernel's geometry; false where the state is too small for it.
+template <typename FP>
+bool LaneGeometry(unsigned n, const unsigned* qs, unsigned k,
+                  const unsigned* cqs, unsigned nc, uint64_t cvals,
+                  LaneGeom& g) {
+  constexpr unsigned kLineQubit = sizeof(FP) == 4 ? 3 : 2;
+  uint64_t targets = 0, skipped = 0, kept = 0;  // kept: controls in the lanes
+  uint64_t kept_bits = 0;
+  g = LaneGeom{};
+  for (unsigned b = 0; b < k; ++b) targets |= uint64_t{1} << qs[b];
+  for (unsigned i = 0; i < nc; ++i) {
+    const uint64_t bit = (cvals >> i) & 1;
+    if (cqs[i] < kLineQubit) {
+      kept |= uint64_t{1} << cqs[i];
+      kept_bits |= bit << cqs[i];
+    } else {
+      skipped |= uint64_t{1} << cqs[i];
+      g.cbits |= bit << cqs[i];
+    }
+  }
+  const unsigned ns = unsigned(__builtin_popcountll(skipped));
+  if (n < 6 + k + ns) return false;
+  unsigned q = 0, nl = 0;
+  uint64_t taken = skipped;
+  for (; nl < 6; ++q) {
+    if ((skipped >> q) & 1) continue;
+    if ((targets >> q) & 1) g.lbit[g.nlow++] = nl;
+    if ((kept >> q) & 1) {
+      g.cmask |= 1u << nl;
+      g.cvals |= unsigned((kept_bits >> q) & 1) << nl;
+    }
+    taken |= uint64_t{1} << q;
+    g.lane[nl++] = q;
+  }
+  unsigned r = 0;
+  for (unsigned o = q; r < g.nlow; ++o) {
+    if (((targets | skipped) >> o) & 1) continue;
+    taken |= uint64_t{1} << o;
+    g.roff[r++] = uint64_t{1} << o;
+  }
+  for (unsigned b = g.nlow; b < k; ++b) {
+    taken |= uint64_t{1} << qs[b];
+    g.roff[r++] = uint64_t{1} << qs[b];
+  }
+  while (g.low < 6 && g.lane[g.low] == g.low) ++g.low;
+  for (unsigned b = g.low; b < n; ++b)
+    if ((taken >> b) & 1) g.ins[g.nins++] = b;
+  g.nchunks = uint64_t{1} << (n - 6 - k - ns);
+  return true;
+}
+
+template <typename FP, int K, typename M>
+int LaunchLane(typename Cplx<FP>::T* s, const LaneGeom& g, const M& m) {
+  const uint64_t blocks =
+      std::min<uint64_t>((g.nchunks + 3) / 4, uint64_t{1} << 20);
+  PassTimerBegin();
+  hipLaunchKernelGGL((GateLaneKernel<FP, K, M>), dim3(unsigned(blocks)),
+                     dim3(256), 0, Stream(), s, g, m);
+  PassTimerEnd();
+  QHIP_LAUNCHED("GateLaneKernel");
+  return QSIM_HIP_OK;
+}
+
 template <typename FP, int K>
 int DispatchK(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
               const unsigned* cqs, unsigned nc, uint64_t cvals, const FP* m) {
@@ -284,6 +461,14 @@ int DispatchK(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
     if (d == nullptr) return QSIM_HIP_ERR_OOM;
     QHIP_TRY(StageMatrix(d, m, bytes));
     mp.p = static_cast<const FP*>(d);
+  }
+
+  if constexpr (K <= 4) {
+    LaneGeom lg;
+    if (LaneGeometry<FP>(n, qs, K, cqs, nc, cvals, lg)) {
+      if constexpr (byval) return LaunchLane<FP, K>(s, lg, mv);
+      else return LaunchLane<FP, K>(s, lg, mp);
+    }
   }
 
   if (lowest >= 5 || n < 5) {

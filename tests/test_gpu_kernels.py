@@ -180,6 +180,41 @@ def test_controlled_gate_vs_oracle(dtype, sim):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("controls", [(), (0,), (1, 2), (2,), (3,), (5,),
+                                      (0, 4), (2, 5, 7), (1, 3, 4, 5, 9)])
+def test_lane_kernel_edges(dtype, controls, sim):
+    # The smallest state the lane kernel takes (6 + k + controls it skips),
+    # one qubit less (the tile kernel) and one more, targets packed at the
+    # bottom, at the top and alternating; amplitudes outside the controls'
+    # subspace keep their bits.
+    rng = np.random.default_rng(77 + len(controls))
+    for k in range(0, 5):
+        for n in range(5 + k + len(controls), 8 + k + len(controls)):
+            free = [q for q in range(n) if q not in controls]
+            if len(free) < k or any(c >= n for c in controls):
+                continue
+            for qs in {tuple(free[:k]), tuple(free[len(free) - k:]),
+                       tuple(free[::2][:k])}:
+                qs = list(qs)
+                vals = int(rng.integers(0, 1 << len(controls)))
+                m = to_interleaved(random_matrix(k, rng), dtype)
+                s = random_state(n, rng, dtype)
+                st = upload(s, n, dtype)
+                sim.apply_controlled_gate(qs, list(controls), vals, m, st)
+                got = st.to_numpy()
+                want = s.copy()
+                oracle.apply_controlled_gate(n, want, qs, list(controls), vals,
+                                             m)
+                assert rel_l2(got, want) < TOL[dtype], (n, qs)
+                idx = np.arange(1 << n)
+                out = np.zeros(1 << n, bool)
+                for i, c in enumerate(controls):
+                    out |= ((idx >> c) & 1) != ((vals >> i) & 1)
+                np.testing.assert_array_equal(got.reshape(-1, 2)[out],
+                                              s.reshape(-1, 2)[out])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_expectation_value_vs_oracle(dtype, sim):
     rng = np.random.default_rng(14)
     for n in (1, 2, 4, 6, 9, 13, 18):
