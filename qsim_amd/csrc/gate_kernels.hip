@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "lane.h"
 #include "reduce.h"
 #include "tile.h"
 
@@ -51,15 +52,6 @@ struct MatPtr {
 template <typename FP, int K>
 constexpr unsigned TileBitsMax() {
   return sizeof(FP) == 4 ? 13u : 12u;
-}
-
-template <int K>
-__device__ __forceinline__ uint64_t MemberOffset(unsigned j,
-                                                 const uint64_t* tbit) {
-  uint64_t o = 0;
-#pragma unroll
-  for (int b = 0; b < K; ++b) o += ((j >> b) & 1) ? tbit[b] : 0;
-  return o;
 }
 
 // out = U v for one group; writes row r through `store(r, value)`.
@@ -162,72 +154,6 @@ GateTileKernel(typename Cplx<FP>::T* __restrict__ s, TileGeom g, M m) {
     __syncthreads();
     TileStore<PER>(s, base, g, lds);
     __syncthreads();
-  }
-}
-
-// Geometry of the lane kernel.  A wave's chunk is 2^(6+K) amplitudes.  Lane
-// bit i is qubit lane[i]: the six lowest qubits, passing over controls that
-// can be skipped.  Register bit j is the amplitude offset roff[j]: first,
-// one per target among the lane qubits, the lowest qubits that are neither
-// lane, target nor control; then the other targets, ascending.  Chunk c
-// starts at c << low (the lane qubits 0 .. low - 1) with zero bits inserted
-// at ins[0..nins) (every other lane qubit, register bit and control,
-// ascending) OR cbits.
-struct LaneGeom {
-  uint64_t nchunks;
-  uint64_t cbits;
-  uint64_t roff[6];
-  unsigned low;
-  unsigned nins;
-  unsigned ins[kMaxInserted];
-  unsigned lane[6];
-  unsigned nlow;        // targets among the lane qubits: bits lbit[0..nlow)
-  unsigned lbit[6];
-  unsigned cmask;       // controls among the lane bits
-  unsigned cvals;
-};
-
-__device__ __forceinline__ float PullLane(unsigned addr, float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(
-                                       int(addr), __builtin_bit_cast(int, v)));
-}
-__device__ __forceinline__ double PullLane(unsigned addr, double v) {
-  const uint2 w = __builtin_bit_cast(uint2, v);
-  const uint2 r{unsigned(__builtin_amdgcn_ds_bpermute(int(addr), int(w.x))),
-                unsigned(__builtin_amdgcn_ds_bpermute(int(addr), int(w.y)))};
-  return __builtin_bit_cast(double, r);
-}
-
-// Swaps lane bit b with register bit I of the D values a lane holds (its own
-// inverse): of each register pair a lane keeps the value whose register bit
-// equals its lane bit and trades the other with its partner lane ^ 2^b.
-template <int K, int I, typename C>
-__device__ __forceinline__ void SwapLaneBit(C (&v)[1 << K], unsigned b) {
-  const unsigned lane = threadIdx.x & 63;
-  const bool hi = (lane >> b) & 1u;
-  const unsigned addr = (lane ^ (1u << b)) * 4;
-#pragma unroll
-  for (int j = 0; j < (1 << K); ++j) {
-    if ((j >> I) & 1) continue;
-    C& lo = v[j];
-    C& up = v[j | (1 << I)];
-    const auto x = PullLane(addr, hi ? lo.x : up.x);
-    const auto y = PullLane(addr, hi ? lo.y : up.y);
-    lo.x = hi ? x : lo.x;
-    lo.y = hi ? y : lo.y;
-    up.x = hi ? up.x : x;
-    up.y = hi ? up.y : y;
-  }
-}
-
-template <int K, int I, typename C>
-__device__ __forceinline__ void SwapLowTargets(C (&v)[1 << K],
-                                               const LaneGeom& g) {
-  if constexpr (I < K) {
-    if (I < int(g.nlow)) {
-      SwapLaneBit<K, I>(v, g.lbit[I]);
-      SwapLowTargets<K, I + 1>(v, g);
-    }
   }
 }
 
@@ -378,57 +304,6 @@ int LaunchTile(typename Cplx<FP>::T* s, const TileGeom& g, const M& m) {
   return QSIM_HIP_OK;
 }
 
-
-// The lane kernel's geometry; false where the state is too small for it.
-template <typename FP>
-bool LaneGeometry(unsigned n, const unsigned* qs, unsigned k,
-                  const unsigned* cqs, unsigned nc, uint64_t cvals,
-                  LaneGeom& g) {
-  constexpr unsigned kLineQubit = sizeof(FP) == 4 ? 3 : 2;
-  uint64_t targets = 0, skipped = 0, kept = 0;  // kept: controls in the lanes
-  uint64_t kept_bits = 0;
-  g = LaneGeom{};
-  for (unsigned b = 0; b < k; ++b) targets |= uint64_t{1} << qs[b];
-  for (unsigned i = 0; i < nc; ++i) {
-    const uint64_t bit = (cvals >> i) & 1;
-    if (cqs[i] < kLineQubit) {
-      kept |= uint64_t{1} << cqs[i];
-      kept_bits |= bit << cqs[i];
-    } else {
-      skipped |= uint64_t{1} << cqs[i];
-      g.cbits |= bit << cqs[i];
-    }
-  }
-  const unsigned ns = unsigned(__builtin_popcountll(skipped));
-  if (n < 6 + k + ns) return false;
-  unsigned q = 0, nl = 0;
-  uint64_t taken = skipped;
-  for (; nl < 6; ++q) {
-    if ((skipped >> q) & 1) continue;
-    if ((targets >> q) & 1) g.lbit[g.nlow++] = nl;
-    if ((kept >> q) & 1) {
-      g.cmask |= 1u << nl;
-      g.cvals |= unsigned((kept_bits >> q) & 1) << nl;
-    }
-    taken |= uint64_t{1} << q;
-    g.lane[nl++] = q;
-  }
-  unsigned r = 0;
-  for (unsigned o = q; r < g.nlow; ++o) {
-    if (((targets | skipped) >> o) & 1) continue;
-    taken |= uint64_t{1} << o;
-    g.roff[r++] = uint64_t{1} << o;
-  }
-  for (unsigned b = g.nlow; b < k; ++b) {
-    taken |= uint64_t{1} << qs[b];
-    g.roff[r++] = uint64_t{1} << qs[b];
-  }
-  while (g.low < 6 && g.lane[g.low] == g.low) ++g.low;
-  for (unsigned b = g.low; b < n; ++b)
-    if ((taken >> b) & 1) g.ins[g.nins++] = b;
-  g.nchunks = uint64_t{1} << (n - 6 - k - ns);
-  return true;
-}
 
 template <typename FP, int K, typename M>
 int LaunchLane(typename Cplx<FP>::T* s, const LaneGeom& g, const M& m) {

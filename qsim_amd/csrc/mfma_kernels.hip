@@ -28,9 +28,12 @@
 // Its operand maps: a[e] = A[l%32][8(l/32) + e], b[e] = B[8(l/32) + e][l%32]
 // for e = 0..7 over a K block of 16, i.e. 4 members per lane half.
 //
-// Two data paths, as for the vector kernels: targets all at qubit >= 5 read
-// the operands straight from HBM (32 lanes = 32 consecutive amplitudes); a
-// target below qubit 5 stages a tile in LDS (XOR-swizzled to spread banks).
+// Data paths: k = 4 holds a group per lane and swaps low targets across
+// lanes (GateMfmaLaneKernel).  k = 5, 6 keep each wave's rows of the matrix in
+// registers (f16_kernels.hip); on states too small for that, targets all at
+// qubit >= 5 read the operands straight from HBM (32 lanes = 32 consecutive
+// amplitudes) and a target below qubit 5 stages a tile in LDS (XOR-swizzled
+// to spread banks).
 
 #include <hip/hip_runtime.h>
 
@@ -39,6 +42,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "lane.h"
 #include "tile.h"
 
 namespace qhip {
@@ -269,6 +273,63 @@ GateMfmaTileKernel(float2* __restrict__ s, TileGeom g,
   }
 }
 
+// k = 4 on any targets, a group per lane (lane.h): a wave's chunk is two
+// batches of 32 groups, every load and store 64 consecutive amplitudes.
+// v_permlane32_swap of a member's real and imaginary parts (lanes = groups
+// 0..63) gives the B operands of both batches -- real parts of a batch on
+// lanes < 32, imaginary on lanes >= 32 -- and the same swap of the two
+// accumulators gives back member registers over 64 groups.  Targets among
+// the lane qubits are swapped into register bits before and back after.
+//
+// Bound by the HBM stream (16 streams at power-of-two distances); the MFMA
+// chains take a third of that time.  Runs of 512 bytes matter: the same
+// product on 32 groups a wave (256-byte runs) took 0.92-1.06 ms.  28 qubits,
+// 0 / 1 / 2 / 3 / 4 targets below qubit 6: 0.74-0.83 / 0.73-0.81 / 0.74-0.87
+// / 0.77-0.81 / 0.80 ms, against 0.85-0.93 (operands straight from HBM, 32
+// groups) and 0.95-1.06 / 0.93 / 0.80-0.87 / 0.80 (LDS tile); 20 qubits:
+// 8-11 us for 8-18.  Three waves a SIMD keep the registers for all 16 loads
+// in flight (two: 0.83 ms with 4 low targets; four spill).
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(3)))
+GateMfmaLaneKernel(float2* __restrict__ s, LaneGeom g,
+                   const float* __restrict__ frag) {
+  const unsigned lane = threadIdx.x & 63;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  RegFragF32<4> af;
+  af.Load(frag);
+  const uint64_t wstride = uint64_t(gridDim.x) * kWaves;
+  for (uint64_t c = uint64_t(blockIdx.x) * kWaves + wave; c < g.nchunks;
+       c += wstride) {
+    float2* p = s + InsertZeros(c << 6, g.ins, g.nins);
+    float2 v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = p[MemberOffset<4>(j, g.roff) + lane];
+    SwapLowTargets<4, 0>(v, g);
+    v16f c0 = v16f{}, c1 = v16f{};
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      TradeLanes<5>(v[t].x, v[t].y);
+      c0 = __builtin_amdgcn_mfma_f32_32x32x2f32(af(0, t), v[t].x, c0, 0, 0, 0);
+      c1 = __builtin_amdgcn_mfma_f32_32x32x2f32(af(0, t), v[t].y, c1, 0, 0, 0);
+    }
+    // Register 4 q + 2 u + component of both: members 4 q + u, 4 q + 2 + u.
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float2 x{c0[4 * q + 2 * u], c0[4 * q + 2 * u + 1]};
+        float2 y{c1[4 * q + 2 * u], c1[4 * q + 2 * u + 1]};
+        TradeLanes<5>(x.x, y.x);
+        TradeLanes<5>(x.y, y.y);
+        v[4 * q + u] = x;
+        v[4 * q + 2 + u] = y;
+      }
+    SwapLowTargets<4, 0>(v, g);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) p[MemberOffset<4>(j, g.roff) + lane] = v[j];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Split-BF16 MFMA: per K block of 16 reals (8 members), lane half h supplies
 // members 8 kb + 4 h + 0..3 as (re, im) pairs.
@@ -390,40 +451,11 @@ uint64_t DepositBits(uint64_t v, uint64_t mask) {
   return r;
 }
 
+// k = 5, 6 on states too small for the row-block kernels: a batch of 32
+// groups per wave, operands straight from HBM or from an LDS tile.
 template <int K>
-int DispatchMfma(float2* s, unsigned n, const unsigned* qs, const double* m64,
-                 bool bf16) {
-  constexpr int D = 1 << K;
-  // Fragments go through the matrix staging ring (64 KiB slots).
-  size_t fbytes;
-  std::vector<float> f32;
-  std::vector<uint16_t> fb;
-  if (!bf16) {
-    f32.resize(size_t(Dims<K>::RB) * D * 64);
-    BuildFragF32(K, m64, f32.data());
-    fbytes = f32.size() * sizeof(float);
-  } else {
-    fb.resize(size_t(Dims<K>::RB) * (2 * D / 16) * 3 * 512);
-    BuildFragBf16(K, m64, fb.data());
-    fbytes = fb.size() * sizeof(uint16_t);
-  }
-  void* dfrag = MatrixBuffer(fbytes);
-  if (dfrag == nullptr) return QSIM_HIP_ERR_OOM;
-  QHIP_TRY(StageMatrix(dfrag, bf16 ? (const void*)fb.data()
-                                   : (const void*)f32.data(),
-                       fbytes));
-  // k = 5, 6 (exact FP32 or split-BF16): each wave keeps its row block of
-  // the matrix in registers (no per-batch fragment reloads through the
-  // cache).
-  if (K >= 5) {
-    const int rc =
-        bf16 ? LaunchRowsBf16(s, n, qs, unsigned(K),
-                              static_cast<const uint16_t*>(dfrag))
-             : LaunchRowsF32(s, n, qs, unsigned(K),
-                             static_cast<const float*>(dfrag));
-    if (rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
-  }
-
+int LaunchBatches(float2* s, unsigned n, const unsigned* qs, void* dfrag,
+                  bool bf16) {
   if (qs[0] >= 5) {
     GateGeom g{};
     g.nins = K;
@@ -521,12 +553,67 @@ int DispatchMfma(float2* s, unsigned n, const unsigned* qs, const double* m64,
   return QSIM_HIP_OK;
 }
 
+template <int K>
+int DispatchMfma(float2* s, unsigned n, const unsigned* qs, const double* m64,
+                 bool bf16) {
+  constexpr int D = 1 << K;
+  // Fragments go through the matrix staging ring (64 KiB slots).
+  size_t fbytes;
+  std::vector<float> f32;
+  std::vector<uint16_t> fb;
+  if (!bf16) {
+    f32.resize(size_t(Dims<K>::RB) * D * 64);
+    BuildFragF32(K, m64, f32.data());
+    fbytes = f32.size() * sizeof(float);
+  } else {
+    fb.resize(size_t(Dims<K>::RB) * (2 * D / 16) * 3 * 512);
+    BuildFragBf16(K, m64, fb.data());
+    fbytes = fb.size() * sizeof(uint16_t);
+  }
+  void* dfrag = MatrixBuffer(fbytes);
+  if (dfrag == nullptr) return QSIM_HIP_ERR_OOM;
+  QHIP_TRY(StageMatrix(dfrag, bf16 ? (const void*)fb.data()
+                                   : (const void*)f32.data(),
+                       fbytes));
+  // k = 5, 6 (exact FP32 or split-BF16): each wave keeps its row block of
+  // the matrix in registers (no per-batch fragment reloads through the
+  // cache).
+  if (K >= 5) {
+    const int rc =
+        bf16 ? LaunchRowsBf16(s, n, qs, unsigned(K),
+                              static_cast<const uint16_t*>(dfrag))
+             : LaunchRowsF32(s, n, qs, unsigned(K),
+                             static_cast<const float*>(dfrag));
+    if (rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
+  }
+
+  if constexpr (K == 4) {
+    LaneGeom g;
+    if (!LaneGeometry<float>(n, qs, K, nullptr, 0, 0, g)) {
+      return QSIM_HIP_ERR_UNSUPPORTED;
+    }
+    const uint64_t blocks = std::min<uint64_t>(
+        (g.nchunks + kWaves - 1) / kWaves, uint64_t{1} << 20);
+    PassTimerBegin();
+    hipLaunchKernelGGL(GateMfmaLaneKernel, dim3(unsigned(blocks)), dim3(256),
+                       0, Stream(), s, g, static_cast<const float*>(dfrag));
+    PassTimerEnd();
+    QHIP_LAUNCHED("GateMfmaLaneKernel");
+    return QSIM_HIP_OK;
+  } else {
+    return LaunchBatches<K>(s, n, qs, dfrag, bf16);
+  }
+}
+
 }  // namespace
 
 int LaunchGateMfma(float2* s, unsigned n, const unsigned* qs, unsigned k,
                    const double* m64, int method) {
-  // Enough groups for whole 32-group batches, and a 4..6-qubit gate.
-  if (k < 4 || k > 6 || n < k + 5) return QSIM_HIP_ERR_UNSUPPORTED;
+  // Enough groups for whole batches (64 groups at k = 4, else 32), and a
+  // 4..6-qubit gate.
+  if (k < 4 || k > 6 || n < (k == 4 ? 10 : k + 5)) {
+    return QSIM_HIP_ERR_UNSUPPORTED;
+  }
   for (unsigned i = 0; i < k; ++i) {
     if (qs[i] >= n || (i > 0 && qs[i] <= qs[i - 1])) {
       SetError("target qubits must be ascending, distinct and < %u", n);
