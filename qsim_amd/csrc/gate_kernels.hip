@@ -524,6 +524,12 @@ int LaunchGate(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
     return QSIM_HIP_ERR_ARG;
   }
   QHIP_TRY(CheckQubits(n, qs, k, cqs, nc));
+  if constexpr (sizeof(FP) == 8) {
+    if (k >= 5 && nc == 0) {
+      const int rc = LaunchGateF64(s, n, qs, k, m);
+      if (rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
+    }
+  }
   switch (k) {
     case 0: return DispatchK<FP, 0>(s, n, qs, cqs, nc, cvals, m);
     case 1: return DispatchK<FP, 1>(s, n, qs, cqs, nc, cvals, m);

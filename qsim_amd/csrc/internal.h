@@ -241,6 +241,12 @@ int LaunchRowsF32(float2* s, unsigned n, const unsigned* qs, unsigned k,
 int LaunchRowsBf16(float2* s, unsigned n, const unsigned* qs, unsigned k,
                    const uint16_t* frag);
 
+// FP64 MFMA for uncontrolled k = 5, 6 gates on complex128 states
+// (f64_kernels.hip; qs checked); QSIM_HIP_ERR_UNSUPPORTED where the vector
+// kernels take it: k = 5 with no low target, states smaller than a set.
+int LaunchGateF64(double2* s, unsigned n, const unsigned* qs, unsigned k,
+                  const double* m);
+
 // Split-BF16 A-operand fragments of a 2^K x 2^K complex matrix (FP64,
 // row-major interleaved): 2^K/16 row blocks x 2^(K+1)/16 K blocks x
 // (hi, mid, lo) x 512.

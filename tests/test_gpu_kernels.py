@@ -214,6 +214,27 @@ def test_lane_kernel_edges(dtype, controls, sim):
                                               s.reshape(-1, 2)[out])
 
 
+@pytest.mark.parametrize("k", [5, 6])
+@pytest.mark.parametrize("n", [9, 10, 11, 12, 16, 22])
+def test_complex128_wide_gates(n, k, sim):
+    # Below, at and above one set (2^10, 2^11 amplitudes), and enough sets
+    # for several per workgroup (2^22: the double-buffered loop); the targets
+    # that end in lanes, members and copies alike.
+    rng = np.random.default_rng(n + k)
+    for qs in (list(range(k)), list(range(n - k, n)),
+               sorted(rng.choice(n, k, replace=False).tolist()),
+               [0] + list(range(n - k + 1, n)),
+               [0, 2, 4] + list(range(n - k + 3, n))):
+        if len(set(qs)) < k:
+            continue
+        m = to_interleaved(random_matrix(k, rng), np.float64)
+        s = random_state(n, rng, np.float64)
+        st = upload(s, n, np.float64)
+        sim.apply_gate(qs, m, st)
+        oracle.apply_gate(n, s, qs, m)
+        assert rel_l2(st.to_numpy(), s) < 1e-14, (n, qs)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_expectation_value_vs_oracle(dtype, sim):
     rng = np.random.default_rng(14)
