@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "internal.h"
 #include "tile.h"
@@ -671,6 +672,234 @@ struct TileIo {
     }
   }
 };
+
+// The FP16 pass over 14-qubit tiles.  One 128 KiB tile fills a CU's LDS, so
+// no second workgroup can hide its HBM phases; the workgroup hides them
+// itself: 8 waves run the ops and 4 waves (one per SIMD) do nothing but move
+// tiles.  The IO waves hold a whole tile in registers (32 16-byte pairs a
+// thread).  While the ops of a tile run they issue, share by share, the
+// stores of the previous tile and, into the registers each store frees, the
+// loads of the next one; a wave that stalls on a full memory queue holds up
+// no op until the barrier that ends it.  Between two tiles they exchange the
+// tile in LDS for the one in registers.  Shares go out with all ops but the
+// last, whose time covers the last loads' latency.
+//
+// The tile is scaled as in GateBlockF16Kernel, but by the first op as it
+// reads (the maximum is known only once the loads have arrived, and the
+// exchange, which nothing overlaps, moves bits unchanged) and on the way out
+// by the stores.
+//
+// Bound by the HBM stream up to 5 ops, then by the ops (about 2.1 ms each:
+// LDS reads and writes of the whole tile, the fp16 split and the MFMA chain
+// in sequence).  32 qubits, tiles of 4 low and 10 random higher qubits, 1 / 3
+// / 5 / 7 ops: 15.4-16.0 / 15.4-15.9 / 16.0-16.2 / 20.3-20.4 ms, against
+// 16.3 / 16.0-17.5 / 18.7-20.1 / 23.2-24.2 with every wave doing both.  The
+// 64 KiB shape has two workgroups a CU, which hide each other's phases, and
+// keeps that structure.
+constexpr unsigned kIoNT = 256;                       // 4 IO waves
+constexpr unsigned kIoThreads = BlockShape<14>::NT + kIoNT;
+
+// Pair i of IO thread t: tile-local amplitudes 2 t + 512 i and its
+// successor.  Positions 9 and up are never in the low run (PrepareGateBlock),
+// so i's bits are the tile's five highest qubits, h[0..4].
+struct TileIoPairs {
+  static constexpr int PER = (1 << 14) / (2 * kIoNT);  // 32 pairs a thread
+  uint64_t tofs;  // t's part of the offset in the state, amplitudes
+  uint64_t h[5];  // wave-uniform
+  unsigned unit;  // t's part of the 16-byte LDS unit
+
+  __device__ __forceinline__ void Init(const BlockGeom& g, unsigned t) {
+    const unsigned a = 2 * t;
+    tofs = (a & ((1u << g.Lc) - 1)) + DepositHigh(a >> g.Lc, g);
+#pragma unroll
+    for (int b = 0; b < 5; ++b) h[b] = g.hbit[9 - g.Lc + b];
+    unit = F16Swz(a) >> 1;
+  }
+  // Addresses of the four pairs 4 C .. 4 C + 3 of the tile at `base`.  The
+  // thread's part is hidden from the optimiser so that the 32 addresses are
+  // not kept in registers across the tile loop, where the pairs are.
+  template <int C>
+  __device__ __forceinline__ void At(float2* s, uint64_t base,
+                                     v4f* (&q)[4]) const {
+    uint64_t o = tofs;
+    asm volatile("" : "+v"(o));
+    uint64_t b = base;
+    if (C & 1) b += h[2];
+    if (C & 2) b += h[3];
+    if (C & 4) b += h[4];
+    float2* p = s + o;
+    q[0] = reinterpret_cast<v4f*>(p + b);
+    q[1] = reinterpret_cast<v4f*>(p + (b + h[0]));
+    q[2] = reinterpret_cast<v4f*>(p + (b + h[1]));
+    q[3] = reinterpret_cast<v4f*>(p + (b + h[0] + h[1]));
+  }
+  __device__ __forceinline__ unsigned Unit(int i) const {
+    unsigned u = unit;
+    asm volatile("" : "+v"(u));
+    return (u ^ ((F16Swz(512u * unsigned(i)) & 15u) >> 1)) +
+           256u * unsigned(i);
+  }
+};
+
+// Maximum of a non-negative value over the wave, in lane 63.
+__device__ __forceinline__ float WaveMaxTo63(float m) {
+  auto step = [&](auto ctrl) {
+    m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                     0, __builtin_bit_cast(int, m), decltype(ctrl)::value, 0xf,
+                     0xf, false)));
+  };
+  step(std::integral_constant<int, 0x111>{});  // row_shr:1, :2, :4, :8
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});  // row_bcast:15, :31
+  step(std::integral_constant<int, 0x143>{});
+  return m;
+}
+
+template <int N, typename F>
+__device__ __forceinline__ void Unrolled(F&& f) {
+  if constexpr (N > 0) {
+    Unrolled<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+// Applies the pass to tiles first, first + stride, ... < end (at least one)
+// of the state at s, with the kIoThreads threads of the workgroup.
+// lds_raw: LDS offset 0, F16Lds<14>::Bytes(p.nops) bytes.
+__device__ __forceinline__ void BlockIoRun(
+    float2* __restrict__ s, const BlockGeom& g, const BlockProgram& p,
+    const uint32_t* __restrict__ recs, char* lds_raw, uint64_t first,
+    uint64_t end, uint64_t stride) {
+  constexpr int NW = BlockShape<14>::kWaves;
+  constexpr int PER = TileIoPairs::PER;
+  constexpr int kShares = PER / 4;
+  v4f* lds4 = reinterpret_cast<v4f*>(lds_raw);
+  float* slots = reinterpret_cast<float*>(lds_raw + F16Lds<14>::kMaxOff);
+  uint32_t* rec = reinterpret_cast<uint32_t*>(lds_raw + F16Lds<14>::kRecOff);
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // The scale exponent of the tile whose wave maxima are in slots 4 par ...
+  auto scale_of = [&](unsigned par) {
+    const float* m = slots + 4 * par;
+    return __builtin_amdgcn_readfirstlane(ScaleExponent(
+        fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), p.headroom));
+  };
+  if (wave < unsigned(NW)) {
+    const int l = threadIdx.x & 63;
+    const unsigned nq = p.nops * unsigned(kF16RecWords / 4);
+    const uint4* src = reinterpret_cast<const uint4*>(recs);
+    uint4* dst = reinterpret_cast<uint4*>(rec);
+    for (unsigned q = threadIdx.x; q < nq; q += 64 * NW) dst[q] = src[q];
+    __syncthreads();
+    unsigned par = 0;
+    // An op's record is read while the op before it finishes.
+    F16Op o;
+    o.Load(rec, l);
+    auto run_op = [&](unsigned op, auto scale, int e) {
+      ApplyTileOpF16<decltype(scale)::value>(o, 32u, wave, NW, e);
+      o.Load(rec + (op + 1 < p.nops ? op + 1 : 0) * unsigned(kF16RecWords), l);
+      __syncthreads();
+    };
+    for (uint64_t tile = first; tile < end; tile += stride) {
+      run_op(0, std::true_type{}, scale_of(par));
+      for (unsigned op = 1; op < p.nops; ++op) run_op(op, std::false_type{}, 0);
+      __syncthreads();
+      par ^= 1u;
+    }
+    return;
+  }
+  const unsigned t = threadIdx.x - 64u * NW;
+  TileIoPairs io;
+  io.Init(g, t);
+  v4f buf[PER];
+  auto load = [&](auto c, uint64_t base) {
+    constexpr int C = decltype(c)::value;
+    v4f* q[4];
+    io.At<C>(s, base, q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) buf[4 * C + i] = *q[i];
+  };
+  auto store = [&](auto c, uint64_t base, int e) {
+    constexpr int C = decltype(c)::value;
+    v4f* q[4];
+    io.At<C>(s, base, q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const v4f v = buf[4 * C + i];
+      *q[i] = v4f{ldexpf(v.x, -e), ldexpf(v.y, -e), ldexpf(v.z, -e),
+                  ldexpf(v.w, -e)};
+    }
+  };
+  // Waits for the loads; the maximum of this wave's values to its slot.
+  auto arrive = [&](unsigned par) {
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const v4f v = buf[i];
+      m = fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y));
+      m = fmaxf(fmaxf(m, fabsf(v.z)), fabsf(v.w));
+    }
+    m = WaveMaxTo63(m);
+    if ((t & 63u) == 63u) slots[4 * par + (t >> 6)] = m;
+  };
+  uint64_t tile = first;
+  uint64_t base = InsertZeros(tile << g.Lc, g.outer, g.nouter);
+  Unrolled<kShares>([&](auto c) { load(c, base); });
+  arrive(0);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) lds4[io.Unit(i)] = buf[i];
+  __syncthreads();
+  unsigned par = 0;
+  uint64_t obase = 0;  // the finished tile in buf
+  int oe = 0;
+  const unsigned spread = p.nops > 1 ? p.nops - 1 : 1;
+  for (bool out = false;; out = true) {
+    const int e = scale_of(par);
+    const bool more = tile + stride < end;
+    tile += stride;
+    const uint64_t nb =
+        more ? InsertZeros(tile << g.Lc, g.outer, g.nouter) : 0;
+    unsigned op = 0;
+    Unrolled<kShares>([&](auto c) {
+      constexpr unsigned C = decltype(c)::value;
+      // Share C goes out with op C spread / 8.
+      for (const unsigned due = C * spread / kShares; op < due; ++op)
+        __syncthreads();
+      if (out) store(c, obase, oe);
+      if (more) load(c, nb);
+    });
+    for (; op + 1 < p.nops; ++op) __syncthreads();
+    par ^= 1u;
+    if (more) arrive(par);
+    __syncthreads();
+    // The exchange: every slot of the tile belongs to one thread here.  The
+    // reads of one step are in flight while the step before is written.
+    constexpr int ST = 2;
+    v4f old[2][ST];
+    auto take = [&](auto c) {
+      constexpr int C = decltype(c)::value;
+#pragma unroll
+      for (int i = 0; i < ST; ++i) old[C & 1][i] = lds4[io.Unit(ST * C + i)];
+    };
+    take(std::integral_constant<int, 0>{});
+    Unrolled<PER / ST>([&](auto c) {
+      constexpr int C = decltype(c)::value;
+      if constexpr (C + 1 < PER / ST) take(std::integral_constant<int, C + 1>{});
+#pragma unroll
+      for (int i = 0; i < ST; ++i) {
+        if (more) lds4[io.Unit(ST * C + i)] = buf[ST * C + i];
+        buf[ST * C + i] = old[C & 1][i];
+      }
+    });
+    __syncthreads();
+    obase = base;
+    oe = e;
+    if (!more) break;
+    base = nb;
+  }
+  Unrolled<kShares>([&](auto c) { store(c, obase, oe); });
+}
 
 }  // namespace tileop
 }  // namespace qhip

@@ -64,15 +64,15 @@ constexpr unsigned kPairChunk = 16;
 template <int NT>
 constexpr unsigned kSweep = 8192 / NT;
 
+// Groups [lo, hi) of a gate.
 template <int NT, int K>
-__device__ void ApplyGateK(float2* __restrict__ s, unsigned n,
-                           const qsim_hip_traj_op& o, const float* lm) {
+__device__ void ApplyGateK(float2* __restrict__ s, const qsim_hip_traj_op& o,
+                           const float* lm, uint64_t lo, uint64_t hi) {
   constexpr unsigned D = 1u << K;
-  const uint64_t ngroups = uint64_t{1} << (n - K);
   unsigned q[K];
 #pragma unroll
   for (int b = 0; b < K; ++b) q[b] = o.q[b];
-  for (uint64_t g = threadIdx.x; g < ngroups; g += NT) {
+  for (uint64_t g = lo + threadIdx.x; g < hi; g += NT) {
     uint64_t base = g;
 #pragma unroll
     for (int b = 0; b < K; ++b) {
@@ -119,19 +119,19 @@ __device__ void ZeroState(float2* __restrict__ s, uint64_t N) {
   }
 }
 
-// A fused gate: its FP32 matrix staged in LDS (lm), then one sweep.
+// Groups [lo, hi) of a fused gate, its FP32 matrix staged in LDS (lm).
 template <int NT>
-__device__ void TrajGate(float2* __restrict__ s, unsigned n,
-                         const qsim_hip_traj_op& o,
-                         const float* __restrict__ mats, float* lm) {
+__device__ void TrajGate(float2* __restrict__ s, const qsim_hip_traj_op& o,
+                         const float* __restrict__ mats, float* lm,
+                         uint64_t lo, uint64_t hi) {
   const unsigned D = 1u << o.k;
   for (unsigned i = threadIdx.x; i < 2 * D * D; i += NT) lm[i] = mats[o.moff + i];
   __syncthreads();
   switch (o.k) {
-    case 1: ApplyGateK<NT, 1>(s, n, o, lm); break;
-    case 2: ApplyGateK<NT, 2>(s, n, o, lm); break;
-    case 3: ApplyGateK<NT, 3>(s, n, o, lm); break;
-    default: ApplyGateK<NT, 4>(s, n, o, lm); break;
+    case 1: ApplyGateK<NT, 1>(s, o, lm, lo, hi); break;
+    case 2: ApplyGateK<NT, 2>(s, o, lm, lo, hi); break;
+    case 3: ApplyGateK<NT, 3>(s, o, lm, lo, hi); break;
+    default: ApplyGateK<NT, 4>(s, o, lm, lo, hi); break;
   }
   __syncthreads();
 }
@@ -148,6 +148,44 @@ __device__ void ScaleState(float2* __restrict__ s, uint64_t N, float a) {
     const float2 v = s[i];
     s[i] = float2{v.x * a, v.y * a};
   }
+}
+
+// The 2^NQ amplitudes of group g over ascending qubits q.
+template <int NQ>
+__device__ __forceinline__ void LoadGroup(const float2* __restrict__ s,
+                                          uint64_t g, const uint32_t* q,
+                                          float2 (&v)[1 << NQ]) {
+  const unsigned q0 = q[0], q1 = NQ > 1 ? q[1] : 0;
+  uint64_t base = ((g >> q0) << (q0 + 1)) | (g & ((uint64_t{1} << q0) - 1));
+  if (NQ > 1) {
+    base = ((base >> q1) << (q1 + 1)) | (base & ((uint64_t{1} << q1) - 1));
+  }
+#pragma unroll
+  for (unsigned j = 0; j < (1u << NQ); ++j) {
+    const uint64_t off = ((j & 1u) ? uint64_t{1} << q0 : 0) |
+                         ((j & 2u) ? uint64_t{1} << q1 : 0);
+    v[j] = s[base + off];
+  }
+}
+
+// Re v^dagger (K^dagger K) v, the matrix K^dagger K at lm.
+template <int NQ>
+__device__ __forceinline__ float GroupQuadratic(const float2 (&v)[1 << NQ],
+                                                const float* lm) {
+  constexpr unsigned D = 1u << NQ;
+  float w = 0.0f;
+#pragma unroll
+  for (unsigned r = 0; r < D; ++r) {
+    float re = 0.0f, im = 0.0f;
+#pragma unroll
+    for (unsigned k = 0; k < D; ++k) {
+      const float mr = lm[2 * (r * D + k)], mi = lm[2 * (r * D + k) + 1];
+      re += mr * v[k].x - mi * v[k].y;
+      im += mr * v[k].y + mi * v[k].x;
+    }
+    w += v[r].x * re + v[r].y * im;
+  }
+  return w;
 }
 
 // A channel that the draw's bounds did not decide (header ops[oi], its
@@ -172,7 +210,6 @@ __device__ void TrajChannelQ(float2* __restrict__ s, unsigned n,
   const unsigned M = h.k;
   const uint64_t N = uint64_t{1} << n;
   const uint64_t ngroups = N >> NQ;
-  const unsigned q0 = h.q[0], q1 = NQ > 1 ? h.q[1] : 0;
   const bool normalise = h.pad & 1u;
   bool have_norm = !normalise;
   double norm = 1.0;
@@ -187,30 +224,9 @@ __device__ void TrajChannelQ(float2* __restrict__ s, unsigned n,
     __syncthreads();
     double acc = 0.0, nacc = 0.0;
     for (uint64_t g = threadIdx.x; g < ngroups; g += NT) {
-      uint64_t base =
-          ((g >> q0) << (q0 + 1)) | (g & ((uint64_t{1} << q0) - 1));
-      if (NQ > 1) {
-        base = ((base >> q1) << (q1 + 1)) | (base & ((uint64_t{1} << q1) - 1));
-      }
       float2 v[D];
-#pragma unroll
-      for (unsigned j = 0; j < D; ++j) {
-        const uint64_t off = ((j & 1u) ? uint64_t{1} << q0 : 0) |
-                             ((j & 2u) ? uint64_t{1} << q1 : 0);
-        v[j] = s[base + off];
-      }
-      float w = 0.0f;  // Re v^dagger (K^dagger K) v
-#pragma unroll
-      for (unsigned r = 0; r < D; ++r) {
-        float re = 0.0f, im = 0.0f;
-#pragma unroll
-        for (unsigned k = 0; k < D; ++k) {
-          const float mr = lm[2 * (r * D + k)], mi = lm[2 * (r * D + k) + 1];
-          re += mr * v[k].x - mi * v[k].y;
-          im += mr * v[k].y + mi * v[k].x;
-        }
-        w += v[r].x * re + v[r].y * im;
-      }
+      LoadGroup<NQ>(s, g, h.q, v);
+      const float w = GroupQuadratic<NQ>(v, lm);
       acc += double(w);
       if (!have_norm) {
 #pragma unroll
@@ -267,8 +283,8 @@ __device__ void TrajChannelQ(float2* __restrict__ s, unsigned n,
   for (unsigned e = threadIdx.x; e < 2 * DK * DK; e += NT)
     lm[e] = mats[c.moff + e] * a;
   __syncthreads();
-  if (c.k == 1) ApplyGateK<NT, 1>(s, n, c, lm);
-  else ApplyGateK<NT, 2>(s, n, c, lm);
+  if (c.k == 1) ApplyGateK<NT, 1>(s, c, lm, 0, N >> 1);
+  else ApplyGateK<NT, 2>(s, c, lm, 0, N >> 2);
   __syncthreads();
 }
 
@@ -300,23 +316,17 @@ __device__ __forceinline__ uint32_t PairSigns(uint64_t i,
   return m;
 }
 
-// <Z_a Z_b> = sum_i |s_i|^2 (-1)^(bit a + bit b) / sum_i |s_i|^2 for the
-// trajectory's pairs, FP64-accumulated.  A non-unitary trajectory ends
-// normalised (lib/qtrajectory.h:377-383): its norm goes to norm_out and the
-// scaling is applied where the state is read (qsim_hip_traj_state), which
-// saves a read-write sweep of every state.
-template <int NT>
-__device__ void TrajFinish(const float2* __restrict__ s,
-                           const qsim_hip_traj_desc& d,
-                           const uint32_t* __restrict__ pairs,
-                           double* __restrict__ zz_out,
-                           double* __restrict__ norm_out, double* red) {
-  constexpr unsigned kS = kSweep<NT>;
+// Sums over amplitudes [lo, hi) of |s_i|^2 (-1)^(bit a + bit b) for the
+// trajectory's pairs (FP64) and of |s_i|^2: put(j, sum) for pair j in every
+// thread (valid in thread 0), put(num_pairs, norm) last.  lo is a multiple
+// of kS NT.
+template <int NT, unsigned kS, typename Put>
+__device__ void PairSums(const float2* __restrict__ s,
+                         const qsim_hip_traj_desc& d,
+                         const uint32_t* __restrict__ pairs, uint64_t lo,
+                         uint64_t hi, double* red, Put put) {
   constexpr unsigned kPC = kPairChunk<NT>;
-  const uint64_t N = uint64_t{1} << d.num_qubits;
-  double total = 0.0;  // the norm, in thread 0
-  bool have_norm = false;
-  for (unsigned p0 = 0; p0 < d.num_pairs; p0 += kPC) {
+  for (unsigned p0 = 0; p0 == 0 || p0 < d.num_pairs; p0 += kPC) {
     const unsigned np = std::min(kPC, d.num_pairs - p0);
     unsigned pa[kPC], pb[kPC];
     double acc[kPC];
@@ -333,13 +343,13 @@ __device__ void TrajFinish(const float2* __restrict__ s,
 #pragma unroll
     for (unsigned u = 0; u < kS; ++u) su[u] = PairSigns(uint64_t(u) * NT, pa, pb);
     double nrm = 0.0;
-    for (uint64_t i0 = threadIdx.x; i0 < N; i0 += kS * NT) {
+    for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kS * NT) {
       const uint32_t s0 = PairSigns(i0, pa, pb);
       float2 a[kS];
 #pragma unroll
       for (unsigned u = 0; u < kS; ++u) {
         const uint64_t i = i0 + u * NT;
-        a[u] = i < N ? s[i] : float2{0.0f, 0.0f};
+        a[u] = i < hi ? s[i] : float2{0.0f, 0.0f};
       }
 #pragma unroll
       for (unsigned u = 0; u < kS; ++u) {
@@ -350,34 +360,36 @@ __device__ void TrajFinish(const float2* __restrict__ s,
         for (unsigned j = 0; j < kPC; ++j) acc[j] += (m >> j) & 1u ? -w : w;
       }
     }
-    nrm = BlockSum<NT>(nrm, red);
-    total = nrm;
-    have_norm = true;
     // Unrolled, so that acc stays in registers.
 #pragma unroll
     for (unsigned j = 0; j < kPC; ++j) {
       const double v = BlockSum<NT>(acc[j], red);
-      if (threadIdx.x == 0 && j < np) zz_out[d.pair_offset + p0 + j] = v / nrm;
+      if (j < np) put(p0 + j, v);
     }
+    if (p0 + kPC >= d.num_pairs) put(d.num_pairs, BlockSum<NT>(nrm, red));
   }
-  if (!(d.pad & 1u)) return;
-  if (!have_norm) {
-    double nrm = 0.0;
-    for (uint64_t i0 = threadIdx.x; i0 < N; i0 += kS * NT) {
-      float2 a[kS];
-#pragma unroll
-      for (unsigned u = 0; u < kS; ++u) {
-        const uint64_t i = i0 + u * NT;
-        a[u] = i < N ? s[i] : float2{0.0f, 0.0f};
-      }
-#pragma unroll
-      for (unsigned u = 0; u < kS; ++u) {
-        nrm += double(a[u].x) * a[u].x + double(a[u].y) * a[u].y;
-      }
-    }
-    total = BlockSum<NT>(nrm, red);
-  }
-  if (threadIdx.x == 0) norm_out[blockIdx.x] = total;
+}
+
+// <Z_a Z_b> = sum_i |s_i|^2 (-1)^(bit a + bit b) / sum_i |s_i|^2 for the
+// trajectory's pairs, FP64-accumulated.  A non-unitary trajectory ends
+// normalised (lib/qtrajectory.h:377-383): its norm goes to norm_out and the
+// scaling is applied where the state is read (qsim_hip_traj_state), which
+// saves a read-write sweep of every state.
+template <int NT>
+__device__ void TrajFinish(const float2* __restrict__ s,
+                           const qsim_hip_traj_desc& d,
+                           const uint32_t* __restrict__ pairs,
+                           double* __restrict__ zz_out,
+                           double* __restrict__ norm_out, double* red) {
+  double nrm = 0.0;  // in thread 0
+  PairSums<NT, kSweep<NT>>(s, d, pairs, 0, uint64_t{1} << d.num_qubits, red,
+               [&](unsigned j, double v) {
+                 if (j == d.num_pairs) nrm = v;
+                 else if (threadIdx.x == 0) zz_out[d.pair_offset + j] = v;
+               });
+  if (threadIdx.x != 0) return;
+  for (unsigned j = 0; j < d.num_pairs; ++j) zz_out[d.pair_offset + j] /= nrm;
+  if (d.pad & 1u) norm_out[blockIdx.x] = nrm;
 }
 
 // Workgroup t runs trajectory t, one sweep of the state per operation.  A
@@ -402,7 +414,7 @@ TrajectoryKernel(const qsim_hip_traj_desc* __restrict__ descs,
   for (uint64_t oi = d.op_begin; oi < d.op_end; ++oi) {
     const qsim_hip_traj_op o = ops[oi];
     if (o.kind == QSIM_HIP_TRAJ_GATE) {
-      TrajGate<NT>(s, n, o, mats, lm);
+      TrajGate<NT>(s, o, mats, lm, 0, uint64_t{1} << (n - o.k));
     } else if (o.kind == QSIM_HIP_TRAJ_CHANNEL) {
       TrajChannel<NT>(s, n, ops, oi, mats, dec_out, red, lm, vals);
       oi += o.k;  // its Kraus operators
@@ -419,25 +431,49 @@ struct TrajTilePass {
   uint64_t rec;
 };
 
-// The tiled kernel's shapes (block_tile.h): TB = 13, tiles of up to 13
-// qubits, 256 threads per trajectory, two workgroups per CU; TB = 14, tiles
-// of up to 14 qubits, 512 threads, one workgroup per CU (twice the bytes in
-// flight per trajectory, fewer passes, half as many trajectories at once).
-// One tile pass of the workgroup's trajectory, with the FP16 arithmetic of
-// the circuit kernel's blocked passes (block_kernels.hip): the pass's op
-// records are copied into LDS once, then for every tile of the state the
-// tile is staged in LDS scaled by a power of two (TileScale), the ops run
-// on it (FP16 MFMA, two parts per operand), and it is stored back scaled
-// the other way, with the next tile's loads in flight meanwhile (in two
-// halves around the first ops).  A pass's ops are unitary or Kraus
-// operators (spectral norm <= 1), so the tile never grows.  The tile sits at
-// LDS offset 0 (no static LDS in the kernel, checked on the host).  FULL:
-// tiles of TB qubits.
-template <int TB, bool FULL>
+// ---- the tiled batch: many workgroups per trajectory -----------------------
+//
+// The tiled batch is a sequence of launches (TrajSchedule on the host), each
+// over work items of many trajectories: a run of a trajectory's tiles for a
+// tile pass, a run of its amplitudes for a sweep.  A trajectory advances by
+// one operation per launch, so the end of a launch is the only
+// synchronisation, and a batch of a few large trajectories fills the chip as
+// well as one of many small ones.
+//
+// One workgroup per trajectory with barriers between its operations, which
+// this replaces, streamed each state at 12-15 GB/s and lasted as long as the
+// largest trajectories' serial chains: 100 trajectories each of 20, 18 and
+// 16 qubits, 4 passes of 5 gates: MEASURED
+struct TrajItem {
+  uint32_t traj;
+  uint32_t op;        // operation index
+  uint32_t first;     // first tile (passes) or sweep chunk
+  uint32_t count;     // tiles (passes); channels: chunks of the trajectory
+  uint64_t part;      // partial sums of chunk 0 (channel sums, finish)
+};
+
+// Amplitudes of a sweep chunk.
+constexpr uint64_t kSweepChunk = uint64_t{1} << 14;
+constexpr int kSweepNT = 256;
+// Partial sums of a channel's chunk: one per Kraus operator, then the norm.
+constexpr unsigned kChanSums = kMaxKraus + 1;
+
+// A pass over tiles of up to 13 qubits, with the FP16 arithmetic of the
+// circuit kernel's blocked passes (block_kernels.hip): the pass's op records
+// are copied into LDS once, then every tile of the item is staged in LDS
+// scaled by a power of two (TileScale), the ops run on it and it is stored
+// back scaled the other way, with the next tile's loads in flight meanwhile
+// (in two halves around the first ops); two workgroups a CU.  A pass's ops
+// are unitary or Kraus operators (spectral norm <= 1), so the tile never
+// grows.  The tile sits at LDS offset 0 (no static LDS in the kernel,
+// checked on the host).  FULL: tiles of 13 qubits.
+template <bool FULL>
 __device__ __forceinline__ void TrajTileRun(float2* __restrict__ s,
                                             const TrajTilePass* __restrict__ tp,
                                             const uint32_t* __restrict__ recs,
-                                            char* lds_raw) {
+                                            char* lds_raw, uint64_t first,
+                                            uint64_t end) {
+  constexpr int TB = 13;
   constexpr int NT = BlockShape<TB>::NT;
   constexpr int NW = BlockShape<TB>::kWaves;
   constexpr int PER = 32;
@@ -452,7 +488,6 @@ __device__ __forceinline__ void TrajTileRun(float2* __restrict__ s,
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned nbatch = (1u << g.tb) >> 9;
   const unsigned nper = (1u << g.tb) / NT;
-  __syncthreads();  // the record area was scratch until now
   {
     const unsigned nq = nops * unsigned(kF16RecWords / 4);
     const uint4* src =
@@ -463,15 +498,16 @@ __device__ __forceinline__ void TrajTileRun(float2* __restrict__ s,
   TileIo<PER, NT, true> io;
   io.Init(g);
   float2 buf[PER];
-  io.template Fetch<FULL, 15u>(s, 0, g, buf);  // tile 0 starts at amplitude 0
+  io.template Fetch<FULL, 15u>(
+      s, InsertZeros(first << g.Lc, g.outer, g.nouter), g, buf);
   int e = TileScale<NW>(LocalMax<PER, FULL>(buf, nper), slots, p.headroom);
   io.template PutScaled<FULL>(g, buf, lds, e);
   __syncthreads();
-  for (uint64_t tile = 0; tile < g.ntiles; ++tile) {
+  for (uint64_t tile = first; tile < end; ++tile) {
     const uint64_t base = InsertZeros(tile << g.Lc, g.outer, g.nouter);
     // The next tile, or this one again after the last (an in-bounds read
     // that is never used).
-    const uint64_t next = tile + 1 < g.ntiles ? tile + 1 : tile;
+    const uint64_t next = tile + 1 < end ? tile + 1 : tile;
     const uint64_t nb = InsertZeros(next << g.Lc, g.outer, g.nouter);
     io.template Fetch<FULL, 3u>(s, nb, g, buf);
     for (unsigned op = 0; op < nops; ++op) {
@@ -489,63 +525,260 @@ __device__ __forceinline__ void TrajTileRun(float2* __restrict__ s,
   }
 }
 
-// Workgroup t runs trajectory t with its gate runs as tile passes: one
-// stream of the state per pass instead of one per fused gate.  Gates outside
-// a pass (states under 9 qubits) and channel decisions run as sweeps over
-// the state with the workgroup's threads; their scratch (the gate matrix,
-// the reduction partials) reuses the record area of the LDS.
-template <int TB>
-__global__ void __launch_bounds__(BlockShape<TB>::NT)
+template <bool FULL>
+__global__ void __launch_bounds__(BlockShape<13>::NT)
 __attribute__((amdgpu_waves_per_eu(2)))
-TrajTileKernel(const qsim_hip_traj_desc* __restrict__ descs,
-               const qsim_hip_traj_op* __restrict__ ops,
-               const float* __restrict__ mats,
-               const TrajTilePass* __restrict__ passes,
-               const uint32_t* __restrict__ recs,
-               const uint32_t* __restrict__ pairs, float2* __restrict__ pool,
-               double* __restrict__ zz_out, double* __restrict__ norm_out,
-               int32_t* __restrict__ dec_out) {
-  constexpr int NT = BlockShape<TB>::NT;
+TrajPass13Kernel(const qsim_hip_traj_desc* __restrict__ descs,
+                 const qsim_hip_traj_op* __restrict__ ops,
+                 const TrajTilePass* __restrict__ passes,
+                 const uint32_t* __restrict__ recs,
+                 const TrajItem* __restrict__ items,
+                 float2* __restrict__ pool) {
   extern __shared__ char lds_raw[];
-  // The record area holds the channel and gate scratch between tile passes.
-  char* aux = lds_raw + F16Lds<TB>::kRecOff;
-  constexpr size_t kLmBytes = 2 * 16 * 16 * sizeof(float);
-  static_assert(kLmBytes + (kRedWords<NT> + 2) * sizeof(double) <=
-                    F16Lds<TB>::Bytes(F16Lds<TB>::kMaxOps) - F16Lds<TB>::kRecOff,
-                "scratch fits the record area");
-  float* lm = reinterpret_cast<float*>(aux);
-  double* red = reinterpret_cast<double*>(aux + kLmBytes);
-  double* vals = red + kRedWords<NT>;
-  const qsim_hip_traj_desc d = descs[blockIdx.x];
-  const unsigned n = d.num_qubits;
-  float2* s = pool + d.state_offset;
-  ZeroState<NT>(s, uint64_t{1} << n);
-  __syncthreads();
-  for (uint64_t oi = d.op_begin; oi < d.op_end; ++oi) {
-    const qsim_hip_traj_op o = ops[oi];
-    if (o.kind == QSIM_HIP_TRAJ_GATE) {
-      TrajGate<NT>(s, n, o, mats, lm);
-    } else if (o.kind == QSIM_HIP_TRAJ_TILE_PASS) {
-      if (passes[o.moff].g.tb == TB) {
-        TrajTileRun<TB, true>(s, passes + o.moff, recs, lds_raw);
-      } else {
-        TrajTileRun<TB, false>(s, passes + o.moff, recs, lds_raw);
-      }
-      oi += o.k;  // the pass's gates
-    } else if (o.kind == QSIM_HIP_TRAJ_CHANNEL) {
-      TrajChannel<NT>(s, n, ops, oi, mats, dec_out, red, lm, vals);
-      oi += o.k;  // its Kraus operators
-    }
-  }
-  TrajFinish<NT>(s, d, pairs, zz_out, norm_out, red);
+  const TrajItem it = items[blockIdx.x];
+  TrajTileRun<FULL>(pool + descs[it.traj].state_offset,
+                    passes + ops[it.op].moff, recs, lds_raw, it.first,
+                    uint64_t(it.first) + it.count);
 }
 
-// Dynamic LDS of the tiled kernel: the tile, the scale slots and the
-// records of the longest pass its shape keeps resident.
-template <int TB>
-constexpr size_t TrajLds() {
-  return F16Lds<TB>::Bytes(F16Lds<TB>::kMaxOps);
+// Passes over 14-qubit tiles: the circuit kernel's run (BlockIoRun).
+__global__ void __launch_bounds__(kIoThreads)
+__attribute__((amdgpu_waves_per_eu(3, 3)))
+TrajPass14Kernel(const qsim_hip_traj_desc* __restrict__ descs,
+                 const qsim_hip_traj_op* __restrict__ ops,
+                 const TrajTilePass* __restrict__ passes,
+                 const uint32_t* __restrict__ recs,
+                 const TrajItem* __restrict__ items,
+                 float2* __restrict__ pool) {
+  extern __shared__ char lds_raw[];
+  const TrajItem it = items[blockIdx.x];
+  const TrajTilePass* tp = passes + ops[it.op].moff;
+  BlockIoRun(pool + descs[it.traj].state_offset, tp->g, tp->p,
+             recs + tp->rec * kF16RecWords, lds_raw, it.first,
+             uint64_t(it.first) + it.count, 1);
 }
+
+// Every state to |0...0>: the pool to zeros, then each first amplitude.
+__global__ void __launch_bounds__(kSweepNT)
+TrajZeroKernel(float2* __restrict__ pool, uint64_t size) {
+  const uint64_t stride = uint64_t(gridDim.x) * kSweepNT;
+  for (uint64_t i = uint64_t(blockIdx.x) * kSweepNT + threadIdx.x; i < size;
+       i += stride)
+    pool[i] = float2{0.0f, 0.0f};
+}
+__global__ void __launch_bounds__(kSweepNT)
+TrajOneKernel(const qsim_hip_traj_desc* __restrict__ descs, unsigned num,
+              float2* __restrict__ pool) {
+  const unsigned t = blockIdx.x * kSweepNT + threadIdx.x;
+  if (t < num) pool[descs[t].state_offset] = float2{1.0f, 0.0f};
+}
+
+// Groups [lo, hi) of sweep chunk `chunk` for operators on k qubits.
+__device__ __forceinline__ void SweepGroups(unsigned n, unsigned k,
+                                            uint64_t chunk, uint64_t& lo,
+                                            uint64_t& hi) {
+  const uint64_t all = uint64_t{1} << (n - k), per = kSweepChunk >> k;
+  lo = chunk * per;
+  hi = lo + per < all ? lo + per : all;
+}
+
+__global__ void __launch_bounds__(kSweepNT)
+TrajGateKernel(const qsim_hip_traj_desc* __restrict__ descs,
+               const qsim_hip_traj_op* __restrict__ ops,
+               const float* __restrict__ mats,
+               const TrajItem* __restrict__ items, float2* __restrict__ pool) {
+  __shared__ float lm[2 * 16 * 16];
+  const TrajItem it = items[blockIdx.x];
+  const qsim_hip_traj_op o = ops[it.op];
+  const qsim_hip_traj_desc d = descs[it.traj];
+  uint64_t lo, hi;
+  SweepGroups(d.num_qubits, o.k, it.first, lo, hi);
+  TrajGate<kSweepNT>(pool + d.state_offset, o, mats, lm, lo, hi);
+}
+
+// Partial sums of <psi|K^dagger K|psi> for every non-unitary operator of a
+// channel (all of them: the walk that may stop early comes after), and of
+// the norm where the trajectory is not unitary.
+template <int NQ>
+__device__ void ChannelSums(const float2* __restrict__ s, unsigned n,
+                            const qsim_hip_traj_op* __restrict__ ops,
+                            uint64_t oi, const float* __restrict__ mats,
+                            uint64_t chunk, double* __restrict__ out,
+                            float* lm) {
+  constexpr unsigned D = 1u << NQ;
+  const qsim_hip_traj_op h = ops[oi];
+  uint64_t lo, hi;
+  SweepGroups(n, NQ, chunk, lo, hi);
+  for (unsigned i = 0; i < h.k; ++i) {
+    const qsim_hip_traj_op c = ops[oi + 1 + i];
+    if (c.pad & 1u) continue;  // unitary: decided by its bound alone
+    __syncthreads();           // earlier reads of lm are done
+    for (unsigned e = threadIdx.x; e < 2 * D * D; e += kSweepNT)
+      lm[e] = mats[c.moff2 + e];
+    __syncthreads();
+    double acc = 0.0;
+    for (uint64_t g = lo + threadIdx.x; g < hi; g += kSweepNT) {
+      float2 v[D];
+      LoadGroup<NQ>(s, g, h.q, v);
+      acc += double(GroupQuadratic<NQ>(v, lm));
+    }
+    acc = BlockSum<kSweepNT>(acc);
+    if (threadIdx.x == 0) out[i] = acc;
+  }
+  if (h.pad & 1u) {
+    uint64_t a0, a1;
+    SweepGroups(n, 0, chunk, a0, a1);
+    double acc = 0.0;
+    for (uint64_t i = a0 + threadIdx.x; i < a1; i += kSweepNT) {
+      const float2 v = s[i];
+      acc += double(v.x) * v.x + double(v.y) * v.y;
+    }
+    acc = BlockSum<kSweepNT>(acc);
+    if (threadIdx.x == 0) out[kMaxKraus] = acc;
+  }
+}
+
+__global__ void __launch_bounds__(kSweepNT)
+TrajChannelSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
+                     const qsim_hip_traj_op* __restrict__ ops,
+                     const float* __restrict__ mats,
+                     const TrajItem* __restrict__ items,
+                     const float2* __restrict__ pool,
+                     double* __restrict__ parts) {
+  __shared__ float lm[2 * 4 * 4];
+  const TrajItem it = items[blockIdx.x];
+  const qsim_hip_traj_desc d = descs[it.traj];
+  const float2* s = pool + d.state_offset;
+  double* out = parts + it.part + uint64_t(it.first) * kChanSums;
+  if (ops[it.op].moff2 == 1)
+    ChannelSums<1>(s, d.num_qubits, ops, it.op, mats, it.first, out, lm);
+  else
+    ChannelSums<2>(s, d.num_qubits, ops, it.op, mats, it.first, out, lm);
+}
+
+// The walk of RunIteration (lib/qtrajectory.h:330-370) over the summed
+// probabilities, the same in every workgroup of the trajectory, then the
+// chosen operator on this item's chunk.
+__global__ void __launch_bounds__(kSweepNT)
+TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
+                       const qsim_hip_traj_op* __restrict__ ops,
+                       const float* __restrict__ mats,
+                       const TrajItem* __restrict__ items,
+                       float2* __restrict__ pool,
+                       const double* __restrict__ parts,
+                       int32_t* __restrict__ dec_out) {
+  __shared__ float lm[2 * 4 * 4];
+  __shared__ double sums[kChanSums];
+  const TrajItem it = items[blockIdx.x];
+  const qsim_hip_traj_desc d = descs[it.traj];
+  const qsim_hip_traj_op h = ops[it.op];
+  const bool normalise = h.pad & 1u;
+  for (unsigned i = 0; i < kChanSums; ++i) {
+    const bool need = i == kMaxKraus
+                          ? normalise
+                          : i < h.k && !(ops[it.op + 1 + i].pad & 1u);
+    if (!need) continue;
+    double acc = 0.0;
+    for (unsigned c = threadIdx.x; c < it.count; c += kSweepNT)
+      acc += parts[it.part + uint64_t(c) * kChanSums + i];
+    acc = BlockSum<kSweepNT>(acc);
+    if (threadIdx.x == 0) sums[i] = acc;
+  }
+  __syncthreads();
+  const double norm = normalise ? sums[kMaxKraus] : 1.0;
+  double cp = h.cp, max_prob = 0.0;
+  int max_index = 0, pick = -1;
+  for (unsigned i = 0; i < h.k; ++i) {
+    const qsim_hip_traj_op c = ops[it.op + 1 + i];
+    if (c.pad & 1u) continue;
+    const double prob = sums[i] / norm;
+    if (prob > max_prob) {
+      max_prob = prob;
+      max_index = int(i);
+    }
+    cp += prob - c.r;
+    if (h.r < cp || i == h.k - 1) {
+      pick = h.r < cp ? int(i) : max_index;
+      break;
+    }
+  }
+  if (it.first == 0 && threadIdx.x == 0) dec_out[h.slot] = pick;
+  const float a = normalise ? float(1.0 / std::sqrt(norm)) : 1.0f;
+  float2* s = pool + d.state_offset;
+  const qsim_hip_traj_op c = ops[it.op + 1 + (pick >= 0 ? pick : 0)];
+  uint64_t lo, hi;
+  if (pick < 0 || c.k == 0) {
+    // Nothing applied (or the identity): the state is only normalised.
+    if (!normalise) return;
+    SweepGroups(d.num_qubits, 0, it.first, lo, hi);
+    for (uint64_t i = lo + threadIdx.x; i < hi; i += kSweepNT) {
+      const float2 v = s[i];
+      s[i] = float2{v.x * a, v.y * a};
+    }
+    return;
+  }
+  const unsigned DK = 1u << c.k;
+  for (unsigned e = threadIdx.x; e < 2 * DK * DK; e += kSweepNT)
+    lm[e] = mats[c.moff + e] * a;
+  __syncthreads();
+  SweepGroups(d.num_qubits, c.k, it.first, lo, hi);
+  if (c.k == 1) ApplyGateK<kSweepNT, 1>(s, c, lm, lo, hi);
+  else ApplyGateK<kSweepNT, 2>(s, c, lm, lo, hi);
+}
+
+// Partial sums of a chunk: one per pair, then the norm.
+__global__ void __launch_bounds__(kSweepNT)
+TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
+                    const uint32_t* __restrict__ pairs,
+                    const TrajItem* __restrict__ items,
+                    const float2* __restrict__ pool,
+                    double* __restrict__ parts) {
+  __shared__ double red[kRedWords<kSweepNT>];
+  const TrajItem it = items[blockIdx.x];
+  const qsim_hip_traj_desc d = descs[it.traj];
+  uint64_t lo, hi;
+  SweepGroups(d.num_qubits, 0, it.first, lo, hi);
+  double* out = parts + it.part + uint64_t(it.first) * (d.num_pairs + 1);
+  PairSums<kSweepNT, 8>(pool + d.state_offset, d, pairs, lo, hi, red,
+                        [&](unsigned j, double v) {
+                          if (threadIdx.x == 0) out[j] = v;
+                        });
+}
+
+// <Z_a Z_b> and the norm of one trajectory from its chunks' sums.
+__global__ void __launch_bounds__(kSweepNT)
+TrajFinishKernel(const qsim_hip_traj_desc* __restrict__ descs,
+                 const TrajItem* __restrict__ items,
+                 const double* __restrict__ parts,
+                 double* __restrict__ zz_out, double* __restrict__ norm_out) {
+  __shared__ double norm_s;
+  const TrajItem it = items[blockIdx.x];
+  const qsim_hip_traj_desc d = descs[it.traj];
+  const unsigned np = d.num_pairs;
+  const double* in = parts + it.part;
+  double nrm = 0.0;
+  for (unsigned c = threadIdx.x; c < it.count; c += kSweepNT)
+    nrm += in[uint64_t(c) * (np + 1) + np];
+  nrm = BlockSum<kSweepNT>(nrm);
+  if (threadIdx.x == 0) norm_s = nrm;
+  __syncthreads();
+  nrm = norm_s;
+  if (threadIdx.x == 0 && (d.pad & 1u)) norm_out[it.traj] = nrm;
+  for (unsigned j = threadIdx.x; j < np; j += kSweepNT) {
+    double acc = 0.0;
+    for (unsigned c = 0; c < it.count; ++c) acc += in[uint64_t(c) * (np + 1) + j];
+    zz_out[d.pair_offset + j] = acc / nrm;
+  }
+}
+
+// One launch of a tiled batch.
+struct TrajLaunch {
+  enum Kind { kPass14, kPass13, kPass12, kGate, kChannelSum, kChannelApply,
+              kFinishSum, kFinish } kind;
+  uint64_t first;   // items
+  uint32_t count;
+  unsigned nops;    // passes: the longest program
+};
 
 struct TrajBatch {
   unsigned num_traj = 0;
@@ -562,7 +795,11 @@ struct TrajBatch {
   int32_t* dec = nullptr;
   TrajTilePass* passes = nullptr;
   uint32_t* recs = nullptr;
-  unsigned max_tile_bits = 0;  // over the batch's tile passes
+  // The tiled batch's launches and their items.
+  std::vector<TrajLaunch> launches;
+  TrajItem* items = nullptr;
+  double* parts = nullptr;
+  uint64_t pool_size = 0;  // amplitudes
   std::vector<uint64_t> state_offset;
   std::vector<unsigned> nq;
   hipStream_t gstream = nullptr;
@@ -578,8 +815,8 @@ void LaunchTraj(TrajBatch& b, hipStream_t st) {
                      b.dec);
 }
 
-// The tiled kernel needs more than 64 KiB of dynamic LDS (allowed once per
-// process, outside any stream capture) and addresses its tile from LDS
+// The pass kernels need more than 64 KiB of dynamic LDS (allowed once per
+// process, outside any stream capture) and address the tile from LDS
 // offset 0, which holds only with no static LDS ahead of the dynamic block.
 int TileKernelReady() {
   static std::once_flag once;
@@ -589,9 +826,13 @@ int TileKernelReady() {
     const struct {
       const void* fn;
       size_t lds;
-    } fns[2] = {
-        {reinterpret_cast<const void*>(&TrajTileKernel<13>), TrajLds<13>()},
-        {reinterpret_cast<const void*>(&TrajTileKernel<14>), TrajLds<14>()}};
+    } fns[3] = {
+        {reinterpret_cast<const void*>(&TrajPass13Kernel<true>),
+         F16Lds<13>::Bytes(F16Lds<13>::kMaxOps)},
+        {reinterpret_cast<const void*>(&TrajPass13Kernel<false>),
+         F16Lds<13>::Bytes(F16Lds<13>::kMaxOps)},
+        {reinterpret_cast<const void*>(&TrajPass14Kernel),
+         F16Lds<14>::Bytes(F16Lds<14>::kMaxOps)}};
     for (const auto& f : fns) {
       hipFuncAttributes fa{};
       if (attr == hipSuccess) attr = hipFuncGetAttributes(&fa, f.fn);
@@ -610,6 +851,181 @@ int TileKernelReady() {
   return QSIM_HIP_OK;
 }
 
+// The launches of a tiled batch.  In turn: gates and channels of every
+// trajectory that stands at one, until all stand at a tile pass or at their
+// end; then one pass of every trajectory.  Passes are cut into items of
+// about a quarter of a CU's share of the launch, largest first, so that the
+// last items to run are short; an item's first load and last store are
+// exposed, so it has at least four tiles where the state has.
+void TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
+                  const std::vector<qsim_hip_traj_op>& ops,
+                  const std::vector<TrajTilePass>& passes, unsigned cus,
+                  std::vector<TrajItem>& items,
+                  std::vector<TrajLaunch>& launches, uint64_t& num_parts) {
+  const uint32_t T = uint32_t(d.size());
+  std::vector<uint64_t> at(T);
+  for (uint32_t t = 0; t < T; ++t) at[t] = d[t].op_begin;
+  num_parts = 1;
+  auto chunks = [&](uint32_t t) {
+    const uint64_t N = uint64_t{1} << d[t].num_qubits;
+    return uint32_t(std::max<uint64_t>(1, N / kSweepChunk));
+  };
+  std::vector<TrajItem> list;
+  auto flush = [&](TrajLaunch::Kind kind, unsigned nops) {
+    if (list.empty()) return;
+    launches.push_back({kind, items.size(), uint32_t(list.size()), nops});
+    items.insert(items.end(), list.begin(), list.end());
+    list.clear();
+  };
+  for (;;) {
+    bool pass = false, sweep = false;
+    std::vector<TrajItem> gates, sums, applies;
+    uint64_t part = 0;
+    for (uint32_t t = 0; t < T; ++t) {
+      if (at[t] >= d[t].op_end) continue;
+      const qsim_hip_traj_op& o = ops[at[t]];
+      if (o.kind == QSIM_HIP_TRAJ_TILE_PASS) {
+        pass = true;
+        continue;
+      }
+      sweep = true;
+      const uint32_t nc = chunks(t);
+      if (o.kind == QSIM_HIP_TRAJ_GATE) {
+        for (uint32_t c = 0; c < nc; ++c)
+          gates.push_back({t, uint32_t(at[t]), c, nc, 0});
+        at[t] += 1;
+      } else {
+        for (uint32_t c = 0; c < nc; ++c) {
+          sums.push_back({t, uint32_t(at[t]), c, nc, part});
+        }
+        part += uint64_t(nc) * kChanSums;
+        at[t] += 1 + o.k;
+      }
+    }
+    num_parts = std::max(num_parts, part);
+    if (sweep) {
+      applies = sums;
+      list.swap(gates);
+      flush(TrajLaunch::kGate, 0);
+      list.swap(sums);
+      flush(TrajLaunch::kChannelSum, 0);
+      list.swap(applies);
+      flush(TrajLaunch::kChannelApply, 0);
+      continue;
+    }
+    if (!pass) break;
+    // The tile qubits of the pass each trajectory stands at (0: its end).
+    std::vector<unsigned> tile_bits(T, 0);
+    for (uint32_t t = 0; t < T; ++t) {
+      if (at[t] < d[t].op_end) tile_bits[t] = passes[ops[at[t]].moff].g.tb;
+    }
+    for (const auto kind :
+         {TrajLaunch::kPass14, TrajLaunch::kPass13, TrajLaunch::kPass12}) {
+      uint64_t tiles = 0;
+      unsigned nops = 0;
+      auto takes = [&](uint32_t t) {
+        const unsigned tb = tile_bits[t];
+        return tb != 0 && kind == (tb == 14   ? TrajLaunch::kPass14
+                                   : tb == 13 ? TrajLaunch::kPass13
+                                              : TrajLaunch::kPass12);
+      };
+      std::vector<uint32_t> who;
+      for (uint32_t t = 0; t < T; ++t) {
+        if (!takes(t)) continue;
+        who.push_back(t);
+        const TrajTilePass& tp = passes[ops[at[t]].moff];
+        tiles += tp.g.ntiles;
+        nops = std::max(nops, tp.p.nops);
+      }
+      if (who.empty()) continue;
+      const uint64_t slots = uint64_t(cus) * (kind == TrajLaunch::kPass14 ? 1 : 2);
+      const uint64_t per = std::max<uint64_t>(4, (tiles + 4 * slots - 1) /
+                                                     (4 * slots));
+      for (const uint32_t t : who) {
+        const uint64_t nt = passes[ops[at[t]].moff].g.ntiles;
+        const uint64_t parts = (nt + per - 1) / per;
+        for (uint64_t i = 0; i < parts; ++i) {
+          const uint64_t a = nt * i / parts, b = nt * (i + 1) / parts;
+          list.push_back({t, uint32_t(at[t]), uint32_t(a), uint32_t(b - a), 0});
+        }
+      }
+      std::stable_sort(list.begin(), list.end(),
+                       [](const TrajItem& x, const TrajItem& y) {
+                         return x.count > y.count;
+                       });
+      flush(kind, nops);
+      for (const uint32_t t : who) at[t] += 1 + ops[at[t]].k;
+    }
+  }
+  uint64_t part = 0;
+  std::vector<TrajItem> ends;
+  for (uint32_t t = 0; t < T; ++t) {
+    const uint32_t nc = chunks(t);
+    for (uint32_t c = 0; c < nc; ++c) list.push_back({t, 0, c, nc, part});
+    ends.push_back({t, 0, 0, nc, part});
+    part += uint64_t(nc) * (d[t].num_pairs + 1);
+  }
+  num_parts = std::max(num_parts, part);
+  flush(TrajLaunch::kFinishSum, 0);
+  list.swap(ends);
+  flush(TrajLaunch::kFinish, 0);
+}
+
+int LaunchTiled(TrajBatch& b, hipStream_t st) {
+  const unsigned zb = unsigned(std::min<uint64_t>(
+      (b.pool_size + kSweepNT - 1) / kSweepNT, uint64_t(NumCUs()) * 32));
+  hipLaunchKernelGGL(TrajZeroKernel, dim3(zb), dim3(kSweepNT), 0, st, b.pool,
+                     b.pool_size);
+  hipLaunchKernelGGL(TrajOneKernel,
+                     dim3((b.num_traj + kSweepNT - 1) / kSweepNT),
+                     dim3(kSweepNT), 0, st, b.descs, b.num_traj, b.pool);
+  for (const TrajLaunch& l : b.launches) {
+    const TrajItem* it = b.items + l.first;
+    const dim3 grid(l.count), nt(kSweepNT);
+    switch (l.kind) {
+      case TrajLaunch::kPass14:
+        hipLaunchKernelGGL(TrajPass14Kernel, grid, dim3(kIoThreads),
+                           F16Lds<14>::Bytes(l.nops), st, b.descs, b.ops,
+                           b.passes, b.recs, it, b.pool);
+        break;
+      case TrajLaunch::kPass13:
+        hipLaunchKernelGGL(TrajPass13Kernel<true>, grid,
+                           dim3(BlockShape<13>::NT),
+                           F16Lds<13>::Bytes(l.nops), st, b.descs, b.ops,
+                           b.passes, b.recs, it, b.pool);
+        break;
+      case TrajLaunch::kPass12:
+        hipLaunchKernelGGL(TrajPass13Kernel<false>, grid,
+                           dim3(BlockShape<13>::NT),
+                           F16Lds<13>::Bytes(l.nops), st, b.descs, b.ops,
+                           b.passes, b.recs, it, b.pool);
+        break;
+      case TrajLaunch::kGate:
+        hipLaunchKernelGGL(TrajGateKernel, grid, nt, 0, st, b.descs, b.ops,
+                           b.mats, it, b.pool);
+        break;
+      case TrajLaunch::kChannelSum:
+        hipLaunchKernelGGL(TrajChannelSumKernel, grid, nt, 0, st, b.descs,
+                           b.ops, b.mats, it, b.pool, b.parts);
+        break;
+      case TrajLaunch::kChannelApply:
+        hipLaunchKernelGGL(TrajChannelApplyKernel, grid, nt, 0, st, b.descs,
+                           b.ops, b.mats, it, b.pool, b.parts, b.dec);
+        break;
+      case TrajLaunch::kFinishSum:
+        hipLaunchKernelGGL(TrajFinishSumKernel, grid, nt, 0, st, b.descs,
+                           b.pairs, it, b.pool, b.parts);
+        break;
+      case TrajLaunch::kFinish:
+        hipLaunchKernelGGL(TrajFinishKernel, grid, nt, 0, st, b.descs, it,
+                           b.parts, b.zz, b.norms);
+        break;
+    }
+  }
+  QHIP_LAUNCHED("tiled trajectory batch");
+  return QSIM_HIP_OK;
+}
+
 int Launch(TrajBatch& b, unsigned threads, hipStream_t st) {
   switch (threads) {
     case 256: LaunchTraj<256>(b, st); break;
@@ -617,20 +1033,7 @@ int Launch(TrajBatch& b, unsigned threads, hipStream_t st) {
     case 1024: LaunchTraj<1024>(b, st); break;
     case QSIM_HIP_TRAJ_TILED:
       QHIP_TRY(TileKernelReady());
-      // The 14-qubit shape when a pass needs it.
-      if (b.max_tile_bits == 14) {
-        hipLaunchKernelGGL(TrajTileKernel<14>, dim3(b.num_traj),
-                           dim3(BlockShape<14>::NT), TrajLds<14>(), st,
-                           b.descs, b.ops, b.mats, b.passes, b.recs, b.pairs,
-                           b.pool, b.zz, b.norms, b.dec);
-      } else {
-        hipLaunchKernelGGL(TrajTileKernel<13>, dim3(b.num_traj),
-                           dim3(BlockShape<13>::NT), TrajLds<13>(), st,
-                           b.descs, b.ops, b.mats, b.passes, b.recs, b.pairs,
-                           b.pool, b.zz, b.norms, b.dec);
-      }
-      QHIP_LAUNCHED("TrajTileKernel");
-      return QSIM_HIP_OK;
+      return LaunchTiled(b, st);
     default:
       SetError("trajectory batches run with 256, 512 or 1024 threads or "
                "tiled (%u), not %u", unsigned(QSIM_HIP_TRAJ_TILED), threads);
@@ -797,6 +1200,8 @@ void Release(TrajBatch* b) {
   (void)hipFree(b->dec);
   (void)hipFree(b->passes);
   (void)hipFree(b->recs);
+  (void)hipFree(b->items);
+  (void)hipFree(b->parts);
   delete b;
 }
 
@@ -922,9 +1327,11 @@ static int TrajPrepare(const qsim_hip_traj_desc* trajs, unsigned num_traj,
   // Released (device buffers included) on every early return or exception.
   std::unique_ptr<TrajBatch, void (*)(TrajBatch*)> b(new TrajBatch, Release);
   b->num_traj = num_traj;
-  for (const TrajTilePass& tp : passes) {
-    b->max_tile_bits = std::max(b->max_tile_bits, tp.g.tb);
-  }
+  std::vector<TrajItem> items;
+  uint64_t num_parts = 0;
+  TrajSchedule(d, ov, passes, unsigned(NumCUs()), items, b->launches,
+               num_parts);
+  b->pool_size = pool;
   b->num_pairs = num_pairs;
   b->num_decisions = num_decisions;
   for (unsigned t = 0; t < num_traj; ++t) {
@@ -936,12 +1343,14 @@ static int TrajPrepare(const qsim_hip_traj_desc* trajs, unsigned num_traj,
   if (rc == QSIM_HIP_OK) rc = Upload(&b->ops, ov.data(), num_ops);
   if (rc == QSIM_HIP_OK) rc = Upload(&b->passes, passes.data(), passes.size());
   if (rc == QSIM_HIP_OK) rc = Upload(&b->recs, recs.data(), recs.size());
+  if (rc == QSIM_HIP_OK) rc = Upload(&b->items, items.data(), items.size());
   if (rc == QSIM_HIP_OK) rc = Upload(&b->mats, matrices, num_floats);
   if (rc == QSIM_HIP_OK) rc = Upload(&b->pairs, pairs, size_t(2) * num_pairs);
   if (rc == QSIM_HIP_OK) {
     hipError_t e = hipMalloc(&b->pool, pool * sizeof(float2));
     if (e == hipSuccess) e = hipMalloc(&b->zz, std::max<size_t>(num_pairs, 1) * 8);
     if (e == hipSuccess) e = hipMalloc(&b->norms, size_t(num_traj) * 8);
+    if (e == hipSuccess) e = hipMalloc(&b->parts, num_parts * sizeof(double));
     if (e == hipSuccess)
       e = hipMalloc(&b->dec, std::max<size_t>(num_decisions, 1) * 4);
     if (e != hipSuccess) rc = HipFail(e, "trajectory batch buffers");
