@@ -442,9 +442,10 @@ class StateSpace:
             mask |= 1 << q
         pn = np.cumsum(self.partial_norms(s))
         r = rgen_draw(pn[-1])
-        m = 0
-        while r > pn[m]:
-            m += 1
+        # The first m with r <= pn[m] (a NaN draw: 0).
+        m = int(np.searchsorted(pn, r)) if r > pn[0] else 0
+        if m == len(pn):
+            raise IndexError("measurement draw past the norm")
         if m > 0:
             r -= pn[m - 1]
         bits = self.find_measured_bits(s, m, r, mask)

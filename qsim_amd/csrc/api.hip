@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <random>
 #include <vector>
 
@@ -36,6 +37,7 @@ struct Device {
   bool mat_ev_used[kSlots] = {};
   int mat_next = 0;
   hipEvent_t ev[64] = {};
+  char* result = nullptr;  // HostResult()
 };
 
 std::mutex g_init_mu;
@@ -114,6 +116,8 @@ static int InitDevice(int device) {
                                        hipEventDisableTiming));
   }
   for (int i = 0; i < 64; ++i) QHIP_CHECK(hipEventCreate(&g_dev.ev[i]));
+  QHIP_CHECK(hipHostMalloc(&g_dev.result, kHostResultBytes,
+                           hipHostMallocDefault));
   QHIP_TRY(InitStaticScratch());
   g_dev.ready = true;
   return QSIM_HIP_OK;
@@ -129,6 +133,8 @@ hipStream_t Stream() { return g_stream; }
 int NumCUs() { return g_dev.cus; }
 
 std::mutex& ScratchLock() { return g_scratch_mu; }
+
+void* HostResult() { return g_dev.result; }
 
 void* DeviceScratch(size_t bytes) {
   if (bytes <= g_dev.scratch_size) return g_dev.scratch;
@@ -247,6 +253,32 @@ int CheckStateArgs(int prec, const void* s, unsigned n) {
 int CheckState(int prec, const void* s, unsigned n) {
   QHIP_TRY(CheckStateArgs(prec, s, n));
   return FlushGateQueue();
+}
+
+// Sorts values that are uniform over [0, 1): one counting pass into as many
+// buckets as values, then insertion (a bucket holds one value on average).
+// 20000 values: about 0.2 ms instead of std::sort's 1 ms.
+void SortUniform(std::vector<double>& v) {
+  const size_t n = v.size();
+  if (n < 64 || n > (size_t{1} << 28)) {
+    std::sort(v.begin(), v.end());
+    return;
+  }
+  auto bucket = [n](double x) {
+    return std::min(size_t(x * double(n)), n - 1);
+  };
+  std::vector<uint32_t> at(n + 1, 0);
+  for (double x : v) ++at[bucket(x) + 1];
+  for (size_t i = 1; i <= n; ++i) at[i] += at[i - 1];
+  std::vector<double> w(n);
+  for (double x : v) w[at[bucket(x)]++] = x;
+  for (size_t i = 1; i < n; ++i) {
+    const double x = w[i];
+    size_t j = i;
+    for (; j > 0 && w[j - 1] > x; --j) w[j] = w[j - 1];
+    w[j] = x;
+  }
+  v.swap(w);
 }
 
 uint64_t ElemBytes(int prec) { return prec == QSIM_HIP_F32 ? 4 : 8; }
@@ -565,18 +597,32 @@ int qsim_hip_sample(int prec, const void* s, unsigned n, const double* draws,
 int qsim_hip_sample_seeded(int prec, const void* s, unsigned n, uint64_t num,
                            unsigned seed, uint64_t* out) {
   return GuardHost([&]() -> int {
-    if (num == 0) return CheckState(prec, s, n);
-    double norm = 0;
-    QHIP_TRY(qsim_hip_norm(prec, s, n, &norm));
-    // The draws of lib/util.h:67-85 (mt19937, uniform_real_distribution, sort).
+    QHIP_TRY(CheckState(prec, s, n));
+    if (num == 0) return QSIM_HIP_OK;
+    if (out == nullptr) {
+      SetError("null sample buffers");
+      return QSIM_HIP_ERR_ARG;
+    }
+    if (num > (uint64_t{1} << 31)) {
+      SetError("too many samples");
+      return QSIM_HIP_ERR_ARG;
+    }
+    // The draws of lib/util.h:67-85 (mt19937, uniform_real_distribution over
+    // [0, norm), sorted) are drawn and sorted over [0, 1) while the device
+    // makes the norm, and scaled by it after: the distribution is the
+    // canonical draw times the norm, and rounding keeps the order.
     std::vector<double> rs;
-    rs.reserve(num + 1);
-    std::mt19937 rgen(seed);
-    std::uniform_real_distribution<double> distr(0.0, norm);
-    for (uint64_t i = 0; i < num; ++i) rs.push_back(distr(rgen));
-    std::sort(rs.begin(), rs.end());
-    rs.push_back(norm);
-    return qsim_hip_sample(prec, s, n, rs.data(), num, out);
+    auto draws = [&]() {
+      rs.resize(num);
+      std::mt19937 rgen(seed);
+      std::uniform_real_distribution<double> distr(0.0, 1.0);
+      for (double& r : rs) r = distr(rgen);
+      SortUniform(rs);
+    };
+    return QHIP_DISPATCH(
+        prec,
+        SampleSeeded<float>((const float2*)s, n, num, draws, rs, out),
+        SampleSeeded<double>((const double2*)s, n, num, draws, rs, out));
   });
 }
 

@@ -203,8 +203,61 @@ GateLaneKernel(typename Cplx<FP>::T* __restrict__ s, LaneGeom g, M m) {
   }
 }
 
-// <psi|U|psi> partial sums; any target positions (reads through the cache
-// hierarchy, like the gate kernels' register path).
+// <psi|U|psi>; products in FP, sums in FP64 (lib/simulator_basic.h:316-317).
+template <typename C>
+__device__ __forceinline__ void AddExpectation(Dbl2& acc, const C& v,
+                                               const C& u) {
+  // conj(v) * u
+  acc.x += double(v.x * u.x + v.y * u.y);
+  acc.y += double(v.x * u.y - v.y * u.x);
+}
+
+// The gate kernels' read side (GateLaneKernel): runs of 64 amplitudes, low
+// targets swapped into registers; bound by the read (27 qubits: 180 us, 6
+// TB/s).  Group by group through the caches (ExpectationKernel): 205 us for
+// k = 1, and 6 us for the final sum and 4 us for its copy in launches of
+// their own.
+template <typename FP, int K, typename M>
+__global__ void __launch_bounds__(256)
+ExpectationLaneKernel(const typename Cplx<FP>::T* __restrict__ s, LaneGeom g,
+                      M m, Dbl2* __restrict__ partials) {
+  using C = typename Cplx<FP>::T;
+  constexpr int D = 1 << K;
+  const unsigned lane = threadIdx.x & 63;
+  const uint64_t stride = uint64_t(gridDim.x) * 4;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Dbl2 acc;
+  auto load = [&](uint64_t c, C(&v)[D]) {
+    const C* p = s + InsertZeros(c << 6, g.ins, g.nins);
+#pragma unroll
+    for (int j = 0; j < D; ++j) v[j] = p[MemberOffset<K>(j, g.roff) + lane];
+  };
+  auto add = [&](C(&v)[D]) {
+    SwapLowTargets<K, 0>(v, g);
+    MatVec<FP, K>(v, m, [&](int r, C u) { AddExpectation(acc, v[r], u); });
+  };
+  uint64_t c = uint64_t(blockIdx.x) * 4 + wave;
+  if constexpr (K == 2) {
+    // Four chunks' loads in flight: 178 us a 27-qubit term against 190; k = 1
+    // is better without (180 against 201).
+    for (; c + 3 * stride < g.nchunks; c += 4 * stride) {
+      C v[4][D];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) load(c + k * stride, v[k]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) add(v[k]);
+    }
+  }
+  for (; c < g.nchunks; c += stride) {
+    C v[D];
+    load(c, v);
+    add(v);
+  }
+  acc = BlockSum<256>(acc);
+  if (threadIdx.x == 0) partials[blockIdx.x] = acc;
+}
+
+// Any sizes (k = 5, 6, and small states): one group per work item.
 template <typename FP, int K, typename M>
 __global__ void __launch_bounds__(256)
 ExpectationKernel(const typename Cplx<FP>::T* __restrict__ s, GateGeom g, M m,
@@ -219,12 +272,7 @@ ExpectationKernel(const typename Cplx<FP>::T* __restrict__ s, GateGeom g, M m,
     C v[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) v[j] = s[base + MemberOffset<K>(j, g.tbit)];
-    MatVec<FP, K>(v, m, [&](int r, C u) {
-      // conj(v_r) * (U v)_r: products in FP, sums in FP64
-      // (lib/simulator_basic.h:316-317).
-      acc.x += double(v[r].x * u.x + v[r].y * u.y);
-      acc.y += double(v[r].x * u.y - v[r].y * u.x);
-    });
+    MatVec<FP, K>(v, m, [&](int r, C u) { AddExpectation(acc, v[r], u); });
   }
   acc = BlockSum<256>(acc);
   if (threadIdx.x == 0) partials[blockIdx.x] = acc;
@@ -458,10 +506,27 @@ int DispatchK(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
   else return LaunchTile<FP, K>(s, g, mp);
 }
 
-template <typename FP, int K>
-int DispatchExpectation(const typename Cplx<FP>::T* s, unsigned n,
-                        const unsigned* qs, const FP* m, double* re,
-                        double* im) {
+// Workgroups of an expectation pass: four waves each, at most eight
+// workgroups a CU of 256.
+constexpr unsigned kExpectBlocks = 2048;
+
+static_assert(kExpectBlocks * sizeof(Dbl2) <= kHostResultBytes, "partials");
+
+// Returns the number of partial sums, one per workgroup, in `partials`.
+template <typename FP, int K, typename M>
+unsigned LaunchExpect(const typename Cplx<FP>::T* s, unsigned n,
+                  const unsigned* qs, const M& m, Dbl2* partials) {
+  if constexpr (K <= 4) {
+    LaneGeom lg;
+    if (LaneGeometry<FP>(n, qs, K, nullptr, 0, 0, lg)) {
+      const uint64_t blocks =
+          std::min<uint64_t>((lg.nchunks + 3) / 4, kExpectBlocks);
+      hipLaunchKernelGGL((ExpectationLaneKernel<FP, K, M>),
+                         dim3(unsigned(blocks)), dim3(256), 0, Stream(), s, lg,
+                         m, partials);
+      return unsigned(blocks);
+    }
+  }
   GateGeom g{};
   g.nins = K;
   for (int b = 0; b < K; ++b) {
@@ -469,41 +534,42 @@ int DispatchExpectation(const typename Cplx<FP>::T* s, unsigned n,
     g.tbit[b] = uint64_t{1} << qs[b];
   }
   g.ngroups = uint64_t{1} << (n - K);
-  g.cbits = 0;
+  const uint64_t blocks = std::max<uint64_t>(
+      1, std::min<uint64_t>((g.ngroups + 255) / 256, kExpectBlocks));
+  hipLaunchKernelGGL((ExpectationKernel<FP, K, M>), dim3(unsigned(blocks)),
+                     dim3(256), 0, Stream(), s, g, m, partials);
+  return unsigned(blocks);
+}
 
+template <typename FP, int K>
+int DispatchExpectation(const typename Cplx<FP>::T* s, unsigned n,
+                        const unsigned* qs, const FP* m, double* re,
+                        double* im) {
   std::lock_guard<std::mutex> lock(ScratchLock());
-  const unsigned max_blocks = 1024;
-  uint64_t blocks = std::min<uint64_t>((g.ngroups + 255) / 256, max_blocks);
-  blocks = std::max<uint64_t>(blocks, 1);
-  Dbl2* partials = static_cast<Dbl2*>(DeviceScratch(sizeof(Dbl2) * (blocks + 1)));
-  if (partials == nullptr) return QSIM_HIP_ERR_OOM;
-
-  MatVal<FP, K> mv;
-  MatPtr<FP> mp{nullptr};
-  constexpr bool byval = kByValue<FP, K>;
-  if constexpr (byval) {
-    std::memcpy(mv.v, m, sizeof(mv.v));
-    hipLaunchKernelGGL((ExpectationKernel<FP, K, MatVal<FP, K>>),
-                       dim3(unsigned(blocks)), dim3(256), 0, Stream(), s, g, mv,
-                       partials + 1);
-  } else {
-    size_t bytes = sizeof(FP) * (size_t{2} << (2 * K));
-    void* d = MatrixBuffer(bytes);
-    if (d == nullptr) return QSIM_HIP_ERR_OOM;
-    QHIP_TRY(StageMatrix(d, m, bytes));
-    mp.p = static_cast<const FP*>(d);
-    hipLaunchKernelGGL((ExpectationKernel<FP, K, MatPtr<FP>>),
-                       dim3(unsigned(blocks)), dim3(256), 0, Stream(), s, g, mp,
-                       partials + 1);
+  Dbl2* partials = static_cast<Dbl2*>(HostResult());
+  unsigned count = 0;
+  int rc = QSIM_HIP_ERR_UNSUPPORTED;
+  if constexpr (K == 4 && sizeof(FP) == 4) {
+    rc = LaunchExpectationMfma(s, n, qs, m, partials, kExpectBlocks, &count);
+    if (rc != QSIM_HIP_OK && rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
   }
-  QHIP_LAUNCHED("ExpectationKernel");
-  hipLaunchKernelGGL((FinalSumKernel<Dbl2>), dim3(1), dim3(256), 0, Stream(),
-                     partials + 1, unsigned(blocks), partials);
-  QHIP_LAUNCHED("FinalSumKernel");
+  if (rc != QSIM_HIP_OK) {
+    if constexpr (kByValue<FP, K>) {
+      MatVal<FP, K> mv;
+      std::memcpy(mv.v, m, sizeof(mv.v));
+      count = LaunchExpect<FP, K>(s, n, qs, mv, partials);
+    } else {
+      size_t bytes = sizeof(FP) * (size_t{2} << (2 * K));
+      void* d = MatrixBuffer(bytes);
+      if (d == nullptr) return QSIM_HIP_ERR_OOM;
+      QHIP_TRY(StageMatrix(d, m, bytes));
+      MatPtr<FP> mp{static_cast<const FP*>(d)};
+      count = LaunchExpect<FP, K>(s, n, qs, mp, partials);
+    }
+  }
+  QHIP_LAUNCHED("expectation kernel");
   Dbl2 r;
-  QHIP_CHECK(hipMemcpyAsync(&r, partials, sizeof(Dbl2), hipMemcpyDeviceToHost,
-                            Stream()));
-  QHIP_CHECK(hipStreamSynchronize(Stream()));
+  QHIP_TRY(HostTotal(count, &r));
   *re = r.x;
   *im = r.y;
   return QSIM_HIP_OK;

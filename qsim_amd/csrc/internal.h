@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -56,6 +57,11 @@ hipStream_t Stream();
 // hold ScratchLock()).  Returns nullptr and sets the error on failure.
 void* DeviceScratch(size_t bytes);
 std::mutex& ScratchLock();
+
+// Host memory that kernels write results to (read after a stream
+// synchronisation); belongs to the holder of ScratchLock().
+constexpr size_t kHostResultBytes = 32768;
+void* HostResult();
 
 // Device buffer for gate matrices too large to travel as kernel arguments.
 void* MatrixBuffer(size_t bytes);
@@ -214,6 +220,13 @@ template <typename FP>
 int Sample(const CT<FP>* s, unsigned n, const double* draws, uint64_t num,
            uint64_t* out);
 
+// `num` samples for draws over [0, 1): draws() fills rs with them, sorted,
+// while the device sums the state; they are scaled by the norm.
+template <typename FP>
+int SampleSeeded(const CT<FP>* s, unsigned n, uint64_t num,
+                 const std::function<void()>& draws, std::vector<double>& rs,
+                 uint64_t* out);
+
 template <typename FP>
 int Gather(const CT<FP>* s, const uint64_t* idx, uint64_t count, CT<FP>* out);
 
@@ -224,6 +237,14 @@ int Convert(void* dst, int dprec, const void* src, int sprec, unsigned n);
 // QSIM_HIP_ERR_UNSUPPORTED when the method cannot handle the gate.
 int LaunchGateMfma(float2* s, unsigned n, const unsigned* qs, unsigned k,
                    const double* m64, int method);
+
+// <psi|U|psi> for a 4-qubit operator on a complex64 state, the product on
+// FP32 MFMA: one launch of at most max_blocks workgroups, whose partial sums
+// go to `partials`; *count of them.  QSIM_HIP_ERR_UNSUPPORTED when the state
+// is too small.
+int LaunchExpectationMfma(const float2* s, unsigned n, const unsigned* qs,
+                          const float* m, Dbl2* partials, unsigned max_blocks,
+                          unsigned* count);
 
 // FP16 MFMA with per-group scaling for uncontrolled k = 5, 6 gates on
 // complex64 states (f16_kernels.hip); QSIM_HIP_ERR_UNSUPPORTED when the

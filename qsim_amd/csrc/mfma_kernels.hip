@@ -43,6 +43,7 @@
 
 #include "internal.h"
 #include "lane.h"
+#include "reduce.h"
 #include "tile.h"
 
 namespace qhip {
@@ -289,6 +290,32 @@ GateMfmaTileKernel(float2* __restrict__ s, TileGeom g,
 // groups) and 0.95-1.06 / 0.93 / 0.80-0.87 / 0.80 (LDS tile); 20 qubits:
 // 8-11 us for 8-18.  Three waves a SIMD keep the registers for all 16 loads
 // in flight (two: 0.83 ms with 4 low targets; four spill).
+// u = U v for the wave's 64 groups (lanes), 16 members in registers; v is
+// left with its lanes exchanged (TradeLanes<5> of a member's parts undoes it).
+__device__ __forceinline__ void LaneProduct(const RegFragF32<4>& af,
+                                            float2 (&v)[16],
+                                            float2 (&u)[16]) {
+  v16f c0 = v16f{}, c1 = v16f{};
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    TradeLanes<5>(v[t].x, v[t].y);
+    c0 = __builtin_amdgcn_mfma_f32_32x32x2f32(af(0, t), v[t].x, c0, 0, 0, 0);
+    c1 = __builtin_amdgcn_mfma_f32_32x32x2f32(af(0, t), v[t].y, c1, 0, 0, 0);
+  }
+  // Register 4 q + 2 w + component of both: members 4 q + w, 4 q + 2 + w.
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      float2 x{c0[4 * q + 2 * w], c0[4 * q + 2 * w + 1]};
+      float2 y{c1[4 * q + 2 * w], c1[4 * q + 2 * w + 1]};
+      TradeLanes<5>(x.x, y.x);
+      TradeLanes<5>(x.y, y.y);
+      u[4 * q + w] = x;
+      u[4 * q + 2 + w] = y;
+    }
+}
+
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(3)))
 GateMfmaLaneKernel(float2* __restrict__ s, LaneGeom g,
@@ -301,33 +328,47 @@ GateMfmaLaneKernel(float2* __restrict__ s, LaneGeom g,
   for (uint64_t c = uint64_t(blockIdx.x) * kWaves + wave; c < g.nchunks;
        c += wstride) {
     float2* p = s + InsertZeros(c << 6, g.ins, g.nins);
-    float2 v[16];
+    float2 v[16], u[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) v[j] = p[MemberOffset<4>(j, g.roff) + lane];
     SwapLowTargets<4, 0>(v, g);
-    v16f c0 = v16f{}, c1 = v16f{};
+    LaneProduct(af, v, u);
+    SwapLowTargets<4, 0>(u, g);
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      TradeLanes<5>(v[t].x, v[t].y);
-      c0 = __builtin_amdgcn_mfma_f32_32x32x2f32(af(0, t), v[t].x, c0, 0, 0, 0);
-      c1 = __builtin_amdgcn_mfma_f32_32x32x2f32(af(0, t), v[t].y, c1, 0, 0, 0);
-    }
-    // Register 4 q + 2 u + component of both: members 4 q + u, 4 q + 2 + u.
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float2 x{c0[4 * q + 2 * u], c0[4 * q + 2 * u + 1]};
-        float2 y{c1[4 * q + 2 * u], c1[4 * q + 2 * u + 1]};
-        TradeLanes<5>(x.x, y.x);
-        TradeLanes<5>(x.y, y.y);
-        v[4 * q + u] = x;
-        v[4 * q + 2 + u] = y;
-      }
-    SwapLowTargets<4, 0>(v, g);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) p[MemberOffset<4>(j, g.roff) + lane] = v[j];
+    for (int j = 0; j < 16; ++j) p[MemberOffset<4>(j, g.roff) + lane] = u[j];
   }
+}
+
+// <psi|U|psi> with the same product: FP32 products, FP64 sums.  27 qubits:
+// 215-270 us; on the vector unit, whose products bound it, 415-450 us.
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(3)))
+ExpectationMfmaKernel(const float2* __restrict__ s, LaneGeom g,
+                      const float* __restrict__ frag,
+                      Dbl2* __restrict__ partials) {
+  const unsigned lane = threadIdx.x & 63;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  RegFragF32<4> af;
+  af.Load(frag);
+  Dbl2 acc;
+  const uint64_t wstride = uint64_t(gridDim.x) * kWaves;
+  for (uint64_t c = uint64_t(blockIdx.x) * kWaves + wave; c < g.nchunks;
+       c += wstride) {
+    const float2* p = s + InsertZeros(c << 6, g.ins, g.nins);
+    float2 v[16], u[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = p[MemberOffset<4>(j, g.roff) + lane];
+    SwapLowTargets<4, 0>(v, g);
+    LaneProduct(af, v, u);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      TradeLanes<5>(v[j].x, v[j].y);
+      acc.x += double(v[j].x * u[j].x + v[j].y * u[j].y);
+      acc.y += double(v[j].x * u[j].y - v[j].y * u[j].x);
+    }
+  }
+  acc = BlockSum<256>(acc);
+  if (threadIdx.x == 0) partials[blockIdx.x] = acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -606,6 +647,28 @@ int DispatchMfma(float2* s, unsigned n, const unsigned* qs, const double* m64,
 }
 
 }  // namespace
+
+int LaunchExpectationMfma(const float2* s, unsigned n, const unsigned* qs,
+                          const float* m, Dbl2* partials, unsigned max_blocks,
+                          unsigned* count) {
+  LaneGeom g;
+  if (!LaneGeometry<float>(n, qs, 4, nullptr, 0, 0, g)) {
+    return QSIM_HIP_ERR_UNSUPPORTED;
+  }
+  double m64[512];
+  std::copy(m, m + 512, m64);
+  float frag[16 * 64];
+  BuildFragF32(4, m64, frag);
+  void* d = MatrixBuffer(sizeof(frag));
+  if (d == nullptr) return QSIM_HIP_ERR_OOM;
+  QHIP_TRY(StageMatrix(d, frag, sizeof(frag)));
+  const uint64_t blocks =
+      std::min<uint64_t>((g.nchunks + kWaves - 1) / kWaves, max_blocks);
+  hipLaunchKernelGGL(ExpectationMfmaKernel, dim3(unsigned(blocks)), dim3(256),
+                     0, Stream(), s, g, static_cast<const float*>(d), partials);
+  *count = unsigned(blocks);
+  return QSIM_HIP_OK;
+}
 
 int LaunchGateMfma(float2* s, unsigned n, const unsigned* qs, unsigned k,
                    const double* m64, int method) {

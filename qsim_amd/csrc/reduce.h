@@ -81,4 +81,27 @@ FinalSumKernel(const Acc* __restrict__ partials, unsigned count,
   if (threadIdx.x == 0) out[0] = acc;
 }
 
+// The end of a reduction whose kernel stored its workgroups' partial sums in
+// host memory (HostResult): waits for the stream and adds them in
+// FinalSumKernel's order (to the bit: the no-allocation entry point, which
+// keeps its sums on the device, returns the same).  A launch for the final
+// sum and the copy of its result took 12 us beside the sweep; a last
+// workgroup that adds up, with the device-wide fence every workgroup then
+// needs, 50 ns per workgroup.
+inline int HostTotal(unsigned count, Dbl2* total) {
+  QHIP_CHECK(hipStreamSynchronize(Stream()));
+  const Dbl2* part = static_cast<const Dbl2*>(HostResult());
+  Dbl2 v[256];
+  for (unsigned i = 0; i < count; ++i) v[i & 255u] += part[i];
+  // Four waves' butterflies, then that of their sums.
+  for (unsigned o = 32; o > 0; o >>= 1)
+    for (unsigned w = 0; w < 4; ++w)
+      for (unsigned l = 0; l < o; ++l) v[64 * w + l] += v[64 * w + l + o];
+  v[0] += v[128];
+  v[64] += v[192];
+  v[0] += v[64];
+  *total = v[0];
+  return QSIM_HIP_OK;
+}
+
 }  // namespace qhip
