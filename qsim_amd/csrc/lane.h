@@ -41,10 +41,22 @@ struct LaneGeom {
   unsigned cvals;
 };
 
+// The value of lane ^ 2^B, B < 4: cross-lane moves within rows of 16.
+template <int B>
+__device__ __forceinline__ unsigned PullLane(unsigned v) {
+  static_assert(B < 4, "row of 16 lanes");
+  // quad_perm [1,0,3,2] and [2,3,0,1]; half mirror (^ 7) after quad_perm
+  // [3,2,1,0] (^ 3); rotation by 8.
+  constexpr int kCtrl[4] = {0xB1, 0x4E, 0x141, 0x128};
+  if (B == 2) v = __builtin_amdgcn_update_dpp(0, v, 0x1B, 0xf, 0xf, true);
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl[B], 0xf, 0xf, true);
+}
+
 // Swaps lane bit B of `lo` with the register bit that tells `lo` from `up`:
 // the lanes of `lo` with bit B set trade places with the lanes of `up`
 // without it (lane ^ 2^B).  Lane bits 5 and 4 are one instruction; the
-// others pull through the LDS crossbar.
+// others move within a row, without ds_bpermute's latency and registers (28
+// qubits, k = 3, 4 with 2-4 low targets: 1-3 % less).
 template <int B>
 __device__ __forceinline__ void TradeLanes(unsigned& lo, unsigned& up) {
   if constexpr (B == 5) {
@@ -56,10 +68,8 @@ __device__ __forceinline__ void TradeLanes(unsigned& lo, unsigned& up) {
     lo = r[0];
     up = r[1];
   } else {
-    const unsigned lane = threadIdx.x & 63;
-    const bool hi = (lane >> B) & 1u;
-    const unsigned x = unsigned(__builtin_amdgcn_ds_bpermute(
-        int((lane ^ (1u << B)) * 4), int(hi ? lo : up)));
+    const bool hi = (threadIdx.x >> B) & 1u;
+    const unsigned x = PullLane<B>(hi ? lo : up);
     lo = hi ? x : lo;
     up = hi ? up : x;
   }
