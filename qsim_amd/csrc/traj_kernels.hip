@@ -57,12 +57,14 @@ namespace {
 using namespace tileop;
 
 // Pairs per <Z_a Z_b> sweep (FP64 accumulators per thread: 32 would not fit
-// beside the tile kernel's registers) and amplitudes per thread per step of
-// a whole-state sweep (64 KiB of loads in flight per workgroup).
+// beside the step's registers) and amplitudes per thread per step of a
+// whole-state sweep.
 template <int NT>
 constexpr unsigned kPairChunk = 16;
 template <int NT>
-constexpr unsigned kSweep = 8192 / NT;
+constexpr unsigned kPairRed = (kPairChunk<NT> + 1) * (NT / 64);
+template <int NT>
+constexpr unsigned kSweep = NT <= 512 ? 16 : 8;
 
 // Groups [lo, hi) of a gate.
 template <int NT, int K>
@@ -316,16 +318,56 @@ __device__ __forceinline__ uint32_t PairSigns(uint64_t i,
   return m;
 }
 
+// w[p] for a wave-uniform p: a scalar branch instead of an indexed register.
+template <unsigned N>
+__device__ __forceinline__ double PickUniform(const double (&w)[N],
+                                              unsigned p) {
+  p = unsigned(__builtin_amdgcn_readfirstlane(int(p)));
+  double v = 0.0;
+  // The empty asm keeps the cases apart: folded into w[p] they would put w
+  // into scratch memory.
+  auto take = [&](auto u) {
+    v = w[decltype(u)::value];
+    asm volatile("" : "+v"(v));
+  };
+  if constexpr (N == 16) {
+    switch (p) {
+      case 8: take(std::integral_constant<int, 8>{}); break;
+      case 9: take(std::integral_constant<int, 9>{}); break;
+      case 10: take(std::integral_constant<int, 10>{}); break;
+      case 11: take(std::integral_constant<int, 11>{}); break;
+      case 12: take(std::integral_constant<int, 12>{}); break;
+      case 13: take(std::integral_constant<int, 13>{}); break;
+      case 14: take(std::integral_constant<int, 14>{}); break;
+      case 15: take(std::integral_constant<int, 15>{}); break;
+    }
+    if (p > 7) return v;
+  }
+  switch (p) {
+    case 0: take(std::integral_constant<int, 0>{}); break;
+    case 1: take(std::integral_constant<int, 1>{}); break;
+    case 2: take(std::integral_constant<int, 2>{}); break;
+    case 3: take(std::integral_constant<int, 3>{}); break;
+    case 4: take(std::integral_constant<int, 4>{}); break;
+    case 5: take(std::integral_constant<int, 5>{}); break;
+    case 6: take(std::integral_constant<int, 6>{}); break;
+    default: take(std::integral_constant<int, 7>{}); break;
+  }
+  return v;
+}
+
 // Sums over amplitudes [lo, hi) of |s_i|^2 (-1)^(bit a + bit b) for the
-// trajectory's pairs (FP64) and of |s_i|^2: put(j, sum) for pair j in every
-// thread (valid in thread 0), put(num_pairs, norm) last.  lo is a multiple
-// of kS NT.
+// trajectory's pairs (FP64) and of |s_i|^2: put(j, sum) for pair j,
+// put(num_pairs, norm) for the norm, each in one thread; ends with a barrier.
+// lo is a multiple of kS NT; red: LDS of kPairRed<NT> doubles.
 template <int NT, unsigned kS, typename Put>
 __device__ void PairSums(const float2* __restrict__ s,
                          const qsim_hip_traj_desc& d,
                          const uint32_t* __restrict__ pairs, uint64_t lo,
                          uint64_t hi, double* red, Put put) {
   constexpr unsigned kPC = kPairChunk<NT>;
+  constexpr unsigned kLog = kS == 16 ? 4 : 3;
+  static_assert(kS == 1u << kLog, "step");
   for (unsigned p0 = 0; p0 == 0 || p0 < d.num_pairs; p0 += kPC) {
     const unsigned np = std::min(kPC, d.num_pairs - p0);
     unsigned pa[kPC], pb[kPC];
@@ -337,36 +379,70 @@ __device__ void PairSums(const float2* __restrict__ s,
       acc[j] = 0.0;
     }
     // Element u of a step is i0 + u NT = i0 | u NT (i0's bits from
-    // log2 NT to log2 (kS NT) are zero): per-element sign masks are
-    // uniform, per-step ones one per thread.
-    uint32_t su[kS];
+    // log2 NT to log2 (kS NT) are zero), so a pair's sign is the thread's
+    // times the step's (scalar work) times the parity of u with the pair's pattern
+    // over u's bits, the same for every thread.
+    uint32_t su[kLog];
 #pragma unroll
-    for (unsigned u = 0; u < kS; ++u) su[u] = PairSigns(uint64_t(u) * NT, pa, pb);
+    for (unsigned b = 0; b < kLog; ++b) su[b] = PairSigns(uint64_t(NT) << b, pa, pb);
     double nrm = 0.0;
-    for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kS * NT) {
-      const uint32_t s0 = PairSigns(i0, pa, pb);
+    const uint32_t st = PairSigns(threadIdx.x, pa, pb);
+    for (uint64_t b0 = lo; b0 < hi; b0 += kS * NT) {
+      const uint64_t i0 = b0 + threadIdx.x;
+      const uint32_t s0 = st ^ PairSigns(b0, pa, pb);
       float2 a[kS];
 #pragma unroll
       for (unsigned u = 0; u < kS; ++u) {
         const uint64_t i = i0 + u * NT;
         a[u] = i < hi ? s[i] : float2{0.0f, 0.0f};
       }
+      // w[p] = sum over u of |a_u|^2 (-1)^parity(u & p): all patterns at once
+      // (a Walsh-Hadamard transform), then one addition per pair and step
+      // instead of one per pair and amplitude.
+      double w[kS];
 #pragma unroll
-      for (unsigned u = 0; u < kS; ++u) {
-        const double w = double(a[u].x) * a[u].x + double(a[u].y) * a[u].y;
-        const uint32_t m = s0 ^ su[u];
-        nrm += w;
+      for (unsigned u = 0; u < kS; ++u)
+        w[u] = double(a[u].x) * a[u].x + double(a[u].y) * a[u].y;
 #pragma unroll
-        for (unsigned j = 0; j < kPC; ++j) acc[j] += (m >> j) & 1u ? -w : w;
+      for (unsigned b = 0; b < kLog; ++b)
+#pragma unroll
+        for (unsigned u = 0; u < kS; ++u) {
+          if ((u >> b) & 1u) continue;
+          const double x = w[u], y = w[u | (1u << b)];
+          w[u] = x + y;
+          w[u | (1u << b)] = x - y;
+        }
+      nrm += w[0];
+#pragma unroll
+      for (unsigned j = 0; j < kPC; ++j) {
+        unsigned p = 0;
+#pragma unroll
+        for (unsigned b = 0; b < kLog; ++b) p |= ((su[b] >> j) & 1u) << b;
+        const double v = PickUniform(w, p);
+        acc[j] += (s0 >> j) & 1u ? -v : v;
       }
     }
-    // Unrolled, so that acc stays in registers.
+    // All sums with one exchange between the waves: one after the other they
+    // took most of a 2^14-amplitude chunk's time.
+    const unsigned wave = threadIdx.x >> 6;
 #pragma unroll
-    for (unsigned j = 0; j < kPC; ++j) {
-      const double v = BlockSum<NT>(acc[j], red);
-      if (j < np) put(p0 + j, v);
+    for (unsigned j = 0; j < kPC; ++j) acc[j] = WaveSum(acc[j]);
+    nrm = WaveSum(nrm);
+    if ((threadIdx.x & 63u) == 0) {
+#pragma unroll
+      for (unsigned j = 0; j < kPC; ++j) red[wave * (kPC + 1) + j] = acc[j];
+      red[wave * (kPC + 1) + kPC] = nrm;
     }
-    if (p0 + kPC >= d.num_pairs) put(d.num_pairs, BlockSum<NT>(nrm, red));
+    __syncthreads();
+    const unsigned j = threadIdx.x;
+    const bool last = p0 + kPC >= d.num_pairs;
+    if (j < np || (j == kPC && last)) {
+      double v = 0.0;
+#pragma unroll
+      for (unsigned w = 0; w < NT / 64; ++w) v += red[w * (kPC + 1) + j];
+      put(j == kPC ? d.num_pairs : p0 + j, v);
+    }
+    __syncthreads();
   }
 }
 
@@ -380,16 +456,18 @@ __device__ void TrajFinish(const float2* __restrict__ s,
                            const qsim_hip_traj_desc& d,
                            const uint32_t* __restrict__ pairs,
                            double* __restrict__ zz_out,
-                           double* __restrict__ norm_out, double* red) {
-  double nrm = 0.0;  // in thread 0
-  PairSums<NT, kSweep<NT>>(s, d, pairs, 0, uint64_t{1} << d.num_qubits, red,
-               [&](unsigned j, double v) {
-                 if (j == d.num_pairs) nrm = v;
-                 else if (threadIdx.x == 0) zz_out[d.pair_offset + j] = v;
-               });
-  if (threadIdx.x != 0) return;
-  for (unsigned j = 0; j < d.num_pairs; ++j) zz_out[d.pair_offset + j] /= nrm;
-  if (d.pad & 1u) norm_out[blockIdx.x] = nrm;
+                           double* __restrict__ norm_out) {
+  __shared__ double pair_red[kPairRed<NT>];
+  __shared__ double nrm;
+  PairSums<NT, kSweep<NT>>(s, d, pairs, 0, uint64_t{1} << d.num_qubits,
+                           pair_red, [&](unsigned j, double v) {
+                             if (j == d.num_pairs) nrm = v;
+                             else zz_out[d.pair_offset + j] = v;
+                           });
+  __threadfence_block();
+  for (unsigned j = threadIdx.x; j < d.num_pairs; j += NT)
+    zz_out[d.pair_offset + j] /= nrm;
+  if (threadIdx.x == 0 && (d.pad & 1u)) norm_out[blockIdx.x] = nrm;
 }
 
 // Workgroup t runs trajectory t, one sweep of the state per operation.  A
@@ -420,7 +498,7 @@ TrajectoryKernel(const qsim_hip_traj_desc* __restrict__ descs,
       oi += o.k;  // its Kraus operators
     }
   }
-  TrajFinish<NT>(s, d, pairs, zz_out, norm_out, red);
+  TrajFinish<NT>(s, d, pairs, zz_out, norm_out);
 }
 
 // A tile pass of a trajectory on the device: geometry, program, and the
@@ -443,7 +521,7 @@ struct TrajTilePass {
 // One workgroup per trajectory with barriers between its operations, which
 // this replaces, streamed each state at 12-15 GB/s and lasted as long as the
 // largest trajectories' serial chains: 100 trajectories each of 20, 18 and
-// 16 qubits, 4 passes of 5 gates: MEASURED
+// 16 qubits, 4 passes of 5 gates: 11.2 ms, against 4.7 ms here.
 struct TrajItem {
   uint32_t traj;
   uint32_t op;        // operation index
@@ -455,8 +533,9 @@ struct TrajItem {
 // Amplitudes of a sweep chunk.
 constexpr uint64_t kSweepChunk = uint64_t{1} << 14;
 constexpr int kSweepNT = 256;
-// Partial sums of a channel's chunk: one per Kraus operator, then the norm.
-constexpr unsigned kChanSums = kMaxKraus + 1;
+// Partial sums of a channel's chunk (ChannelSums), at most.
+constexpr unsigned kChanSums = 16;
+static_assert(kMaxChannelQubits == 2, "channel sums");
 
 // A pass over tiles of up to 13 qubits, with the FP16 arithmetic of the
 // circuit kernel's blocked passes (block_kernels.hip): the pass's op records
@@ -596,67 +675,91 @@ TrajGateKernel(const qsim_hip_traj_desc* __restrict__ descs,
   TrajGate<kSweepNT>(pool + d.state_offset, o, mats, lm, lo, hi);
 }
 
-// Partial sums of <psi|K^dagger K|psi> for every non-unitary operator of a
-// channel (all of them: the walk that may stop early comes after), and of
-// the norm where the trajectory is not unitary.
+// Partial sums P_rc = sum conj(v_r) v_c over the groups v of the channel's
+// qubits, r <= c (FP64 of FP32 amplitudes): its reduced density matrix, from
+// which every operator's probability and the norm follow without another
+// sweep.  Order: the diagonal, then (re, im) of the pairs r < c.
 template <int NQ>
 __device__ void ChannelSums(const float2* __restrict__ s, unsigned n,
-                            const qsim_hip_traj_op* __restrict__ ops,
-                            uint64_t oi, const float* __restrict__ mats,
-                            uint64_t chunk, double* __restrict__ out,
-                            float* lm) {
+                            const uint32_t* q, uint64_t chunk,
+                            double* __restrict__ out) {
   constexpr unsigned D = 1u << NQ;
-  const qsim_hip_traj_op h = ops[oi];
+  double acc[D * D];
+#pragma unroll
+  for (unsigned e = 0; e < D * D; ++e) acc[e] = 0.0;
   uint64_t lo, hi;
   SweepGroups(n, NQ, chunk, lo, hi);
-  for (unsigned i = 0; i < h.k; ++i) {
-    const qsim_hip_traj_op c = ops[oi + 1 + i];
-    if (c.pad & 1u) continue;  // unitary: decided by its bound alone
-    __syncthreads();           // earlier reads of lm are done
-    for (unsigned e = threadIdx.x; e < 2 * D * D; e += kSweepNT)
-      lm[e] = mats[c.moff2 + e];
-    __syncthreads();
-    double acc = 0.0;
-    for (uint64_t g = lo + threadIdx.x; g < hi; g += kSweepNT) {
-      float2 v[D];
-      LoadGroup<NQ>(s, g, h.q, v);
-      acc += double(GroupQuadratic<NQ>(v, lm));
+  constexpr int U = NQ == 1 ? 4 : 2;  // groups in flight
+  for (uint64_t g0 = lo + threadIdx.x; g0 < hi; g0 += U * kSweepNT) {
+    float2 v[U][D];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t g = g0 + u * kSweepNT;
+      if (g < hi) {
+        LoadGroup<NQ>(s, g, q, v[u]);
+      } else {
+#pragma unroll
+        for (unsigned r = 0; r < D; ++r) v[u][r] = float2{0.0f, 0.0f};
+      }
     }
-    acc = BlockSum<kSweepNT>(acc);
-    if (threadIdx.x == 0) out[i] = acc;
-  }
-  if (h.pad & 1u) {
-    uint64_t a0, a1;
-    SweepGroups(n, 0, chunk, a0, a1);
-    double acc = 0.0;
-    for (uint64_t i = a0 + threadIdx.x; i < a1; i += kSweepNT) {
-      const float2 v = s[i];
-      acc += double(v.x) * v.x + double(v.y) * v.y;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      unsigned e = D;
+#pragma unroll
+      for (unsigned r = 0; r < D; ++r) {
+        const double x = v[u][r].x, y = v[u][r].y;
+        acc[r] += x * x + y * y;
+#pragma unroll
+        for (unsigned c = r + 1; c < D; ++c) {
+          const double cx = v[u][c].x, cy = v[u][c].y;
+          acc[e++] += x * cx + y * cy;
+          acc[e++] += x * cy - y * cx;
+        }
+      }
     }
-    acc = BlockSum<kSweepNT>(acc);
-    if (threadIdx.x == 0) out[kMaxKraus] = acc;
   }
+#pragma unroll
+  for (unsigned e = 0; e < D * D; ++e) {
+    const double v = BlockSum<kSweepNT>(acc[e]);
+    if (threadIdx.x == 0) out[e] = v;
+  }
+}
+
+// <psi|M|psi> from the sums, M = K^dagger K at m (FP32 pairs, row-major).
+__device__ __forceinline__ double ChannelProb(const double* p, unsigned D,
+                                              const float* __restrict__ m) {
+  double prob = 0.0;
+  unsigned e = D;
+  for (unsigned r = 0; r < D; ++r) {
+    prob += double(m[2 * (r * D + r)]) * p[r];
+    for (unsigned c = r + 1; c < D; ++c, e += 2) {
+      // Re(M_rc P_rc + M_cr conj(P_rc))
+      prob += (double(m[2 * (r * D + c)]) + m[2 * (c * D + r)]) * p[e] -
+              (double(m[2 * (r * D + c) + 1]) - m[2 * (c * D + r) + 1]) *
+                  p[e + 1];
+    }
+  }
+  return prob;
 }
 
 __global__ void __launch_bounds__(kSweepNT)
 TrajChannelSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
                      const qsim_hip_traj_op* __restrict__ ops,
-                     const float* __restrict__ mats,
                      const TrajItem* __restrict__ items,
                      const float2* __restrict__ pool,
                      double* __restrict__ parts) {
-  __shared__ float lm[2 * 4 * 4];
   const TrajItem it = items[blockIdx.x];
   const qsim_hip_traj_desc d = descs[it.traj];
   const float2* s = pool + d.state_offset;
   double* out = parts + it.part + uint64_t(it.first) * kChanSums;
-  if (ops[it.op].moff2 == 1)
-    ChannelSums<1>(s, d.num_qubits, ops, it.op, mats, it.first, out, lm);
+  const qsim_hip_traj_op h = ops[it.op];
+  if (h.moff2 == 1)
+    ChannelSums<1>(s, d.num_qubits, h.q, it.first, out);
   else
-    ChannelSums<2>(s, d.num_qubits, ops, it.op, mats, it.first, out, lm);
+    ChannelSums<2>(s, d.num_qubits, h.q, it.first, out);
 }
 
-// The walk of RunIteration (lib/qtrajectory.h:330-370) over the summed
+// The walk of RunIteration (lib/qtrajectory.h:330-370) over the operators'
 // probabilities, the same in every workgroup of the trajectory, then the
 // chosen operator on this item's chunk.
 __global__ void __launch_bounds__(kSweepNT)
@@ -673,11 +776,8 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
   const qsim_hip_traj_desc d = descs[it.traj];
   const qsim_hip_traj_op h = ops[it.op];
   const bool normalise = h.pad & 1u;
-  for (unsigned i = 0; i < kChanSums; ++i) {
-    const bool need = i == kMaxKraus
-                          ? normalise
-                          : i < h.k && !(ops[it.op + 1 + i].pad & 1u);
-    if (!need) continue;
+  const unsigned DC = 1u << h.moff2;  // states of the channel's qubits
+  for (unsigned i = 0; i < DC * DC; ++i) {
     double acc = 0.0;
     for (unsigned c = threadIdx.x; c < it.count; c += kSweepNT)
       acc += parts[it.part + uint64_t(c) * kChanSums + i];
@@ -685,13 +785,17 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
     if (threadIdx.x == 0) sums[i] = acc;
   }
   __syncthreads();
-  const double norm = normalise ? sums[kMaxKraus] : 1.0;
+  double norm = 1.0;
+  if (normalise) {
+    norm = 0.0;
+    for (unsigned r = 0; r < DC; ++r) norm += sums[r];
+  }
   double cp = h.cp, max_prob = 0.0;
   int max_index = 0, pick = -1;
   for (unsigned i = 0; i < h.k; ++i) {
     const qsim_hip_traj_op c = ops[it.op + 1 + i];
     if (c.pad & 1u) continue;
-    const double prob = sums[i] / norm;
+    const double prob = ChannelProb(sums, DC, mats + c.moff2) / norm;
     if (prob > max_prob) {
       max_prob = prob;
       max_index = int(i);
@@ -733,16 +837,14 @@ TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
                     const TrajItem* __restrict__ items,
                     const float2* __restrict__ pool,
                     double* __restrict__ parts) {
-  __shared__ double red[kRedWords<kSweepNT>];
+  __shared__ double red[kPairRed<kSweepNT>];
   const TrajItem it = items[blockIdx.x];
   const qsim_hip_traj_desc d = descs[it.traj];
   uint64_t lo, hi;
   SweepGroups(d.num_qubits, 0, it.first, lo, hi);
   double* out = parts + it.part + uint64_t(it.first) * (d.num_pairs + 1);
-  PairSums<kSweepNT, 8>(pool + d.state_offset, d, pairs, lo, hi, red,
-                        [&](unsigned j, double v) {
-                          if (threadIdx.x == 0) out[j] = v;
-                        });
+  PairSums<kSweepNT, 16>(pool + d.state_offset, d, pairs, lo, hi, red,
+                         [&](unsigned j, double v) { out[j] = v; });
 }
 
 // <Z_a Z_b> and the norm of one trajectory from its chunks' sums.
@@ -1006,7 +1108,7 @@ int LaunchTiled(TrajBatch& b, hipStream_t st) {
         break;
       case TrajLaunch::kChannelSum:
         hipLaunchKernelGGL(TrajChannelSumKernel, grid, nt, 0, st, b.descs,
-                           b.ops, b.mats, it, b.pool, b.parts);
+                           b.ops, it, b.pool, b.parts);
         break;
       case TrajLaunch::kChannelApply:
         hipLaunchKernelGGL(TrajChannelApplyKernel, grid, nt, 0, st, b.descs,
