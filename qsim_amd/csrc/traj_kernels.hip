@@ -48,6 +48,7 @@
 
 #include "block_tile.h"
 #include "internal.h"
+#include "lane.h"
 #include "reduce.h"
 
 namespace qhip {
@@ -521,7 +522,7 @@ struct TrajTilePass {
 // One workgroup per trajectory with barriers between its operations, which
 // this replaces, streamed each state at 12-15 GB/s and lasted as long as the
 // largest trajectories' serial chains: 100 trajectories each of 20, 18 and
-// 16 qubits, 4 passes of 5 gates: 11.2 ms, against 4.7 ms here.
+// 16 qubits, 4 passes of 5 gates: 11.1 ms, against 4.3 ms here.
 struct TrajItem {
   uint32_t traj;
   uint32_t op;        // operation index
@@ -830,21 +831,141 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
   else ApplyGateK<kSweepNT, 2>(s, c, lm, lo, hi);
 }
 
-// Partial sums of a chunk: one per pair, then the norm.
-__global__ void __launch_bounds__(kSweepNT)
+// One step of a Walsh-Hadamard transform over the lanes of a wave: lane bit
+// B's pairs become sum (bit clear) and difference (bit set).
+template <int B>
+__device__ __forceinline__ double LaneButterfly(double v) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, v);
+  const unsigned l = unsigned(w), h = unsigned(w >> 32);
+  const unsigned neg = ((threadIdx.x >> B) & 1u) << 31;
+  auto join = [](unsigned lo, unsigned hi) {
+    return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+  };
+  if constexpr (B < 4) {
+    return join(PullLane<B>(l), PullLane<B>(h)) + join(l, h ^ neg);
+  } else {
+    // Swapped with itself: [0] holds the clear lanes' values in both, [1]
+    // the set lanes'.
+    unsigned l0, l1, h0, h1;
+    if constexpr (B == 4) {
+      const auto x = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+      const auto y = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+      l0 = x[0]; l1 = x[1]; h0 = y[0]; h1 = y[1];
+    } else {
+      const auto x = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+      l0 = x[0]; l1 = x[1]; h0 = y[0]; h1 = y[1];
+    }
+    return join(l0, h0) + join(l1, h1 ^ neg);
+  }
+}
+
+// The transform over all six lane bits: lane m gets sum (-1)^|l & m| v_l.
+__device__ __forceinline__ double LaneTransform(double v) {
+  v = LaneButterfly<0>(v);
+  v = LaneButterfly<1>(v);
+  v = LaneButterfly<2>(v);
+  v = LaneButterfly<3>(v);
+  v = LaneButterfly<4>(v);
+  return LaneButterfly<5>(v);
+}
+
+// Partial sums of a chunk: one per pair, then the norm.  A pair's sum over
+// the chunk is the Walsh-Hadamard coefficient of |s_i|^2 at (1 << a) ^
+// (1 << b) (the chunk's own bits give a sign), so the coefficients of at most
+// two set bits are made once, whatever the number of pairs, from one read of
+// the chunk.  Index bits of a chunk: 0-5 the lane, 6-7 the wave, 8-13 "own":
+// a thread's 64 amplitudes, 16 a step.  A thread sums 1 + 6 + 15 coefficients
+// over its own bits; the first 7 take a transform over the lanes, the last 15
+// (two bits already) are needed at lane 0 only; the four waves are combined
+// by the threads that write.  100 trajectories each of 20, 18 and 16 qubits, all
+// grid pairs: 375 us, 800 us with a sum per pair (branches for the sign pattern of
+// each pair and step, and the chunk read once per 16 pairs).
+constexpr unsigned kChunkOwn = 6;
+constexpr unsigned kChunkSums =
+    64 * (1 + kChunkOwn) + kChunkOwn * (kChunkOwn - 1) / 2;
+__global__ void __launch_bounds__(kSweepNT, 4)
 TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
                     const uint32_t* __restrict__ pairs,
                     const TrajItem* __restrict__ items,
                     const float2* __restrict__ pool,
                     double* __restrict__ parts) {
-  __shared__ double red[kPairRed<kSweepNT>];
+  static_assert(kSweepNT == 256 && kSweepChunk == kSweepNT << kChunkOwn,
+                "chunk's index bits");
+  __shared__ double red[kSweepNT / 64][kChunkSums];
   const TrajItem it = items[blockIdx.x];
   const qsim_hip_traj_desc d = descs[it.traj];
+  const float2* __restrict__ s = pool + d.state_offset;
   uint64_t lo, hi;
   SweepGroups(d.num_qubits, 0, it.first, lo, hi);
+  auto two = [](unsigned b, unsigned c) { return c * (c - 1) / 2 + b; };
+  double none = 0.0, one[kChunkOwn] = {}, both[15] = {};
+  // Unrolled, all steps' loads would be issued first and their values spilled.
+#pragma unroll 1
+  for (unsigned t = 0; t < 4; ++t) {
+    // The signs of the step's two bits.
+    const double s4 = t & 1u ? -1.0 : 1.0, s5 = t & 2u ? -1.0 : 1.0;
+    double w[16];
+#pragma unroll
+    for (unsigned u = 0; u < 16; ++u) {
+      const uint64_t i = lo + (t * 16 + u) * kSweepNT + threadIdx.x;
+      const float2 a = i < hi ? s[i] : float2{0.0f, 0.0f};
+      w[u] = double(a.x) * a.x + double(a.y) * a.y;
+    }
+#pragma unroll
+    for (unsigned b = 0; b < 4; ++b)
+#pragma unroll
+      for (unsigned u = 0; u < 16; ++u) {
+        if ((u >> b) & 1u) continue;
+        const double x = w[u], y = w[u | (1u << b)];
+        w[u] = x + y;
+        w[u | (1u << b)] = x - y;
+      }
+    none += w[0];
+    one[4] = fma(s4, w[0], one[4]);
+    one[5] = fma(s5, w[0], one[5]);
+    both[two(4, 5)] = fma(s4 * s5, w[0], both[two(4, 5)]);
+#pragma unroll
+    for (unsigned b = 0; b < 4; ++b) {
+      const double v = w[1u << b];
+      one[b] += v;
+      both[two(b, 4)] = fma(s4, v, both[two(b, 4)]);
+      both[two(b, 5)] = fma(s5, v, both[two(b, 5)]);
+#pragma unroll
+      for (unsigned c = b + 1; c < 4; ++c)
+        both[two(b, c)] += w[(1u << b) | (1u << c)];
+    }
+  }
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  red[wave][lane] = LaneTransform(none);
+#pragma unroll
+  for (unsigned b = 0; b < kChunkOwn; ++b)
+    red[wave][64 * (1 + b) + lane] = LaneTransform(one[b]);
+#pragma unroll
+  for (unsigned j = 0; j < 15; ++j) {
+    const double v = LaneTransform(both[j]);
+    if (lane == 0) red[wave][64 * (1 + kChunkOwn) + j] = v;
+  }
+  __syncthreads();
   double* out = parts + it.part + uint64_t(it.first) * (d.num_pairs + 1);
-  PairSums<kSweepNT, 16>(pool + d.state_offset, d, pairs, lo, hi, red,
-                         [&](unsigned j, double v) { out[j] = v; });
+  for (unsigned j = threadIdx.x; j <= d.num_pairs; j += kSweepNT) {
+    uint64_t m = 0;  // at most two bits; none for the norm
+    if (j < d.num_pairs)
+      m = (uint64_t{1} << pairs[2 * (d.pair_offset + j)]) ^
+          (uint64_t{1} << pairs[2 * (d.pair_offset + j) + 1]);
+    const unsigned own = unsigned(m >> 8) & 63u, waves = unsigned(m >> 6) & 3u;
+    unsigned at = unsigned(m) & 63u;
+    if (own != 0) {
+      const unsigned c = 31 - __builtin_clz(own), rest = own ^ (1u << c);
+      at = rest == 0 ? 64 * (1 + c) + at
+                     : 64 * (1 + kChunkOwn) + two(31 - __builtin_clz(rest), c);
+    }
+    double v = 0.0;
+#pragma unroll
+    for (unsigned w = 0; w < kSweepNT / 64; ++w)
+      v += __builtin_popcount(w & waves) & 1 ? -red[w][at] : red[w][at];
+    out[j] = __builtin_popcountll(lo & m) & 1 ? -v : v;
+  }
 }
 
 // <Z_a Z_b> and the norm of one trajectory from its chunks' sums.
