@@ -213,10 +213,8 @@ __device__ __forceinline__ void AddExpectation(Dbl2& acc, const C& v,
 }
 
 // The gate kernels' read side (GateLaneKernel): runs of 64 amplitudes, low
-// targets swapped into registers; bound by the read (27 qubits: 180 us, 6
-// TB/s).  Group by group through the caches (ExpectationKernel): 205 us for
-// k = 1, and 6 us for the final sum and 4 us for its copy in launches of
-// their own.
+// targets swapped into registers; bound by the read.  LaunchExpect says where
+// it beats ExpectationKernel.
 template <typename FP, int K, typename M>
 __global__ void __launch_bounds__(256)
 ExpectationLaneKernel(const typename Cplx<FP>::T* __restrict__ s, LaneGeom g,
@@ -227,37 +225,20 @@ ExpectationLaneKernel(const typename Cplx<FP>::T* __restrict__ s, LaneGeom g,
   const uint64_t stride = uint64_t(gridDim.x) * 4;
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   Dbl2 acc;
-  auto load = [&](uint64_t c, C(&v)[D]) {
+  for (uint64_t c = uint64_t(blockIdx.x) * 4 + wave; c < g.nchunks;
+       c += stride) {
     const C* p = s + InsertZeros(c << 6, g.ins, g.nins);
+    C v[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) v[j] = p[MemberOffset<K>(j, g.roff) + lane];
-  };
-  auto add = [&](C(&v)[D]) {
     SwapLowTargets<K, 0>(v, g);
     MatVec<FP, K>(v, m, [&](int r, C u) { AddExpectation(acc, v[r], u); });
-  };
-  uint64_t c = uint64_t(blockIdx.x) * 4 + wave;
-  if constexpr (K == 2) {
-    // Four chunks' loads in flight: 178 us a 27-qubit term against 190; k = 1
-    // is better without (180 against 201).
-    for (; c + 3 * stride < g.nchunks; c += 4 * stride) {
-      C v[4][D];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) load(c + k * stride, v[k]);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) add(v[k]);
-    }
-  }
-  for (; c < g.nchunks; c += stride) {
-    C v[D];
-    load(c, v);
-    add(v);
   }
   acc = BlockSum<256>(acc);
   if (threadIdx.x == 0) partials[blockIdx.x] = acc;
 }
 
-// Any sizes (k = 5, 6, and small states): one group per work item.
+// Any sizes, one group per work item; the members come through the caches.
 template <typename FP, int K, typename M>
 __global__ void __launch_bounds__(256)
 ExpectationKernel(const typename Cplx<FP>::T* __restrict__ s, GateGeom g, M m,
@@ -506,9 +487,10 @@ int DispatchK(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
   else return LaunchTile<FP, K>(s, g, mp);
 }
 
-// Workgroups of an expectation pass: four waves each, at most eight
-// workgroups a CU of 256.
-constexpr unsigned kExpectBlocks = 2048;
+// Workgroups of an expectation pass: at most eight a CU of 256, or four
+// (kExpectBlocksFew), which is better for ExpectationKernel and for
+// complex128 k = 1 (27 qubits: 353-392 us against 372-408).
+constexpr unsigned kExpectBlocks = 2048, kExpectBlocksFew = 1024;
 
 static_assert(kExpectBlocks * sizeof(Dbl2) <= kHostResultBytes, "partials");
 
@@ -516,11 +498,22 @@ static_assert(kExpectBlocks * sizeof(Dbl2) <= kHostResultBytes, "partials");
 template <typename FP, int K, typename M>
 unsigned LaunchExpect(const typename Cplx<FP>::T* s, unsigned n,
                   const unsigned* qs, const M& m, Dbl2* partials) {
-  if constexpr (K <= 4) {
+  if constexpr (K <= 4 && K != 2) {
+    // Where swapping low targets across lanes beats reading groups through the
+    // caches; calls on 27 qubits, lanes against groups (us):
+    //   complex64   k = 1 183-197 : 225-234; k = 2 201-215 : 186-190;
+    //               k = 3 215 : 237 without a target in the lanes, else
+    //               245-286 : 236-245
+    //   complex128  k = 1 353-392 : 359-397; k = 2 362-394 : 360-378; k = 3
+    //               440 : 540 with 3 targets in the lanes, 391 : 392 with 1;
+    //               k = 4 543 : 555 without, 593-673 : 555-629 with
+    constexpr bool f32 = sizeof(FP) == 4;
     LaneGeom lg;
-    if (LaneGeometry<FP>(n, qs, K, nullptr, 0, 0, lg)) {
-      const uint64_t blocks =
-          std::min<uint64_t>((lg.nchunks + 3) / 4, kExpectBlocks);
+    if (LaneGeometry<FP>(n, qs, K, nullptr, 0, 0, lg) &&
+        (K < 3 || (K == 3 && !f32 ? lg.nlow > 1 : lg.nlow == 0))) {
+      const uint64_t blocks = std::min<uint64_t>(
+          (lg.nchunks + 3) / 4,
+          K == 1 && !f32 ? kExpectBlocksFew : kExpectBlocks);
       hipLaunchKernelGGL((ExpectationLaneKernel<FP, K, M>),
                          dim3(unsigned(blocks)), dim3(256), 0, Stream(), s, lg,
                          m, partials);
@@ -535,7 +528,7 @@ unsigned LaunchExpect(const typename Cplx<FP>::T* s, unsigned n,
   }
   g.ngroups = uint64_t{1} << (n - K);
   const uint64_t blocks = std::max<uint64_t>(
-      1, std::min<uint64_t>((g.ngroups + 255) / 256, kExpectBlocks));
+      1, std::min<uint64_t>((g.ngroups + 255) / 256, kExpectBlocksFew));
   hipLaunchKernelGGL((ExpectationKernel<FP, K, M>), dim3(unsigned(blocks)),
                      dim3(256), 0, Stream(), s, g, m, partials);
   return unsigned(blocks);

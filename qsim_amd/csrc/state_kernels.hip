@@ -530,7 +530,11 @@ unsigned ReduceBlocks(uint64_t size) {
 template <typename FP>
 unsigned LaunchDot(const C_t<FP>* a, const C_t<FP>* b, uint64_t size,
                    bool real, Dbl2* part) {
-  const dim3 blocks(ReduceBlocks<FP>(size)), bs(kBS);
+  // A norm reads one state: half the workgroups (29 qubits: 709 us complex64,
+  // 1396 complex128, against 737 and 1430; two states 1400 and 2776 against
+  // 1383 and 2743).
+  const unsigned most = real && a == b ? kReduceBlocks / 2 : kReduceBlocks;
+  const dim3 blocks(std::min(ReduceBlocks<FP>(size), most)), bs(kBS);
   const hipStream_t st = Stream();
   if (real && a == b)
     hipLaunchKernelGGL((DotKernel<C_t<FP>, true, true>), blocks, bs, 0, st, a,
