@@ -715,12 +715,14 @@ struct TileIoPairs {
     for (int b = 0; b < 5; ++b) h[b] = g.hbit[9 - g.Lc + b];
     unit = F16Swz(a) >> 1;
   }
+  // A state is aligned to an amplitude only.
+  typedef float Pair __attribute__((ext_vector_type(4), aligned(8)));
   // Addresses of the four pairs 4 C .. 4 C + 3 of the tile at `base`.  The
   // thread's part is hidden from the optimiser so that the 32 addresses are
   // not kept in registers across the tile loop, where the pairs are.
   template <int C>
   __device__ __forceinline__ void At(float2* s, uint64_t base,
-                                     v4f* (&q)[4]) const {
+                                     Pair* (&q)[4]) const {
     uint64_t o = tofs;
     asm volatile("" : "+v"(o));
     uint64_t b = base;
@@ -728,10 +730,10 @@ struct TileIoPairs {
     if (C & 2) b += h[3];
     if (C & 4) b += h[4];
     float2* p = s + o;
-    q[0] = reinterpret_cast<v4f*>(p + b);
-    q[1] = reinterpret_cast<v4f*>(p + (b + h[0]));
-    q[2] = reinterpret_cast<v4f*>(p + (b + h[1]));
-    q[3] = reinterpret_cast<v4f*>(p + (b + h[0] + h[1]));
+    q[0] = reinterpret_cast<Pair*>(p + b);
+    q[1] = reinterpret_cast<Pair*>(p + (b + h[0]));
+    q[2] = reinterpret_cast<Pair*>(p + (b + h[1]));
+    q[3] = reinterpret_cast<Pair*>(p + (b + h[0] + h[1]));
   }
   __device__ __forceinline__ unsigned Unit(int i) const {
     unsigned u = unit;
@@ -815,14 +817,14 @@ __device__ __forceinline__ void BlockIoRun(
   v4f buf[PER];
   auto load = [&](auto c, uint64_t base) {
     constexpr int C = decltype(c)::value;
-    v4f* q[4];
+    TileIoPairs::Pair* q[4];
     io.At<C>(s, base, q);
 #pragma unroll
     for (int i = 0; i < 4; ++i) buf[4 * C + i] = *q[i];
   };
   auto store = [&](auto c, uint64_t base, int e) {
     constexpr int C = decltype(c)::value;
-    v4f* q[4];
+    TileIoPairs::Pair* q[4];
     io.At<C>(s, base, q);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
