@@ -4,11 +4,11 @@
 // (the operation of SimulatorCUDA::ApplyGate / ApplyControlledGate,
 // lib/simulator_cuda.h:70-207; arithmetic as lib/simulator_basic.h:167-275):
 //
-//  * GateLaneKernel -- k <= 4, any targets and controls, states of at least
+//  * GateLaneKernel -- k <= 4, low targets or controls, states of at least
 //    2^(6+k) amplitudes per control pattern.  A wave loads 2^k runs of 64
 //    consecutive amplitudes; targets among the lane qubits move to register
 //    bits by swaps across lanes.  No LDS, no barriers.
-//  * GateRegKernel  -- k = 5, 6 with all targets and controls at qubit >= 5:
+//  * GateRegKernel  -- all targets and controls at qubit >= 5 (not k = 4):
 //    one group per work item, held in registers.
 //  * GateTileKernel -- the rest (k = 5, 6 with a qubit below 5, and small
 //    states).  A workgroup stages a tile of 2^tb amplitudes (the Lc lowest
@@ -368,8 +368,15 @@ int DispatchK(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
   }
 
   if constexpr (K <= 4) {
+    // Nothing to bring into the lanes (no target or control below qubit 5):
+    // GateRegKernel, up to k = 3.  Against the lane kernel, complex64 k = 2
+    // 28 qubits, highest targets 803 us : 853, k = 3 20 qubits 8.2 : 8.9;
+    // complex128 k = 3 20 qubits 12.1 : 13.8, 29 qubits 3231 : 3340; equal
+    // for k = 1.  With controls, complex128 is 2-5 % better on the lanes (27
+    // qubits 191-210 : 187-198), and k = 4 too (20 qubits 26 : 16).
+    const bool reg = lowest >= 5 && K <= 3 && (nc == 0 || sizeof(FP) == 4);
     LaneGeom lg;
-    if (LaneGeometry<FP>(n, qs, K, cqs, nc, cvals, lg)) {
+    if (!reg && LaneGeometry<FP>(n, qs, K, cqs, nc, cvals, lg)) {
       if constexpr (byval) return LaunchLane<FP, K>(s, lg, mv);
       else return LaunchLane<FP, K>(s, lg, mp);
     }
