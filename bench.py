@@ -86,13 +86,14 @@ SWEEP_PATHS = [f"fp32-k{k}" for k in range(2, 7)]
 # HBM bytes per amplitude per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE
 # runs, scaled by what the counters read for a copy of known size (reads x 2,
 # writes x 1); profiles/gate_passes_32q_blocked_vs_fused.md.
-MEASURED_HBM_BYTES_PER_AMP = {"GateBlockF16Kernel": 16.03,  # 14-qubit tiles
+MEASURED_HBM_BYTES_PER_AMP = {"GateBlockF16IoKernel": 16.00,
                               "GateBlockKernel": 16.04}
 
 # MFMA flops issued per amplitude per 4-qubit op of a blocked pass: a batch
 # of 32 groups (512 amplitudes) takes 2 K blocks x (3 FP16 or 4 split-BF16
 # products) MFMAs of 32 x 32 x 16.
-BLOCK_FLOPS_PER_AMP_OP = {"GateBlockF16Kernel": 6 * 2 * 32 * 32 * 16 / 512.0,
+BLOCK_FLOPS_PER_AMP_OP = {"GateBlockF16IoKernel": 6 * 2 * 32 * 32 * 16 / 512.0,
+                          "GateBlockF16Kernel": 6 * 2 * 32 * 32 * 16 / 512.0,
                           "GateBlockKernel": 8 * 2 * 32 * 32 * 16 / 512.0}
 # Dense MFMA peak of MI355X, fp16 and bf16 alike.
 MFMA_F16_PEAK_TFLOPS = 2500.0
@@ -131,11 +132,13 @@ def available_paths():
 def kernel_family(circ, i, qubits, method, n, arith="f16"):
     """The gate kernel a pass runs (qsim_amd/csrc: gate_kernels.hip,
     mfma_kernels.hip, f16_kernels.hip and block_kernels.hip dispatch).
-    Blocked passes of unitary gates run GateBlockF16Kernel unless the
-    split-BF16 arithmetic is asked for."""
+    Blocked passes of unitary gates run the FP16 kernels (14 tile qubits:
+    GateBlockF16IoKernel) unless the split-BF16 arithmetic is asked for."""
     from qsim_amd import driver
     if circ.pass_kind(i) == driver.PASS_BLOCKED:
-        return "GateBlockF16Kernel" if arith == "f16" else "GateBlockKernel"
+        if arith != "f16":
+            return "GateBlockKernel"
+        return "GateBlockF16IoKernel" if len(qubits) == 14 else "GateBlockF16Kernel"
     k = len(qubits)
     low = bool(qubits) and min(qubits) < 5
     if method != 1 and 4 <= k <= 6 and n >= k + 5:
@@ -147,7 +150,11 @@ def kernel_family(circ, i, qubits, method, n, arith="f16"):
             return "GateF16SetKernel" if low else "GateF16RegKernel"
         if method == 0 and k >= 5 and n >= 11:
             return "GateF32RowSetKernel" if low else "GateF32RowRegKernel"
+        if k == 4:
+            return "GateMfmaLaneKernel"
         return "GateMfmaTileKernel" if low else "GateMfmaRegKernel"
+    if n >= k + 6 and (k == 4 or (k < 4 and low)):
+        return "GateLaneKernel"
     return "GateTileKernel" if low else "GateRegKernel"
 
 

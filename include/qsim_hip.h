@@ -36,8 +36,9 @@ enum { QSIM_HIP_F32 = 0, QSIM_HIP_F64 = 1 };
 
 /* Arithmetic used for an uncontrolled gate pass (qsim_hip_set_gate_method). */
 enum {
-  /* complex64, uncontrolled k >= 4: FP32 MFMA (exact FP32 products and
-   * sums); everything else: the FP32 / FP64 vector kernels */
+  /* uncontrolled complex64 k >= 4: FP32 MFMA (exact FP32 products and
+   * sums); uncontrolled complex128 k = 5, 6: FP64 MFMA; everything else: the
+   * FP32 / FP64 vector kernels */
   QSIM_HIP_METHOD_AUTO = 0,
   QSIM_HIP_METHOD_VECTOR = 1,       /* always the vector kernels */
   QSIM_HIP_METHOD_MFMA_BF16X3 = 2,  /* as AUTO, but k >= 5 on split-BF16
@@ -357,9 +358,10 @@ int qsim_hip_pass_timer_start(unsigned capacity);
 int qsim_hip_pass_timer_stop(float* ms, unsigned max_count, unsigned* count);
 
 /* ---- batched noisy trajectories -------------------------------------------
- * Many quantum trajectories (of possibly different qubit counts) run in ONE
- * kernel launch, one workgroup per trajectory, each with its own state in a
- * device pool and its own operation stream: fused gates (FP32 matrices, the
+ * Many quantum trajectories (of possibly different qubit counts) run at once,
+ * each with its own state in a device pool and its own operation stream (one
+ * launch with a workgroup per trajectory, or one launch per step with many
+ * workgroups per trajectory): fused gates (FP32 matrices, the
  * Kraus operators already sampled on the host folded in) and channel
  * decisions that need the state (taken on the device, in FP64).  At the end
  * every trajectory writes <Z_a Z_b> for its qubit pairs (FP64).  Replaces
@@ -384,8 +386,8 @@ enum {
   /* The header of a tile pass over the k gate operations that follow it
    * (1 <= k <= 32): q[0] | q[1] << 32 is the mask of its tile qubits (9..14
    * of them, starting with qubits 0, 1, 2), and every gate lies inside the
-   * tile.  The tiled kernel applies the k gates with one stream of the
-   * state (tiles staged in LDS, split-BF16 MFMA, as
+   * tile.  The tiled batch applies the k gates with one stream of the
+   * state (tiles staged in LDS, FP16 MFMA with a scale per tile, as
    * qsim_hip_apply_gate_block does); the per-gate kernels ignore the header
    * and apply the gates one by one.  moff is not read. */
   QSIM_HIP_TRAJ_TILE_PASS = 2,
@@ -395,8 +397,8 @@ enum {
    * bit 0 = unitary. */
   QSIM_HIP_TRAJ_KRAUS = 3
 };
-/* qsim_hip_traj_run's `threads` value for the tiled kernel: 256 threads
- * per trajectory, or 512 when a tile pass has 14 qubits. */
+/* qsim_hip_traj_run's `threads` value for the tiled batch: every step of the
+ * streams is one launch over many workgroups per trajectory. */
 enum { QSIM_HIP_TRAJ_TILED = 1 };
 
 typedef struct {
@@ -431,9 +433,9 @@ int qsim_hip_traj_prepare(const qsim_hip_traj_desc* trajs, unsigned num_traj,
                           const float* matrices, uint64_t num_floats,
                           const uint32_t* pairs, uint32_t num_pairs,
                           uint32_t num_decisions, void** handle);
-/* One launch of the whole batch with `threads` (256, 512 or 1024) per
- * trajectory, or with the tiled kernel (QSIM_HIP_TRAJ_TILED); with
- * use_graph the launch is captured once in a hipGraph and replayed after.
+/* Runs the whole batch: one launch with `threads` (256, 512 or 1024) per
+ * trajectory, or the tiled batch's launches (QSIM_HIP_TRAJ_TILED); with
+ * use_graph they are captured once in a hipGraph and replayed after.
  * Waits for completion. */
 int qsim_hip_traj_run(void* handle, unsigned threads, int use_graph);
 /* <Z_a Z_b> of every pair (FP64, pair order of the batch) and the decision

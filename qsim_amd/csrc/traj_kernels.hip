@@ -1,18 +1,20 @@
-// traj_kernels.hip -- batched noisy trajectories in one launch.
+// traj_kernels.hip -- batched noisy trajectories.
 //
 // qsim's trajectory simulator (lib/qtrajectory.h:112-387) runs trajectories
 // one after another, each gate batch as its own set of kernel launches with a
 // host synchronisation at every channel whose Kraus operator depends on the
 // state.  Here a whole batch -- hundreds of trajectories of uneven qubit
-// counts -- is ONE launch: workgroup t owns trajectory t, its state in a
-// device pool and its operation stream, and walks the stream with nothing
-// but workgroup barriers between operations:
+// counts, their states in a device pool -- runs at once.  The per-gate kernels
+// are ONE launch: workgroup t owns trajectory t and walks its operation stream
+// with nothing but workgroup barriers between operations.  The tiled batch is
+// one launch per step of the streams, over pieces of all trajectories.  The
+// operations:
 //
 //   gate      a fused gate (k <= 4, FP32 matrix in LDS) over all 2^(n-k)
 //             groups of the trajectory's state;
 //   tile pass a run of gates applied tile by tile through LDS with the
 //             FP16 MFMA product of the circuit kernel's blocked passes (the
-//             tiled kernel; the per-gate kernels run the gates one by one);
+//             tiled batch; the per-gate kernels run the gates one by one);
 //   channel   a channel whose draw fell past the probability bounds: FP64
 //             sweeps for <psi|K^dagger K|psi> operator by operator (the
 //             first also giving the norm), the choice exactly as
@@ -27,8 +29,8 @@
 // trajectory writes <Z_a Z_b> of its qubit pairs, FP64-accumulated and
 // divided by the norm (the normalisation of lib/qtrajectory.h:377-383).
 //
-// Workgroups are dispatched in trajectory order, so the host puts the
-// largest states first (longest-processing-time-first balancing across CUs).
+// Workgroups are dispatched in order, so the host puts the largest states and
+// items first (longest-processing-time-first balancing across CUs).
 
 #include <hip/hip_runtime.h>
 

@@ -1,5 +1,5 @@
 """Batched noisy trajectories on the GPU (include/qsim_hip_driver.h,
-qsim_traj_*): many trajectories of uneven qubit counts in one launch.
+qsim_traj_*): many trajectories of uneven qubit counts at once.
 
 A noisy circuit is either a qsim grid circuit with a depolarising channel
 after every gate (on each of its qubits) and an amplitude-damping channel
@@ -111,8 +111,8 @@ class TrajectoryBatch:
         return time.time() - t0
 
     def run(self, threads=512, use_graph=False):
-        """One launch of the planned batch: ``threads`` 256, 512 or 1024
-        (per-gate kernels) or ``TILED`` (tile passes, 256 threads)."""
+        """Runs the planned batch: ``threads`` 256, 512 or 1024 (per-gate
+        kernels, one launch) or ``TILED`` (tile passes, a launch per step)."""
         _check(driver_lib().qsim_traj_run(self.h, threads, int(use_graph)))
 
     def zz(self, t: int) -> np.ndarray:
