@@ -321,6 +321,10 @@ DotKernel(const C* __restrict__ a, const C* __restrict__ b, uint64_t size,
 // amplitudes ends it: the range is read little more than once, in parallel.
 // (One scan of the whole range, 256 amplitudes per step: 65 us for 2^16
 // amplitudes.)
+// A piece is entered because its sum puts r inside it, so one of its
+// amplitudes is not zero.  Its parts, added in another order, may fall short
+// of r by rounding: then its last part that is not zero is taken, down to its
+// last such amplitude, never an index of probability zero.
 template <typename C>
 __global__ void __launch_bounds__(1024)
 FindFirstKernel(const C* __restrict__ s, uint64_t i0, uint64_t i1, double r,
@@ -335,7 +339,7 @@ FindFirstKernel(const C* __restrict__ s, uint64_t i0, uint64_t i1, double r,
   };
   double before = 0;  // the sum ahead of lo
   uint64_t lo = i0, hi = i1;
-  bool none = false;
+  bool none = false, inside = false;  // inside: a piece was entered
   while (hi - lo > 64 && !none) {
     const uint64_t piece = (hi - lo + 15) / 16;
     const uint64_t a = std::min(hi, lo + w * piece);
@@ -354,15 +358,26 @@ FindFirstKernel(const C* __restrict__ s, uint64_t i0, uint64_t i1, double r,
     if (l == 0) tot[w] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
-      double c = before;
-      int k = 0;
-      while (k < 16 && !(r < c + tot[k])) c += tot[k++];
+      double c = before, c_last = before;
+      int k = 0, last = 16;
+      while (k < 16 && !(r < c + tot[k])) {
+        if (tot[k] > 0) {
+          last = k;
+          c_last = c;
+        }
+        c += tot[k++];
+      }
+      if (k == 16 && inside) {
+        k = last;
+        c = c_last;
+      }
       lo_s = k < 16 ? std::min(hi, lo + k * piece) : hi;
       hi_s = k < 16 ? std::min(hi, lo + (k + 1) * piece) : hi;
       before_s = c;
     }
     __syncthreads();
     none = lo_s == hi_s;
+    inside = true;
     lo = lo_s;
     hi = hi_s;
     before = before_s;
@@ -372,13 +387,14 @@ FindFirstKernel(const C* __restrict__ s, uint64_t i0, uint64_t i1, double r,
   uint64_t found = ~uint64_t{0};
   if (!none) {
     const uint64_t i = lo + l;
-    const double incl = WaveInclusiveScan(i < hi ? prob(i) : 0.0);
+    const double p = i < hi ? prob(i) : 0.0;
+    const double incl = WaveInclusiveScan(p);
     const unsigned long long ballot = __ballot(i < hi && r < before + incl);
+    const unsigned long long some = __ballot(p > 0);
     if (ballot != 0) {
       found = lo + __builtin_ctzll(ballot);
-    } else if (hi < i1) {
-      // The pieces' sums put r inside [lo, hi), their rounding past it.
-      found = hi;
+    } else if (inside && some != 0) {
+      found = lo + 63 - __builtin_clzll(some);
     }
   }
   if (l == 0) out[0] = found;

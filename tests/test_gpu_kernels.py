@@ -347,6 +347,32 @@ def test_measurement_vs_oracle(dtype):
         assert rel_l2(st.to_numpy(), s) < TOL[dtype] * 4
 
 
+@pytest.mark.parametrize("n,run", [(18, 64), (24, 64), (24, 1024)])
+def test_measured_index_has_probability(n, run):
+    # Draws at the sums ahead of runs of zeros, to the last bits of rounding:
+    # whichever way they round, the index found is the last amplitude of the
+    # run before or the first of the next one, never a zero.
+    rng = np.random.default_rng(n + run)
+    ss = qsim_amd.StateSpace(np.float64)
+    size = 1 << n
+    c = rng.normal(size=size) * ((np.arange(size) // run) % 2 == 0)
+    c /= np.sqrt(np.sum(c * c))
+    a = np.zeros(2 * size)
+    a[0::2] = c
+    st = upload(a, n, np.float64)
+    parts = len(ss.partial_norms(st))
+    part = size // parts
+    for m in range(0, parts, max(1, parts // 64)):
+        p = c[m * part:(m + 1) * part] ** 2
+        # The last runs of a part have no run after them.
+        for b in range(run, part - run, 2 * run):
+            total = p[:b].sum()
+            for ulps in range(-4, 5):
+                r = total + ulps * np.spacing(total)
+                k = ss.find_measured_bits(st, m, r, size - 1) - m * part
+                assert k in (b - 1, b + run), (m, b, ulps, k)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_state_fills_and_elementwise(dtype):
     ss = qsim_amd.StateSpace(dtype)
