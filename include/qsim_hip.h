@@ -34,7 +34,9 @@ enum {
 /* Element type of a state vector. */
 enum { QSIM_HIP_F32 = 0, QSIM_HIP_F64 = 1 };
 
-/* Arithmetic used for an uncontrolled gate pass (qsim_hip_set_gate_method). */
+/* Arithmetic used for an uncontrolled gate pass (qsim_hip_set_gate_method).
+ * Expectation values of complex64 states on 4 qubits use FP32 MFMA, except
+ * with METHOD_VECTOR. */
 enum {
   /* uncontrolled complex64 k >= 4: FP32 MFMA (exact FP32 products and
    * sums); uncontrolled complex128 k = 5, 6: FP64 MFMA; everything else: the

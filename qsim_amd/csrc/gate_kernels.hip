@@ -505,9 +505,10 @@ static_assert(kExpectBlocks * sizeof(Dbl2) <= kHostResultBytes, "partials");
 template <typename FP, int K, typename M>
 unsigned LaunchExpect(const typename Cplx<FP>::T* s, unsigned n,
                   const unsigned* qs, const M& m, Dbl2* partials) {
-  if constexpr (K <= 4 && K != 2) {
+  if constexpr (K != 2 && K <= (sizeof(FP) == 4 ? 3 : 4)) {
     // Where swapping low targets across lanes beats reading groups through the
-    // caches; calls on 27 qubits, lanes against groups (us):
+    // caches (complex64 k = 4 is LaunchExpectationMfma's, here only with the
+    // vector kernels asked for); calls on 27 qubits, lanes against groups (us):
     //   complex64   k = 1 183-197 : 225-234; k = 2 201-215 : 186-190;
     //               k = 3 215 : 237 without a target in the lanes, else
     //               245-286 : 236-245
@@ -550,8 +551,10 @@ int DispatchExpectation(const typename Cplx<FP>::T* s, unsigned n,
   unsigned count = 0;
   int rc = QSIM_HIP_ERR_UNSUPPORTED;
   if constexpr (K == 4 && sizeof(FP) == 4) {
-    rc = LaunchExpectationMfma(s, n, qs, m, partials, kExpectBlocks, &count);
-    if (rc != QSIM_HIP_OK && rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
+    if (qsim_hip_get_gate_method() != QSIM_HIP_METHOD_VECTOR) {
+      rc = LaunchExpectationMfma(s, n, qs, m, partials, kExpectBlocks, &count);
+      if (rc != QSIM_HIP_OK && rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
+    }
   }
   if (rc != QSIM_HIP_OK) {
     if constexpr (kByValue<FP, K>) {
@@ -591,7 +594,8 @@ int LaunchGate(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
   }
   QHIP_TRY(CheckQubits(n, qs, k, cqs, nc));
   if constexpr (sizeof(FP) == 8) {
-    if (k >= 5 && nc == 0) {
+    if (k >= 5 && nc == 0 &&
+        qsim_hip_get_gate_method() != QSIM_HIP_METHOD_VECTOR) {
       const int rc = LaunchGateF64(s, n, qs, k, m);
       if (rc != QSIM_HIP_ERR_UNSUPPORTED) return rc;
     }

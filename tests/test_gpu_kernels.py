@@ -504,6 +504,58 @@ def test_fp32_methods_vs_oracle(method, sim):
         qsim_amd.set_gate_method(qsim_amd.METHOD_AUTO)
 
 
+@pytest.mark.parametrize("k", [5, 6])
+def test_vector_method_complex128_wide_gates(k, sim):
+    # METHOD_VECTOR names the vector kernels in both precisions.  The FP64
+    # matrix-unit kernel returns the same bits, so its time tells which ran:
+    # at 20 qubits with low targets 16 (k = 5) and 26 us (k = 6) against 39 and
+    # 355 us.
+    n, qs = 20, list(range(k))
+    rng = np.random.default_rng(k)
+    m = to_interleaved(random_matrix(k, rng), np.float64)
+    s = random_state(n, rng, np.float64)
+    ms, got = {}, {}
+    for method in (qsim_amd.METHOD_VECTOR, qsim_amd.METHOD_AUTO):
+        st = upload(s, n, np.float64)
+        qsim_amd.set_gate_method(method)
+        try:
+            sim.apply_gate(qs, m, st)
+            got[method] = st.to_numpy()
+            qsim_amd.PassTimer.start(32)
+            for _ in range(20):
+                sim.apply_gate(qs, m, st)
+            ms[method] = np.median(qsim_amd.PassTimer.stop(32))
+        finally:
+            qsim_amd.set_gate_method(qsim_amd.METHOD_AUTO)
+    oracle.apply_gate(n, s, qs, m)
+    for method, a in got.items():
+        assert rel_l2(a, s) < 1e-14, method
+    assert ms[qsim_amd.METHOD_VECTOR] > 1.5 * ms[qsim_amd.METHOD_AUTO], ms
+
+
+def test_vector_method_expectation_values(sim):
+    # The 4-qubit complex64 kernels add their FP64 sums in different orders:
+    # over amplitudes of many magnitudes (sums that round) the last bits tell
+    # which ran.
+    n, rng = 16, np.random.default_rng(40)
+    s = random_state(n, rng, np.float32) * np.exp2(rng.uniform(-60, 0, 2 << n))
+    s = (s / np.linalg.norm(s)).astype(np.float32)
+    st = upload(s, n, np.float32)
+    differ = 0
+    for qs in _target_sets(n, 4, rng):
+        m = to_interleaved(random_matrix(4, rng, unitary=False), np.float32)
+        ref = oracle.expectation_value(n, s, qs, m)
+        auto = sim.expectation_value(qs, m, st)
+        qsim_amd.set_gate_method(qsim_amd.METHOD_VECTOR)
+        try:
+            vector = sim.expectation_value(qs, m, st)
+        finally:
+            qsim_amd.set_gate_method(qsim_amd.METHOD_AUTO)
+        assert abs(auto - ref) < 2e-6 and abs(vector - ref) < 2e-6, qs
+        differ += auto != vector
+    assert differ > 0
+
+
 def test_bf16x3_mfma_accuracy(sim):
     # Split-BF16 x3 products carry ~2^-16 relative error per product: per pass
     # the state stays within 5e-5 relative L2 of the FP64 result.
