@@ -253,15 +253,22 @@ def _u32(a: Sequence[int]):
     return arr, arr.ctypes.data_as(_u32p)
 
 
+_SEQUENCES = (list, tuple, range)
+
+
 def _qubits(qs):
     """Qubit indices as uint32: their owner, address and count.  Plain
-    sequences of ints skip numpy (1.6 us of a 12-qubit gate's 6.3)."""
-    try:
-        a = array("I", qs)
-        return a, a.buffer_info()[0], len(a)
-    except TypeError:  # numpy takes it, or says why not
-        a = _u32(qs)[0]
-        return a, a.ctypes.data, len(a)
+    sequences of ints skip numpy (1.6 us of a 12-qubit gate's 6.3); the rest,
+    such as bytes, whose contents array() would take for words, goes through
+    it, and so does what array() refuses."""
+    if type(qs) in _SEQUENCES:
+        try:
+            a = array("I", qs)
+            return a, a.buffer_info()[0], len(a)
+        except (TypeError, OverflowError, DeprecationWarning):
+            pass
+    a = _u32(qs)[0]
+    return a, a.ctypes.data, len(a)
 
 
 _PREC = {np.dtype(t): p for t, p in ((np.float32, F32), (np.complex64, F32),
