@@ -525,13 +525,40 @@ struct TrajTilePass {
 // this replaces, streamed each state at 12-15 GB/s and lasted as long as the
 // largest trajectories' serial chains: 100 trajectories each of 20, 18 and
 // 16 qubits, 4 passes of 5 gates: 11.1 ms, against 4.3 ms here.
+// An item of a tile pass: a run of tiles, one workgroup.
 struct TrajItem {
+  uint64_t op;        // operation index
   uint32_t traj;
-  uint32_t op;        // operation index
-  uint32_t first;     // first tile (passes) or sweep chunk
-  uint32_t count;     // tiles (passes); channels: chunks of the trajectory
-  uint64_t part;      // partial sums of chunk 0 (channel sums, finish)
+  uint32_t first;     // first tile
+  uint32_t count;     // tiles
 };
+// A trajectory's share of a sweep launch: one workgroup per chunk.  (An item
+// per chunk would hold 24 bytes per 2^14 amplitudes and gate, on the host and
+// the device: 200 MB for 8000 gates on 24 qubits.)
+struct TrajSweep {
+  uint64_t op;        // operation index
+  uint64_t part;      // partial sums of chunk 0 (channel sums, finish)
+  uint32_t traj;
+  uint32_t first;     // workgroup of chunk 0
+  uint32_t count;     // chunks
+};
+
+// The entry of this workgroup, the last of e[0..n) whose first workgroup is
+// not past it: each wave compares 64 entries at a time (two loads up to 4096
+// trajectories).
+__device__ __forceinline__ TrajSweep SweepOf(const TrajSweep* __restrict__ e,
+                                             unsigned n) {
+  const unsigned l = threadIdx.x & 63;
+  unsigned lo = 0;
+  while (n > 1) {
+    const unsigned step = (n + 63) / 64, at = l * step;
+    const bool le = at < n && e[lo + at].first <= blockIdx.x;
+    const unsigned last = __builtin_popcountll(__ballot(le)) - 1;
+    lo += last * step;
+    n = step < n - last * step ? step : n - last * step;
+  }
+  return e[__builtin_amdgcn_readfirstlane(lo)];
+}
 
 // Amplitudes of a sweep chunk.
 constexpr uint64_t kSweepChunk = uint64_t{1} << 14;
@@ -668,13 +695,14 @@ __global__ void __launch_bounds__(kSweepNT)
 TrajGateKernel(const qsim_hip_traj_desc* __restrict__ descs,
                const qsim_hip_traj_op* __restrict__ ops,
                const float* __restrict__ mats,
-               const TrajItem* __restrict__ items, float2* __restrict__ pool) {
+               const TrajSweep* __restrict__ sweeps, unsigned num, float2* __restrict__ pool) {
   __shared__ float lm[2 * 16 * 16];
-  const TrajItem it = items[blockIdx.x];
+  const TrajSweep it = SweepOf(sweeps, num);
+  const unsigned chunk = blockIdx.x - it.first;
   const qsim_hip_traj_op o = ops[it.op];
   const qsim_hip_traj_desc d = descs[it.traj];
   uint64_t lo, hi;
-  SweepGroups(d.num_qubits, o.k, it.first, lo, hi);
+  SweepGroups(d.num_qubits, o.k, chunk, lo, hi);
   TrajGate<kSweepNT>(pool + d.state_offset, o, mats, lm, lo, hi);
 }
 
@@ -748,18 +776,19 @@ __device__ __forceinline__ double ChannelProb(const double* p, unsigned D,
 __global__ void __launch_bounds__(kSweepNT)
 TrajChannelSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
                      const qsim_hip_traj_op* __restrict__ ops,
-                     const TrajItem* __restrict__ items,
+                     const TrajSweep* __restrict__ sweeps, unsigned num,
                      const float2* __restrict__ pool,
                      double* __restrict__ parts) {
-  const TrajItem it = items[blockIdx.x];
+  const TrajSweep it = SweepOf(sweeps, num);
+  const unsigned chunk = blockIdx.x - it.first;
   const qsim_hip_traj_desc d = descs[it.traj];
   const float2* s = pool + d.state_offset;
-  double* out = parts + it.part + uint64_t(it.first) * kChanSums;
+  double* out = parts + it.part + uint64_t(chunk) * kChanSums;
   const qsim_hip_traj_op h = ops[it.op];
   if (h.moff2 == 1)
-    ChannelSums<1>(s, d.num_qubits, h.q, it.first, out);
+    ChannelSums<1>(s, d.num_qubits, h.q, chunk, out);
   else
-    ChannelSums<2>(s, d.num_qubits, h.q, it.first, out);
+    ChannelSums<2>(s, d.num_qubits, h.q, chunk, out);
 }
 
 // The walk of RunIteration (lib/qtrajectory.h:330-370) over the operators'
@@ -769,13 +798,14 @@ __global__ void __launch_bounds__(kSweepNT)
 TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
                        const qsim_hip_traj_op* __restrict__ ops,
                        const float* __restrict__ mats,
-                       const TrajItem* __restrict__ items,
+                       const TrajSweep* __restrict__ sweeps, unsigned num,
                        float2* __restrict__ pool,
                        const double* __restrict__ parts,
                        int32_t* __restrict__ dec_out) {
   __shared__ float lm[2 * 4 * 4];
   __shared__ double sums[kChanSums];
-  const TrajItem it = items[blockIdx.x];
+  const TrajSweep it = SweepOf(sweeps, num);
+  const unsigned chunk = blockIdx.x - it.first;
   const qsim_hip_traj_desc d = descs[it.traj];
   const qsim_hip_traj_op h = ops[it.op];
   const bool normalise = h.pad & 1u;
@@ -809,7 +839,7 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
       break;
     }
   }
-  if (it.first == 0 && threadIdx.x == 0) dec_out[h.slot] = pick;
+  if (chunk == 0 && threadIdx.x == 0) dec_out[h.slot] = pick;
   const float a = normalise ? float(1.0 / std::sqrt(norm)) : 1.0f;
   float2* s = pool + d.state_offset;
   const qsim_hip_traj_op c = ops[it.op + 1 + (pick >= 0 ? pick : 0)];
@@ -817,7 +847,7 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
   if (pick < 0 || c.k == 0) {
     // Nothing applied (or the identity): the state is only normalised.
     if (!normalise) return;
-    SweepGroups(d.num_qubits, 0, it.first, lo, hi);
+    SweepGroups(d.num_qubits, 0, chunk, lo, hi);
     for (uint64_t i = lo + threadIdx.x; i < hi; i += kSweepNT) {
       const float2 v = s[i];
       s[i] = float2{v.x * a, v.y * a};
@@ -828,7 +858,7 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
   for (unsigned e = threadIdx.x; e < 2 * DK * DK; e += kSweepNT)
     lm[e] = mats[c.moff + e] * a;
   __syncthreads();
-  SweepGroups(d.num_qubits, c.k, it.first, lo, hi);
+  SweepGroups(d.num_qubits, c.k, chunk, lo, hi);
   if (c.k == 1) ApplyGateK<kSweepNT, 1>(s, c, lm, lo, hi);
   else ApplyGateK<kSweepNT, 2>(s, c, lm, lo, hi);
 }
@@ -889,17 +919,18 @@ constexpr unsigned kChunkSums =
 __global__ void __launch_bounds__(kSweepNT, 4)
 TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
                     const uint32_t* __restrict__ pairs,
-                    const TrajItem* __restrict__ items,
+                    const TrajSweep* __restrict__ sweeps, unsigned num,
                     const float2* __restrict__ pool,
                     double* __restrict__ parts) {
   static_assert(kSweepNT == 256 && kSweepChunk == kSweepNT << kChunkOwn,
                 "chunk's index bits");
   __shared__ double red[kSweepNT / 64][kChunkSums];
-  const TrajItem it = items[blockIdx.x];
+  const TrajSweep it = SweepOf(sweeps, num);
+  const unsigned chunk = blockIdx.x - it.first;
   const qsim_hip_traj_desc d = descs[it.traj];
   const float2* __restrict__ s = pool + d.state_offset;
   uint64_t lo, hi;
-  SweepGroups(d.num_qubits, 0, it.first, lo, hi);
+  SweepGroups(d.num_qubits, 0, chunk, lo, hi);
   auto two = [](unsigned b, unsigned c) { return c * (c - 1) / 2 + b; };
   double none = 0.0, one[kChunkOwn] = {}, both[15] = {};
   // Unrolled, all steps' loads would be issued first and their values spilled.
@@ -949,7 +980,7 @@ TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
     if (lane == 0) red[wave][64 * (1 + kChunkOwn) + j] = v;
   }
   __syncthreads();
-  double* out = parts + it.part + uint64_t(it.first) * (d.num_pairs + 1);
+  double* out = parts + it.part + uint64_t(chunk) * (d.num_pairs + 1);
   for (unsigned j = threadIdx.x; j <= d.num_pairs; j += kSweepNT) {
     uint64_t m = 0;  // at most two bits; none for the norm
     if (j < d.num_pairs)
@@ -973,11 +1004,11 @@ TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
 // <Z_a Z_b> and the norm of one trajectory from its chunks' sums.
 __global__ void __launch_bounds__(kSweepNT)
 TrajFinishKernel(const qsim_hip_traj_desc* __restrict__ descs,
-                 const TrajItem* __restrict__ items,
+                 const TrajSweep* __restrict__ sweeps,
                  const double* __restrict__ parts,
                  double* __restrict__ zz_out, double* __restrict__ norm_out) {
   __shared__ double norm_s;
-  const TrajItem it = items[blockIdx.x];
+  const TrajSweep it = sweeps[blockIdx.x];
   const qsim_hip_traj_desc d = descs[it.traj];
   const unsigned np = d.num_pairs;
   const double* in = parts + it.part;
@@ -1000,9 +1031,18 @@ TrajFinishKernel(const qsim_hip_traj_desc* __restrict__ descs,
 struct TrajLaunch {
   enum Kind { kPass14, kPass13, kPass12, kGate, kChannelSum, kChannelApply,
               kFinishSum, kFinish } kind;
-  uint64_t first;   // items
+  uint64_t first;   // items (passes), sweep entries (the rest)
   uint32_t count;
+  uint32_t blocks;  // workgroups
   unsigned nops;    // passes: the longest program
+};
+
+// The launches of a tiled batch, and what they read.
+struct TrajPlan {
+  std::vector<TrajLaunch> launches;
+  std::vector<TrajItem> items;
+  std::vector<TrajSweep> sweeps;
+  uint64_t num_parts = 1;  // partial sums
 };
 
 struct TrajBatch {
@@ -1020,11 +1060,14 @@ struct TrajBatch {
   int32_t* dec = nullptr;
   TrajTilePass* passes = nullptr;
   uint32_t* recs = nullptr;
-  // The tiled batch's launches and their items.
+  // The tiled batch's launches, their items and sweep entries (BuildTiled).
+  bool tiled = false;
   std::vector<TrajLaunch> launches;
   TrajItem* items = nullptr;
+  TrajSweep* sweeps = nullptr;
   double* parts = nullptr;
   uint64_t pool_size = 0;  // amplitudes
+  uint64_t num_ops = 0;
   std::vector<uint64_t> state_offset;
   std::vector<unsigned> nq;
   hipStream_t gstream = nullptr;
@@ -1082,29 +1125,34 @@ int TileKernelReady() {
 // about a quarter of a CU's share of the launch, largest first, so that the
 // last items to run are short; an item's first load and last store are
 // exposed, so it has at least four tiles where the state has.
-void TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
-                  const std::vector<qsim_hip_traj_op>& ops,
-                  const std::vector<TrajTilePass>& passes, unsigned cus,
-                  std::vector<TrajItem>& items,
-                  std::vector<TrajLaunch>& launches, uint64_t& num_parts) {
+TrajPlan TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
+                      const std::vector<qsim_hip_traj_op>& ops,
+                      const std::vector<TrajTilePass>& passes, unsigned cus) {
+  TrajPlan plan;
   const uint32_t T = uint32_t(d.size());
   std::vector<uint64_t> at(T);
   for (uint32_t t = 0; t < T; ++t) at[t] = d[t].op_begin;
-  num_parts = 1;
   auto chunks = [&](uint32_t t) {
     const uint64_t N = uint64_t{1} << d[t].num_qubits;
     return uint32_t(std::max<uint64_t>(1, N / kSweepChunk));
   };
-  std::vector<TrajItem> list;
-  auto flush = [&](TrajLaunch::Kind kind, unsigned nops) {
+  // A launch over the trajectories of `list`; blocks: one workgroup an entry
+  // or (0) one a chunk.
+  auto sweep = [&](TrajLaunch::Kind kind, std::vector<TrajSweep> list,
+                   uint32_t blocks) {
     if (list.empty()) return;
-    launches.push_back({kind, items.size(), uint32_t(list.size()), nops});
-    items.insert(items.end(), list.begin(), list.end());
-    list.clear();
+    uint32_t total = 0;
+    for (TrajSweep& e : list) {
+      e.first = total;
+      total += e.count;
+    }
+    plan.launches.push_back({kind, plan.sweeps.size(), uint32_t(list.size()),
+                             blocks ? blocks : total, 0});
+    plan.sweeps.insert(plan.sweeps.end(), list.begin(), list.end());
   };
   for (;;) {
-    bool pass = false, sweep = false;
-    std::vector<TrajItem> gates, sums, applies;
+    bool pass = false;
+    std::vector<TrajSweep> gates, channels;
     uint64_t part = 0;
     for (uint32_t t = 0; t < T; ++t) {
       if (at[t] >= d[t].op_end) continue;
@@ -1113,29 +1161,21 @@ void TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
         pass = true;
         continue;
       }
-      sweep = true;
       const uint32_t nc = chunks(t);
       if (o.kind == QSIM_HIP_TRAJ_GATE) {
-        for (uint32_t c = 0; c < nc; ++c)
-          gates.push_back({t, uint32_t(at[t]), c, nc, 0});
+        gates.push_back({at[t], 0, t, 0, nc});
         at[t] += 1;
       } else {
-        for (uint32_t c = 0; c < nc; ++c) {
-          sums.push_back({t, uint32_t(at[t]), c, nc, part});
-        }
+        channels.push_back({at[t], part, t, 0, nc});
         part += uint64_t(nc) * kChanSums;
         at[t] += 1 + o.k;
       }
     }
-    num_parts = std::max(num_parts, part);
-    if (sweep) {
-      applies = sums;
-      list.swap(gates);
-      flush(TrajLaunch::kGate, 0);
-      list.swap(sums);
-      flush(TrajLaunch::kChannelSum, 0);
-      list.swap(applies);
-      flush(TrajLaunch::kChannelApply, 0);
+    plan.num_parts = std::max(plan.num_parts, part);
+    if (!gates.empty() || !channels.empty()) {
+      sweep(TrajLaunch::kGate, gates, 0);
+      sweep(TrajLaunch::kChannelSum, channels, 0);
+      sweep(TrajLaunch::kChannelApply, channels, 0);
       continue;
     }
     if (!pass) break;
@@ -1166,34 +1206,36 @@ void TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
       const uint64_t slots = uint64_t(cus) * (kind == TrajLaunch::kPass14 ? 1 : 2);
       const uint64_t per = std::max<uint64_t>(4, (tiles + 4 * slots - 1) /
                                                      (4 * slots));
+      std::vector<TrajItem> list;
       for (const uint32_t t : who) {
         const uint64_t nt = passes[ops[at[t]].moff].g.ntiles;
         const uint64_t parts = (nt + per - 1) / per;
         for (uint64_t i = 0; i < parts; ++i) {
           const uint64_t a = nt * i / parts, b = nt * (i + 1) / parts;
-          list.push_back({t, uint32_t(at[t]), uint32_t(a), uint32_t(b - a), 0});
+          list.push_back({at[t], t, uint32_t(a), uint32_t(b - a)});
         }
       }
       std::stable_sort(list.begin(), list.end(),
                        [](const TrajItem& x, const TrajItem& y) {
                          return x.count > y.count;
                        });
-      flush(kind, nops);
+      plan.launches.push_back({kind, plan.items.size(), uint32_t(list.size()),
+                               uint32_t(list.size()), nops});
+      plan.items.insert(plan.items.end(), list.begin(), list.end());
       for (const uint32_t t : who) at[t] += 1 + ops[at[t]].k;
     }
   }
   uint64_t part = 0;
-  std::vector<TrajItem> ends;
+  std::vector<TrajSweep> ends;
   for (uint32_t t = 0; t < T; ++t) {
     const uint32_t nc = chunks(t);
-    for (uint32_t c = 0; c < nc; ++c) list.push_back({t, 0, c, nc, part});
-    ends.push_back({t, 0, 0, nc, part});
+    ends.push_back({0, part, t, 0, nc});
     part += uint64_t(nc) * (d[t].num_pairs + 1);
   }
-  num_parts = std::max(num_parts, part);
-  flush(TrajLaunch::kFinishSum, 0);
-  list.swap(ends);
-  flush(TrajLaunch::kFinish, 0);
+  plan.num_parts = std::max(plan.num_parts, part);
+  sweep(TrajLaunch::kFinishSum, ends, 0);
+  sweep(TrajLaunch::kFinish, ends, T);
+  return plan;
 }
 
 int LaunchTiled(TrajBatch& b, hipStream_t st) {
@@ -1206,7 +1248,8 @@ int LaunchTiled(TrajBatch& b, hipStream_t st) {
                      dim3(kSweepNT), 0, st, b.descs, b.num_traj, b.pool);
   for (const TrajLaunch& l : b.launches) {
     const TrajItem* it = b.items + l.first;
-    const dim3 grid(l.count), nt(kSweepNT);
+    const TrajSweep* sw = b.sweeps + l.first;
+    const dim3 grid(l.blocks), nt(kSweepNT);
     switch (l.kind) {
       case TrajLaunch::kPass14:
         hipLaunchKernelGGL(TrajPass14Kernel, grid, dim3(kIoThreads),
@@ -1227,22 +1270,23 @@ int LaunchTiled(TrajBatch& b, hipStream_t st) {
         break;
       case TrajLaunch::kGate:
         hipLaunchKernelGGL(TrajGateKernel, grid, nt, 0, st, b.descs, b.ops,
-                           b.mats, it, b.pool);
+                           b.mats, sw, l.count, b.pool);
         break;
       case TrajLaunch::kChannelSum:
         hipLaunchKernelGGL(TrajChannelSumKernel, grid, nt, 0, st, b.descs,
-                           b.ops, it, b.pool, b.parts);
+                           b.ops, sw, l.count, b.pool, b.parts);
         break;
       case TrajLaunch::kChannelApply:
         hipLaunchKernelGGL(TrajChannelApplyKernel, grid, nt, 0, st, b.descs,
-                           b.ops, b.mats, it, b.pool, b.parts, b.dec);
+                           b.ops, b.mats, sw, l.count, b.pool, b.parts,
+                           b.dec);
         break;
       case TrajLaunch::kFinishSum:
         hipLaunchKernelGGL(TrajFinishSumKernel, grid, nt, 0, st, b.descs,
-                           b.pairs, it, b.pool, b.parts);
+                           b.pairs, sw, l.count, b.pool, b.parts);
         break;
       case TrajLaunch::kFinish:
-        hipLaunchKernelGGL(TrajFinishKernel, grid, nt, 0, st, b.descs, it,
+        hipLaunchKernelGGL(TrajFinishKernel, grid, nt, 0, st, b.descs, sw,
                            b.parts, b.zz, b.norms);
         break;
     }
@@ -1257,7 +1301,6 @@ int Launch(TrajBatch& b, unsigned threads, hipStream_t st) {
     case 512: LaunchTraj<512>(b, st); break;
     case 1024: LaunchTraj<1024>(b, st); break;
     case QSIM_HIP_TRAJ_TILED:
-      QHIP_TRY(TileKernelReady());
       return LaunchTiled(b, st);
     default:
       SetError("trajectory batches run with 256, 512 or 1024 threads or "
@@ -1411,6 +1454,41 @@ int Upload(T** dst, const T* src, size_t count) {
   return QSIM_HIP_OK;
 }
 
+// What a tiled run reads beside the streams.  Batches with tile passes have it
+// from the start; the rest, planned for the per-gate kernels, not before they
+// are first run tiled (from their streams on the device).
+int BuildTiled(TrajBatch& b, const std::vector<qsim_hip_traj_desc>& d,
+               const std::vector<qsim_hip_traj_op>& ops,
+               const std::vector<TrajTilePass>& passes) {
+  QHIP_TRY(TileKernelReady());
+  TrajPlan plan = TrajSchedule(d, ops, passes, unsigned(NumCUs()));
+  // A first try may have ended for want of memory.
+  (void)hipFree(b.items);
+  (void)hipFree(b.sweeps);
+  (void)hipFree(b.parts);
+  b.items = nullptr;
+  b.sweeps = nullptr;
+  b.parts = nullptr;
+  QHIP_TRY(Upload(&b.items, plan.items.data(), plan.items.size()));
+  QHIP_TRY(Upload(&b.sweeps, plan.sweeps.data(), plan.sweeps.size()));
+  QHIP_CHECK(hipMalloc(&b.parts, plan.num_parts * sizeof(double)));
+  b.launches = std::move(plan.launches);
+  b.tiled = true;
+  return QSIM_HIP_OK;
+}
+
+int BuildTiledFromDevice(TrajBatch& b) {
+  std::vector<qsim_hip_traj_desc> d(b.num_traj);
+  std::vector<qsim_hip_traj_op> ops(b.num_ops);
+  QHIP_CHECK(hipMemcpy(d.data(), b.descs, d.size() * sizeof(d[0]),
+                       hipMemcpyDeviceToHost));
+  if (!ops.empty()) {
+    QHIP_CHECK(hipMemcpy(ops.data(), b.ops, ops.size() * sizeof(ops[0]),
+                         hipMemcpyDeviceToHost));
+  }
+  return BuildTiled(b, d, ops, {});
+}
+
 void Release(TrajBatch* b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -1426,6 +1504,7 @@ void Release(TrajBatch* b) {
   (void)hipFree(b->passes);
   (void)hipFree(b->recs);
   (void)hipFree(b->items);
+  (void)hipFree(b->sweeps);
   (void)hipFree(b->parts);
   delete b;
 }
@@ -1547,16 +1626,12 @@ static int TrajPrepare(const qsim_hip_traj_desc* trajs, unsigned num_traj,
       }
     }
     QHIP_TRY(BuildTilePasses(jobs, matrices, passes, recs));
-    if (!passes.empty()) QHIP_TRY(TileKernelReady());
   }
   // Released (device buffers included) on every early return or exception.
   std::unique_ptr<TrajBatch, void (*)(TrajBatch*)> b(new TrajBatch, Release);
   b->num_traj = num_traj;
-  std::vector<TrajItem> items;
-  uint64_t num_parts = 0;
-  TrajSchedule(d, ov, passes, unsigned(NumCUs()), items, b->launches,
-               num_parts);
   b->pool_size = pool;
+  b->num_ops = num_ops;
   b->num_pairs = num_pairs;
   b->num_decisions = num_decisions;
   for (unsigned t = 0; t < num_traj; ++t) {
@@ -1568,18 +1643,17 @@ static int TrajPrepare(const qsim_hip_traj_desc* trajs, unsigned num_traj,
   if (rc == QSIM_HIP_OK) rc = Upload(&b->ops, ov.data(), num_ops);
   if (rc == QSIM_HIP_OK) rc = Upload(&b->passes, passes.data(), passes.size());
   if (rc == QSIM_HIP_OK) rc = Upload(&b->recs, recs.data(), recs.size());
-  if (rc == QSIM_HIP_OK) rc = Upload(&b->items, items.data(), items.size());
   if (rc == QSIM_HIP_OK) rc = Upload(&b->mats, matrices, num_floats);
   if (rc == QSIM_HIP_OK) rc = Upload(&b->pairs, pairs, size_t(2) * num_pairs);
   if (rc == QSIM_HIP_OK) {
     hipError_t e = hipMalloc(&b->pool, pool * sizeof(float2));
     if (e == hipSuccess) e = hipMalloc(&b->zz, std::max<size_t>(num_pairs, 1) * 8);
     if (e == hipSuccess) e = hipMalloc(&b->norms, size_t(num_traj) * 8);
-    if (e == hipSuccess) e = hipMalloc(&b->parts, num_parts * sizeof(double));
     if (e == hipSuccess)
       e = hipMalloc(&b->dec, std::max<size_t>(num_decisions, 1) * 4);
     if (e != hipSuccess) rc = HipFail(e, "trajectory batch buffers");
   }
+  if (rc == QSIM_HIP_OK && !passes.empty()) rc = BuildTiled(*b, d, ov, passes);
   if (rc != QSIM_HIP_OK) return rc;
   *handle = b.release();
   return QSIM_HIP_OK;
@@ -1607,6 +1681,9 @@ int qsim_hip_traj_run(void* handle, unsigned threads, int use_graph) {
   QHIP_TRY(FlushGateQueue());
   auto* b = static_cast<TrajBatch*>(handle);
   if (b == nullptr) return QSIM_HIP_ERR_ARG;
+  if (threads == QSIM_HIP_TRAJ_TILED && !b->tiled) {
+    QHIP_TRY(GuardHost([&]() -> int { return BuildTiledFromDevice(*b); }));
+  }
   // Undecided slots read -1 (the decision kernel writes the reached ones).
   hipLaunchKernelGGL(FillInt, dim3((b->num_decisions + 255) / 256 + 1),
                      dim3(256), 0, Stream(), b->dec, b->num_decisions, -1);

@@ -6,6 +6,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 import qsim_amd
 from helpers import random_matrix, to_interleaved
@@ -72,17 +73,21 @@ class Batch:
                            len(self.pairs), int(normalise)))
         self.pairs += pairs
 
-    def run(self, threads, graph=0, repeats=1):
-        lib = qsim_amd.lib()
+    def prepare(self):
         descs, ops = np.array(self.descs, DESC), np.stack(self.ops).astype(OP)
         mats = np.concatenate(self.mats).astype(np.float32)
         pr = np.asarray(self.pairs, np.uint32).reshape(-1)
         h = ctypes.c_void_p()
-        qsim_amd._check(lib.qsim_hip_traj_prepare(
+        qsim_amd._check(qsim_amd.lib().qsim_hip_traj_prepare(
             descs.ctypes.data, len(descs), ops.ctypes.data, len(ops),
             mats.ctypes.data, mats.size,
             pr.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)),
             len(self.pairs), self.slots, ctypes.byref(h)))
+        return h
+
+    def run(self, threads, graph=0, repeats=1):
+        lib = qsim_amd.lib()
+        h = self.prepare()
         zz = np.zeros(len(self.pairs), np.float64)
         dec = np.zeros(self.slots, np.int32)
         states = [np.zeros(2 << n, np.float32) for n, *_ in self.descs]
@@ -184,3 +189,28 @@ def test_tiled_batch_matches_per_gate_kernel(tile_bits, sizes):
         for n, (x, y) in zip(sizes, zip(st, states)):
             assert np.linalg.norm(x - y) < 1e-5, n
             assert abs(np.linalg.norm(x) - 1) < 1e-5
+
+
+def test_batch_memory_follows_its_streams():
+    # 8000 gates on 24 qubits: 1024 sweep chunks a gate.  Beyond the state and
+    # the operations (64 bytes a gate), a batch takes a few bytes a gate, not
+    # a few a chunk, before it is run tiled and after.
+    n, gates = 24, 8000
+    u = random_matrix(1, np.random.default_rng(3))
+    b = Batch()
+    moff = b.put(u)
+
+    def build(b):
+        for i in range(gates):
+            b.op(GATE, [i % n], moff=moff)
+    b.trajectory(n, build, False, [(0, n - 1)])
+    lib = qsim_amd.lib()
+    free0 = torch.cuda.mem_get_info()[0]
+    h = b.prepare()
+    try:
+        limit = (8 << n) + 64 * gates + (16 << 20)
+        assert free0 - torch.cuda.mem_get_info()[0] < limit
+        qsim_amd._check(lib.qsim_hip_traj_run(h, TILED, 0))
+        assert free0 - torch.cuda.mem_get_info()[0] < limit + (16 << 20)
+    finally:
+        qsim_amd._check(lib.qsim_hip_traj_free(h))
