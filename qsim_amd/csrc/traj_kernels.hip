@@ -560,8 +560,15 @@ __device__ __forceinline__ TrajSweep SweepOf(const TrajSweep* __restrict__ e,
   return e[__builtin_amdgcn_readfirstlane(lo)];
 }
 
-// Amplitudes of a sweep chunk.
+// Amplitudes of a sweep chunk: 2^14, and more where a trajectory would have
+// over 1024 chunks, so that the steps that add up a trajectory's chunks in one
+// workgroup (TrajChannelPickKernel, TrajFinishKernel) stay short.
 constexpr uint64_t kSweepChunk = uint64_t{1} << 14;
+constexpr unsigned kMaxChunkBits = 10;
+__host__ __device__ inline uint64_t ChunkSize(unsigned n) {
+  return n > 14 + kMaxChunkBits ? uint64_t{1} << (n - kMaxChunkBits)
+                                : kSweepChunk;
+}
 constexpr int kSweepNT = 256;
 // Partial sums of a channel's chunk (ChannelSums), at most.
 constexpr unsigned kChanSums = 16;
@@ -686,7 +693,7 @@ TrajOneKernel(const qsim_hip_traj_desc* __restrict__ descs, unsigned num,
 __device__ __forceinline__ void SweepGroups(unsigned n, unsigned k,
                                             uint64_t chunk, uint64_t& lo,
                                             uint64_t& hi) {
-  const uint64_t all = uint64_t{1} << (n - k), per = kSweepChunk >> k;
+  const uint64_t all = uint64_t{1} << (n - k), per = ChunkSize(n) >> k;
   lo = chunk * per;
   hi = lo + per < all ? lo + per : all;
 }
@@ -791,22 +798,20 @@ TrajChannelSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
     ChannelSums<2>(s, d.num_qubits, h.q, chunk, out);
 }
 
-// The walk of RunIteration (lib/qtrajectory.h:330-370) over the operators'
-// probabilities, the same in every workgroup of the trajectory, then the
-// chosen operator on this item's chunk.
-__global__ void __launch_bounds__(kSweepNT)
-TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
-                       const qsim_hip_traj_op* __restrict__ ops,
-                       const float* __restrict__ mats,
-                       const TrajSweep* __restrict__ sweeps, unsigned num,
-                       float2* __restrict__ pool,
-                       const double* __restrict__ parts,
-                       int32_t* __restrict__ dec_out) {
-  __shared__ float lm[2 * 4 * 4];
+// A channel's choice: the operator (-1: none) and the scale that normalises
+// the state.
+struct TrajPick {
+  int32_t op;
+  float scale;
+};
+
+// The trajectory's chunk sums added up by the workgroup, then the walk of
+// RunIteration (lib/qtrajectory.h:330-370) over the operators' probabilities,
+// the same in every thread.
+__device__ __forceinline__ TrajPick PickOperator(
+    const qsim_hip_traj_op* __restrict__ ops, const float* __restrict__ mats,
+    const TrajSweep& it, const double* __restrict__ parts) {
   __shared__ double sums[kChanSums];
-  const TrajSweep it = SweepOf(sweeps, num);
-  const unsigned chunk = blockIdx.x - it.first;
-  const qsim_hip_traj_desc d = descs[it.traj];
   const qsim_hip_traj_op h = ops[it.op];
   const bool normalise = h.pad & 1u;
   const unsigned DC = 1u << h.moff2;  // states of the channel's qubits
@@ -839,8 +844,48 @@ TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
       break;
     }
   }
-  if (chunk == 0 && threadIdx.x == 0) dec_out[h.slot] = pick;
-  const float a = normalise ? float(1.0 / std::sqrt(norm)) : 1.0f;
+  return TrajPick{pick, normalise ? float(1.0 / std::sqrt(norm)) : 1.0f};
+}
+
+// The choices of a launch's channels, one workgroup a trajectory, where a
+// trajectory has more than kPickChunks chunks.  Picked by every workgroup of
+// the apply launch, the sums read grow with the square of the chunks; a launch
+// more costs 2 us.  Four channels on one qubit, picked there / here: 18 qubits
+// (16 chunks) 124 / 131 us, 22 (256) 176 / 169, 24 422 / 365, 28 21.2 / 6.1
+// ms; on two qubits 28 qubits 66.1 / 6.2 ms.
+constexpr unsigned kPickChunks = 64;
+__global__ void __launch_bounds__(kSweepNT)
+TrajChannelPickKernel(const qsim_hip_traj_op* __restrict__ ops,
+                      const float* __restrict__ mats,
+                      const TrajSweep* __restrict__ sweeps,
+                      const double* __restrict__ parts,
+                      TrajPick* __restrict__ picks) {
+  const TrajSweep it = sweeps[blockIdx.x];
+  const TrajPick p = PickOperator(ops, mats, it, parts);
+  if (threadIdx.x == 0) picks[it.traj] = p;
+}
+
+// The chosen operator (PICK: chosen here) on this workgroup's chunk.
+template <bool PICK>
+__global__ void __launch_bounds__(kSweepNT)
+TrajChannelApplyKernel(const qsim_hip_traj_desc* __restrict__ descs,
+                       const qsim_hip_traj_op* __restrict__ ops,
+                       const float* __restrict__ mats,
+                       const TrajSweep* __restrict__ sweeps, unsigned num,
+                       float2* __restrict__ pool,
+                       const double* __restrict__ parts,
+                       const TrajPick* __restrict__ picks,
+                       int32_t* __restrict__ dec_out) {
+  __shared__ float lm[2 * 4 * 4];
+  const TrajSweep it = SweepOf(sweeps, num);
+  const unsigned chunk = blockIdx.x - it.first;
+  const qsim_hip_traj_desc d = descs[it.traj];
+  const bool normalise = ops[it.op].pad & 1u;
+  const TrajPick p =
+      PICK ? PickOperator(ops, mats, it, parts) : picks[it.traj];
+  const int pick = p.op;
+  const float a = p.scale;
+  if (chunk == 0 && threadIdx.x == 0) dec_out[ops[it.op].slot] = pick;
   float2* s = pool + d.state_offset;
   const qsim_hip_traj_op c = ops[it.op + 1 + (pick >= 0 ? pick : 0)];
   uint64_t lo, hi;
@@ -902,11 +947,11 @@ __device__ __forceinline__ double LaneTransform(double v) {
   return LaneButterfly<5>(v);
 }
 
-// Partial sums of a chunk: one per pair, then the norm.  A pair's sum over
-// the chunk is the Walsh-Hadamard coefficient of |s_i|^2 at (1 << a) ^
-// (1 << b) (the chunk's own bits give a sign), so the coefficients of at most
-// two set bits are made once, whatever the number of pairs, from one read of
-// the chunk.  Index bits of a chunk: 0-5 the lane, 6-7 the wave, 8-13 "own":
+// Partial sums of a chunk: one per pair, then the norm, 2^14 amplitudes a
+// round.  A pair's sum over a round is the Walsh-Hadamard coefficient of
+// |s_i|^2 at (1 << a) ^ (1 << b) (the higher index bits give a sign), so the
+// coefficients of at most two set bits are made once, whatever the number of
+// pairs, from one read of the round.  Index bits of a round: 0-5 the lane, 6-7 the wave, 8-13 "own":
 // a thread's 64 amplitudes, 16 a step.  A thread sums 1 + 6 + 15 coefficients
 // over its own bits; the first 7 take a transform over the lanes, the last 15
 // (two bits already) are needed at lane 0 only; the four waves are combined
@@ -929,75 +974,80 @@ TrajFinishSumKernel(const qsim_hip_traj_desc* __restrict__ descs,
   const unsigned chunk = blockIdx.x - it.first;
   const qsim_hip_traj_desc d = descs[it.traj];
   const float2* __restrict__ s = pool + d.state_offset;
-  uint64_t lo, hi;
-  SweepGroups(d.num_qubits, 0, chunk, lo, hi);
+  double* out = parts + it.part + uint64_t(chunk) * (d.num_pairs + 1);
+  uint64_t begin, hi;
+  SweepGroups(d.num_qubits, 0, chunk, begin, hi);
   auto two = [](unsigned b, unsigned c) { return c * (c - 1) / 2 + b; };
-  double none = 0.0, one[kChunkOwn] = {}, both[15] = {};
-  // Unrolled, all steps' loads would be issued first and their values spilled.
+  // One round, more in the long chunks of more than 24 qubits.
+  for (uint64_t lo = begin; lo < hi; lo += kSweepChunk) {
+    if (lo != begin) __syncthreads();  // red is read
+    double none = 0.0, one[kChunkOwn] = {}, both[15] = {};
+    // Unrolled, all steps' loads would be issued first and their values spilled.
 #pragma unroll 1
-  for (unsigned t = 0; t < 4; ++t) {
-    // The signs of the step's two bits.
-    const double s4 = t & 1u ? -1.0 : 1.0, s5 = t & 2u ? -1.0 : 1.0;
-    double w[16];
-#pragma unroll
-    for (unsigned u = 0; u < 16; ++u) {
-      const uint64_t i = lo + (t * 16 + u) * kSweepNT + threadIdx.x;
-      const float2 a = i < hi ? s[i] : float2{0.0f, 0.0f};
-      w[u] = double(a.x) * a.x + double(a.y) * a.y;
-    }
-#pragma unroll
-    for (unsigned b = 0; b < 4; ++b)
+    for (unsigned t = 0; t < 4; ++t) {
+      // The signs of the step's two bits.
+      const double s4 = t & 1u ? -1.0 : 1.0, s5 = t & 2u ? -1.0 : 1.0;
+      double w[16];
 #pragma unroll
       for (unsigned u = 0; u < 16; ++u) {
-        if ((u >> b) & 1u) continue;
-        const double x = w[u], y = w[u | (1u << b)];
-        w[u] = x + y;
-        w[u | (1u << b)] = x - y;
+        const uint64_t i = lo + (t * 16 + u) * kSweepNT + threadIdx.x;
+        const float2 a = i < hi ? s[i] : float2{0.0f, 0.0f};
+        w[u] = double(a.x) * a.x + double(a.y) * a.y;
       }
-    none += w[0];
-    one[4] = fma(s4, w[0], one[4]);
-    one[5] = fma(s5, w[0], one[5]);
-    both[two(4, 5)] = fma(s4 * s5, w[0], both[two(4, 5)]);
 #pragma unroll
-    for (unsigned b = 0; b < 4; ++b) {
-      const double v = w[1u << b];
-      one[b] += v;
-      both[two(b, 4)] = fma(s4, v, both[two(b, 4)]);
-      both[two(b, 5)] = fma(s5, v, both[two(b, 5)]);
+      for (unsigned b = 0; b < 4; ++b)
 #pragma unroll
-      for (unsigned c = b + 1; c < 4; ++c)
-        both[two(b, c)] += w[(1u << b) | (1u << c)];
+        for (unsigned u = 0; u < 16; ++u) {
+          if ((u >> b) & 1u) continue;
+          const double x = w[u], y = w[u | (1u << b)];
+          w[u] = x + y;
+          w[u | (1u << b)] = x - y;
+        }
+      none += w[0];
+      one[4] = fma(s4, w[0], one[4]);
+      one[5] = fma(s5, w[0], one[5]);
+      both[two(4, 5)] = fma(s4 * s5, w[0], both[two(4, 5)]);
+#pragma unroll
+      for (unsigned b = 0; b < 4; ++b) {
+        const double v = w[1u << b];
+        one[b] += v;
+        both[two(b, 4)] = fma(s4, v, both[two(b, 4)]);
+        both[two(b, 5)] = fma(s5, v, both[two(b, 5)]);
+#pragma unroll
+        for (unsigned c = b + 1; c < 4; ++c)
+          both[two(b, c)] += w[(1u << b) | (1u << c)];
+      }
     }
-  }
-  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  red[wave][lane] = LaneTransform(none);
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    red[wave][lane] = LaneTransform(none);
 #pragma unroll
-  for (unsigned b = 0; b < kChunkOwn; ++b)
-    red[wave][64 * (1 + b) + lane] = LaneTransform(one[b]);
+    for (unsigned b = 0; b < kChunkOwn; ++b)
+      red[wave][64 * (1 + b) + lane] = LaneTransform(one[b]);
 #pragma unroll
-  for (unsigned j = 0; j < 15; ++j) {
-    const double v = LaneTransform(both[j]);
-    if (lane == 0) red[wave][64 * (1 + kChunkOwn) + j] = v;
-  }
-  __syncthreads();
-  double* out = parts + it.part + uint64_t(chunk) * (d.num_pairs + 1);
-  for (unsigned j = threadIdx.x; j <= d.num_pairs; j += kSweepNT) {
-    uint64_t m = 0;  // at most two bits; none for the norm
-    if (j < d.num_pairs)
-      m = (uint64_t{1} << pairs[2 * (d.pair_offset + j)]) ^
-          (uint64_t{1} << pairs[2 * (d.pair_offset + j) + 1]);
-    const unsigned own = unsigned(m >> 8) & 63u, waves = unsigned(m >> 6) & 3u;
-    unsigned at = unsigned(m) & 63u;
-    if (own != 0) {
-      const unsigned c = 31 - __builtin_clz(own), rest = own ^ (1u << c);
-      at = rest == 0 ? 64 * (1 + c) + at
-                     : 64 * (1 + kChunkOwn) + two(31 - __builtin_clz(rest), c);
+    for (unsigned j = 0; j < 15; ++j) {
+      const double v = LaneTransform(both[j]);
+      if (lane == 0) red[wave][64 * (1 + kChunkOwn) + j] = v;
     }
-    double v = 0.0;
+    __syncthreads();
+    for (unsigned j = threadIdx.x; j <= d.num_pairs; j += kSweepNT) {
+      uint64_t m = 0;  // at most two bits; none for the norm
+      if (j < d.num_pairs)
+        m = (uint64_t{1} << pairs[2 * (d.pair_offset + j)]) ^
+            (uint64_t{1} << pairs[2 * (d.pair_offset + j) + 1]);
+      const unsigned own = unsigned(m >> 8) & 63u, waves = unsigned(m >> 6) & 3u;
+      unsigned at = unsigned(m) & 63u;
+      if (own != 0) {
+        const unsigned c = 31 - __builtin_clz(own), rest = own ^ (1u << c);
+        at = rest == 0 ? 64 * (1 + c) + at
+                       : 64 * (1 + kChunkOwn) + two(31 - __builtin_clz(rest), c);
+      }
+      double v = 0.0;
 #pragma unroll
-    for (unsigned w = 0; w < kSweepNT / 64; ++w)
-      v += __builtin_popcount(w & waves) & 1 ? -red[w][at] : red[w][at];
-    out[j] = __builtin_popcountll(lo & m) & 1 ? -v : v;
+      for (unsigned w = 0; w < kSweepNT / 64; ++w)
+        v += __builtin_popcount(w & waves) & 1 ? -red[w][at] : red[w][at];
+      if (__builtin_popcountll(lo & m) & 1) v = -v;
+      out[j] = lo == begin ? v : out[j] + v;
+    }
   }
 }
 
@@ -1022,6 +1072,7 @@ TrajFinishKernel(const qsim_hip_traj_desc* __restrict__ descs,
   if (threadIdx.x == 0 && (d.pad & 1u)) norm_out[it.traj] = nrm;
   for (unsigned j = threadIdx.x; j < np; j += kSweepNT) {
     double acc = 0.0;
+#pragma unroll 4
     for (unsigned c = 0; c < it.count; ++c) acc += in[uint64_t(c) * (np + 1) + j];
     zz_out[d.pair_offset + j] = acc / nrm;
   }
@@ -1029,8 +1080,8 @@ TrajFinishKernel(const qsim_hip_traj_desc* __restrict__ descs,
 
 // One launch of a tiled batch.
 struct TrajLaunch {
-  enum Kind { kPass14, kPass13, kPass12, kGate, kChannelSum, kChannelApply,
-              kFinishSum, kFinish } kind;
+  enum Kind { kPass14, kPass13, kPass12, kGate, kChannelSum, kChannelPick,
+              kChannelApply, kChannelPickApply, kFinishSum, kFinish } kind;
   uint64_t first;   // items (passes), sweep entries (the rest)
   uint32_t count;
   uint32_t blocks;  // workgroups
@@ -1066,6 +1117,7 @@ struct TrajBatch {
   TrajItem* items = nullptr;
   TrajSweep* sweeps = nullptr;
   double* parts = nullptr;
+  TrajPick* picks = nullptr;  // by trajectory
   uint64_t pool_size = 0;  // amplitudes
   uint64_t num_ops = 0;
   std::vector<uint64_t> state_offset;
@@ -1134,7 +1186,7 @@ TrajPlan TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
   for (uint32_t t = 0; t < T; ++t) at[t] = d[t].op_begin;
   auto chunks = [&](uint32_t t) {
     const uint64_t N = uint64_t{1} << d[t].num_qubits;
-    return uint32_t(std::max<uint64_t>(1, N / kSweepChunk));
+    return uint32_t(std::max<uint64_t>(1, N / ChunkSize(d[t].num_qubits)));
   };
   // A launch over the trajectories of `list`; blocks: one workgroup an entry
   // or (0) one a chunk.
@@ -1175,7 +1227,14 @@ TrajPlan TrajSchedule(const std::vector<qsim_hip_traj_desc>& d,
     if (!gates.empty() || !channels.empty()) {
       sweep(TrajLaunch::kGate, gates, 0);
       sweep(TrajLaunch::kChannelSum, channels, 0);
-      sweep(TrajLaunch::kChannelApply, channels, 0);
+      if (std::any_of(channels.begin(), channels.end(), [](const TrajSweep& e) {
+            return e.count > kPickChunks;
+          })) {
+        sweep(TrajLaunch::kChannelPick, channels, uint32_t(channels.size()));
+        sweep(TrajLaunch::kChannelApply, channels, 0);
+      } else {
+        sweep(TrajLaunch::kChannelPickApply, channels, 0);
+      }
       continue;
     }
     if (!pass) break;
@@ -1276,10 +1335,19 @@ int LaunchTiled(TrajBatch& b, hipStream_t st) {
         hipLaunchKernelGGL(TrajChannelSumKernel, grid, nt, 0, st, b.descs,
                            b.ops, sw, l.count, b.pool, b.parts);
         break;
+      case TrajLaunch::kChannelPick:
+        hipLaunchKernelGGL(TrajChannelPickKernel, grid, nt, 0, st, b.ops,
+                           b.mats, sw, b.parts, b.picks);
+        break;
       case TrajLaunch::kChannelApply:
-        hipLaunchKernelGGL(TrajChannelApplyKernel, grid, nt, 0, st, b.descs,
-                           b.ops, b.mats, sw, l.count, b.pool, b.parts,
-                           b.dec);
+        hipLaunchKernelGGL(TrajChannelApplyKernel<false>, grid, nt, 0, st,
+                           b.descs, b.ops, b.mats, sw, l.count, b.pool,
+                           b.parts, b.picks, b.dec);
+        break;
+      case TrajLaunch::kChannelPickApply:
+        hipLaunchKernelGGL(TrajChannelApplyKernel<true>, grid, nt, 0, st,
+                           b.descs, b.ops, b.mats, sw, l.count, b.pool,
+                           b.parts, b.picks, b.dec);
         break;
       case TrajLaunch::kFinishSum:
         hipLaunchKernelGGL(TrajFinishSumKernel, grid, nt, 0, st, b.descs,
@@ -1466,12 +1534,15 @@ int BuildTiled(TrajBatch& b, const std::vector<qsim_hip_traj_desc>& d,
   (void)hipFree(b.items);
   (void)hipFree(b.sweeps);
   (void)hipFree(b.parts);
+  (void)hipFree(b.picks);
   b.items = nullptr;
   b.sweeps = nullptr;
   b.parts = nullptr;
+  b.picks = nullptr;
   QHIP_TRY(Upload(&b.items, plan.items.data(), plan.items.size()));
   QHIP_TRY(Upload(&b.sweeps, plan.sweeps.data(), plan.sweeps.size()));
   QHIP_CHECK(hipMalloc(&b.parts, plan.num_parts * sizeof(double)));
+  QHIP_CHECK(hipMalloc(&b.picks, b.num_traj * sizeof(TrajPick)));
   b.launches = std::move(plan.launches);
   b.tiled = true;
   return QSIM_HIP_OK;
@@ -1506,6 +1577,7 @@ void Release(TrajBatch* b) {
   (void)hipFree(b->items);
   (void)hipFree(b->sweeps);
   (void)hipFree(b->parts);
+  (void)hipFree(b->picks);
   delete b;
 }
 

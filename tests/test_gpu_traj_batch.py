@@ -191,6 +191,19 @@ def test_tiled_batch_matches_per_gate_kernel(tile_bits, sizes):
             assert abs(np.linalg.norm(x) - 1) < 1e-5
 
 
+def test_long_chunks_match_per_gate_kernel():
+    # Above 24 qubits a chunk has more than 2^14 amplitudes: four rounds of
+    # the final sums here, channels on one and two qubits, 17 pairs.
+    sizes = [9, 10, 11, 26]
+    b = random_batch(sizes, 14, np.random.default_rng(26))
+    zz, dec, states = b.run(512)
+    zt, dt, st = b.run(TILED)
+    np.testing.assert_array_equal(dt, dec)
+    np.testing.assert_allclose(zt, zz, atol=1e-5, rtol=0)
+    for n, x, y in zip(sizes, st, states):
+        assert np.linalg.norm(x - y) < 1e-5, n
+
+
 def test_batch_memory_follows_its_streams():
     # 8000 gates on 24 qubits: 1024 sweep chunks a gate.  Beyond the state and
     # the operations (64 bytes a gate), a batch takes a few bytes a gate, not
