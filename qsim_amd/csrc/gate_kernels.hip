@@ -174,7 +174,7 @@ GateTileKernel(typename Cplx<FP>::T* __restrict__ s, TileGeom g, M m) {
 // half line) cannot skip memory: its lanes load and store too and keep
 // their values; masked partial lines measured 7 % slower (28 qubits,
 // control 0).  Controls above are skipped as any other high qubit.
-template <typename FP, int K, typename M>
+template <typename FP, int K, bool FAR, typename M>
 __global__ void __launch_bounds__(256)
 GateLaneKernel(typename Cplx<FP>::T* __restrict__ s, LaneGeom g, M m) {
   using C = typename Cplx<FP>::T;
@@ -186,8 +186,7 @@ GateLaneKernel(typename Cplx<FP>::T* __restrict__ s, LaneGeom g, M m) {
   for (int b = 0; b < 6; ++b) loff += uint64_t((lane >> b) & 1u) << g.lane[b];
   const uint64_t stride = uint64_t(gridDim.x) * 4;
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (uint64_t c = uint64_t(blockIdx.x) * 4 + wave; c < g.nchunks;
-       c += stride) {
+  for (uint64_t c = LaneBlock<FAR>() * 4 + wave; c < g.nchunks; c += stride) {
     C* p = s + (InsertZeros(c << g.low, g.ins, g.nins) | g.cbits);
     C v[D], u[D];
 #pragma unroll
@@ -339,8 +338,14 @@ int LaunchLane(typename Cplx<FP>::T* s, const LaneGeom& g, const M& m) {
   const uint64_t blocks =
       std::min<uint64_t>((g.nchunks + 3) / 4, uint64_t{1} << 20);
   PassTimerBegin();
-  hipLaunchKernelGGL((GateLaneKernel<FP, K, M>), dim3(unsigned(blocks)),
-                     dim3(256), 0, Stream(), s, g, m);
+  // Only what LaneFar can answer with true.
+  constexpr bool far = K == 4 || (K == 2 && sizeof(FP) == 4);
+  if (far && LaneFar<FP, K>(g))
+    hipLaunchKernelGGL((GateLaneKernel<FP, K, far, M>), dim3(unsigned(blocks)),
+                       dim3(256), 0, Stream(), s, g, m);
+  else
+    hipLaunchKernelGGL((GateLaneKernel<FP, K, false, M>),
+                       dim3(unsigned(blocks)), dim3(256), 0, Stream(), s, g, m);
   PassTimerEnd();
   QHIP_LAUNCHED("GateLaneKernel");
   return QSIM_HIP_OK;

@@ -316,6 +316,7 @@ __device__ __forceinline__ void LaneProduct(const RegFragF32<4>& af,
     }
 }
 
+template <bool FAR>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(3)))
 GateMfmaLaneKernel(float2* __restrict__ s, LaneGeom g,
@@ -325,7 +326,7 @@ GateMfmaLaneKernel(float2* __restrict__ s, LaneGeom g,
   RegFragF32<4> af;
   af.Load(frag);
   const uint64_t wstride = uint64_t(gridDim.x) * kWaves;
-  for (uint64_t c = uint64_t(blockIdx.x) * kWaves + wave; c < g.nchunks;
+  for (uint64_t c = LaneBlock<FAR>() * kWaves + wave; c < g.nchunks;
        c += wstride) {
     float2* p = s + InsertZeros(c << 6, g.ins, g.nins);
     float2 v[16], u[16];
@@ -636,8 +637,13 @@ int DispatchMfma(float2* s, unsigned n, const unsigned* qs, const double* m64,
     const uint64_t blocks = std::min<uint64_t>(
         (g.nchunks + kWaves - 1) / kWaves, uint64_t{1} << 20);
     PassTimerBegin();
-    hipLaunchKernelGGL(GateMfmaLaneKernel, dim3(unsigned(blocks)), dim3(256),
-                       0, Stream(), s, g, static_cast<const float*>(dfrag));
+    const float* frag = static_cast<const float*>(dfrag);
+    if (LaneFar<float, K>(g))
+      hipLaunchKernelGGL(GateMfmaLaneKernel<true>, dim3(unsigned(blocks)),
+                         dim3(256), 0, Stream(), s, g, frag);
+    else
+      hipLaunchKernelGGL(GateMfmaLaneKernel<false>, dim3(unsigned(blocks)),
+                         dim3(256), 0, Stream(), s, g, frag);
     PassTimerEnd();
     QHIP_LAUNCHED("GateMfmaLaneKernel");
     return QSIM_HIP_OK;

@@ -214,6 +214,28 @@ def test_lane_kernel_edges(dtype, controls, sim):
                                               s.reshape(-1, 2)[out])
 
 
+@pytest.mark.parametrize("dtype,n,qs,controls", [
+    (np.float32, 23, [19, 20, 21, 22], []),
+    (np.float32, 24, [19, 21, 22, 23], []),
+    (np.float64, 22, [18, 19, 20, 21], []),
+    (np.float64, 23, [18, 20, 21, 22], [5]),
+    (np.float32, 17, [9, 16], [1]),
+    (np.float32, 18, [16, 17], [0, 2]),
+    (np.float32, 20, [7, 18], [1, 9])])
+def test_lane_kernel_far_members(dtype, n, qs, controls, sim):
+    # Workgroups in runs of 32 per XCD: members 4 MiB apart, and two targets
+    # with a control below qubit 3, at the smallest grids (a multiple of 256
+    # workgroups, and one below it).
+    rng = np.random.default_rng(n)
+    m = to_interleaved(random_matrix(len(qs), rng), dtype)
+    s = random_state(n, rng, dtype)
+    st = upload(s, n, dtype)
+    cvals = (1 << len(controls)) - 1
+    sim.apply_controlled_gate(qs, controls, cvals, m, st)
+    oracle.apply_controlled_gate(n, s, qs, controls, cvals, m)
+    assert rel_l2(st.to_numpy(), s) < TOL[dtype]
+
+
 @pytest.mark.parametrize("k", [5, 6])
 @pytest.mark.parametrize("n", [9, 10, 11, 12, 16, 22])
 def test_complex128_wide_gates(n, k, sim):
