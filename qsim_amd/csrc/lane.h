@@ -44,8 +44,9 @@ struct LaneGeom {
 // This workgroup's place.  Workgroups go to the XCDs in turn; taken in order,
 // an XCD's waves in flight lie eight workgroups apart in every member's run,
 // and with the members at large powers of two they meet few HBM channels: 29
-// qubits, complex64 k = 4, targets 19..22 2.41 ms, 23..26 1.52.  FAR: an XCD
-// takes runs of 32 consecutive workgroups instead, where LaneFar says so.
+// qubits, complex64 k = 4, targets 19..22 2.46 ms, 23..26 1.53.  FAR: an XCD
+// takes runs of 32 consecutive workgroups instead (1.60 and 1.56), where
+// LaneFar says so.
 template <bool FAR>
 __device__ __forceinline__ uint64_t LaneBlock() {
   constexpr unsigned kRun = 32;

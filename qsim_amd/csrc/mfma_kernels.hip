@@ -29,8 +29,9 @@
 // for e = 0..7 over a K block of 16, i.e. 4 members per lane half.
 //
 // Data paths: k = 4 holds a group per lane and swaps low targets across
-// lanes (GateMfmaLaneKernel).  k = 5, 6 keep each wave's rows of the matrix in
-// registers (f16_kernels.hip); on states too small for that, targets all at
+// lanes (GateMfmaLaneKernel), except on up to 20 qubits without a target below
+// qubit 5.  k = 5, 6 keep each wave's rows of the matrix in
+// registers (f16_kernels.hip).  On smaller states, targets all at
 // qubit >= 5 read the operands straight from HBM (32 lanes = 32 consecutive
 // amplitudes) and a target below qubit 5 stages a tile in LDS (XOR-swizzled
 // to spread banks).
@@ -493,40 +494,47 @@ uint64_t DepositBits(uint64_t v, uint64_t mask) {
   return r;
 }
 
-// k = 5, 6 on states too small for the row-block kernels: a batch of 32
-// groups per wave, operands straight from HBM or from an LDS tile.
+// A batch of 32 groups per wave, operands straight from HBM: no target below
+// qubit 5.
+template <int K>
+int LaunchBatchesReg(float2* s, unsigned n, const unsigned* qs, void* dfrag,
+                     bool bf16) {
+  GateGeom g{};
+  g.nins = K;
+  for (int b = 0; b < K; ++b) {
+    g.ins[b] = qs[b];
+    g.tbit[b] = uint64_t{1} << qs[b];
+  }
+  g.ngroups = uint64_t{1} << (n - K);
+  g.cbits = 0;
+  // Every wave batch is 32 consecutive groups (no target below qubit 5).
+  uint64_t nbatch = g.ngroups >> 5;
+  // About one batch per wave: equal short waves leave no partial last
+  // round of resident waves.
+  uint64_t blocks = std::min<uint64_t>((nbatch + kWaves - 1) / kWaves,
+                                       uint64_t{1} << 20);
+  blocks = std::max<uint64_t>(blocks, 1);
+  PassTimerBegin();
+  if (!bf16) {
+    hipLaunchKernelGGL(GateMfmaRegKernel<K>, dim3(unsigned(blocks)),
+                       dim3(256), 0, Stream(), reinterpret_cast<float*>(s), g,
+                       static_cast<const float*>(dfrag));
+  } else if constexpr (K >= 5) {
+    hipLaunchKernelGGL(GateBf16RegKernel<K>, dim3(unsigned(blocks)),
+                       dim3(256), 0, Stream(), s, g,
+                       static_cast<const uint16_t*>(dfrag));
+  }
+  PassTimerEnd();
+  QHIP_LAUNCHED("GateMfmaRegKernel");
+  return QSIM_HIP_OK;
+}
+
+// k = 5, 6 on states too small for the row-block kernels: batches of 32
+// groups, straight from HBM or from an LDS tile.
 template <int K>
 int LaunchBatches(float2* s, unsigned n, const unsigned* qs, void* dfrag,
                   bool bf16) {
-  if (qs[0] >= 5) {
-    GateGeom g{};
-    g.nins = K;
-    for (int b = 0; b < K; ++b) {
-      g.ins[b] = qs[b];
-      g.tbit[b] = uint64_t{1} << qs[b];
-    }
-    g.ngroups = uint64_t{1} << (n - K);
-    g.cbits = 0;
-    // Every wave batch is 32 consecutive groups (no target below qubit 5).
-    uint64_t nbatch = g.ngroups >> 5;
-    // About one batch per wave: equal short waves leave no partial last
-    // round of resident waves.
-    uint64_t blocks = std::min<uint64_t>((nbatch + kWaves - 1) / kWaves,
-                                         uint64_t{1} << 20);
-    blocks = std::max<uint64_t>(blocks, 1);
-    PassTimerBegin();
-    if (!bf16)
-      hipLaunchKernelGGL(GateMfmaRegKernel<K>, dim3(unsigned(blocks)),
-                         dim3(256), 0, Stream(), reinterpret_cast<float*>(s), g,
-                         static_cast<const float*>(dfrag));
-    else
-      hipLaunchKernelGGL(GateBf16RegKernel<K>, dim3(unsigned(blocks)),
-                         dim3(256), 0, Stream(), s, g,
-                         static_cast<const uint16_t*>(dfrag));
-    PassTimerEnd();
-    QHIP_LAUNCHED("GateMfmaRegKernel");
-    return QSIM_HIP_OK;
-  }
+  if (qs[0] >= 5) return LaunchBatchesReg<K>(s, n, qs, dfrag, bf16);
 
   // Tile path: 2^12 amplitudes (32 KiB) or 2^13 (64 KiB).  The tile is 2^h
   // contiguous runs of 2^Lc amplitudes (h = targets at or above Lc); 13 bits
@@ -630,6 +638,12 @@ int DispatchMfma(float2* s, unsigned n, const unsigned* qs, const double* m64,
   }
 
   if constexpr (K == 4) {
+    // Small states without a target below qubit 5: twice the waves, each with
+    // half the chain.  12-19 qubits 6.5-6.9 us (lane kernel 6.8-7.3, with
+    // target 5 7.0-7.7), 20 7.8 (7.9-8.5); 22 16.4 (15.3).
+    if (qs[0] >= 5 && n <= 20) {
+      return LaunchBatchesReg<K>(s, n, qs, dfrag, false);
+    }
     LaneGeom g;
     if (!LaneGeometry<float>(n, qs, K, nullptr, 0, 0, g)) {
       return QSIM_HIP_ERR_UNSUPPORTED;

@@ -236,6 +236,20 @@ def test_lane_kernel_far_members(dtype, n, qs, controls, sim):
     assert rel_l2(st.to_numpy(), s) < TOL[dtype]
 
 
+@pytest.mark.parametrize("n", [10, 13, 20, 21])
+def test_four_qubit_gates_around_the_small_state_kernel(n, sim):
+    # complex64 k = 4 without a target below qubit 5: up to 20 qubits 32 groups
+    # a wave, above it the lane kernel (which also takes target 4 at any size).
+    rng = np.random.default_rng(n)
+    for qs in ([5, 6, 7, 8], [6, 7, 8, 9], list(range(n - 4, n)), [4, 6, 7, 9]):
+        m = to_interleaved(random_matrix(4, rng), np.float32)
+        s = random_state(n, rng, np.float32)
+        st = upload(s, n, np.float32)
+        sim.apply_gate(qs, m, st)
+        oracle.apply_gate(n, s, qs, m)
+        assert rel_l2(st.to_numpy(), s) < 1e-6, qs
+
+
 @pytest.mark.parametrize("k", [5, 6])
 @pytest.mark.parametrize("n", [9, 10, 11, 12, 16, 22])
 def test_complex128_wide_gates(n, k, sim):
