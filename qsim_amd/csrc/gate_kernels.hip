@@ -518,12 +518,14 @@ unsigned LaunchExpect(const typename Cplx<FP>::T* s, unsigned n,
     //               k = 3 215 : 237 without a target in the lanes, else
     //               245-286 : 236-245
     //   complex128  k = 1 353-392 : 359-397; k = 2 362-394 : 360-378; k = 3
-    //               440 : 540 with 3 targets in the lanes, 391 : 392 with 1;
+    //               440 : 540 with 3 targets in the lanes, 420 : 395 with 2 (24
+    //               qubits 66 : 59, 29 1621 : 1522), 391 : 392 with 1;
     //               k = 4 543 : 555 without, 593-673 : 555-629 with
+    // The same choices are no more than 3 % behind on 12-30 qubits.
     constexpr bool f32 = sizeof(FP) == 4;
     LaneGeom lg;
     if (LaneGeometry<FP>(n, qs, K, nullptr, 0, 0, lg) &&
-        (K < 3 || (K == 3 && !f32 ? lg.nlow > 1 : lg.nlow == 0))) {
+        (K < 3 || lg.nlow == (K == 3 && !f32 ? 3 : 0))) {
       const uint64_t blocks = std::min<uint64_t>(
           (lg.nchunks + 3) / 4,
           K == 1 && !f32 ? kExpectBlocksFew : kExpectBlocks);
