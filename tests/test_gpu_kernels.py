@@ -287,6 +287,22 @@ def test_expectation_value_vs_oracle(dtype, sim):
                 assert abs(got - ref) < tol, (n, k, qs, got, ref)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_expectation_value_many_chunks(dtype, sim):
+    # 24 qubits: more chunks (lane and MFMA kernels) and groups than one round
+    # of the grid holds, targets in the lanes and above.
+    n, rng = 24, np.random.default_rng(41)
+    s = random_state(n, rng, dtype)
+    st = upload(s, n, dtype)
+    for k in range(1, 5):
+        for qs in (list(range(k)), [6 + 4 * b for b in range(k)],
+                   [2] + [n - k + 1 + b for b in range(k - 1)]):
+            m = to_interleaved(random_matrix(k, rng, unitary=False), dtype)
+            got = sim.expectation_value(qs, m, st)
+            ref = oracle.expectation_value(n, s, qs, m)
+            assert abs(got - ref) < (2e-6 if dtype == np.float32 else 1e-12), qs
+
+
 def test_expectation_value2_known_answer(sim):
     exp = known_answers()["expectation2"]["expected_real"]
     n, ops = expectation2_circuit()
@@ -341,6 +357,39 @@ def test_sample_identical_to_oracle(dtype):
         np.testing.assert_array_equal(got, oracle.sample(n, s, 1000, 5))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [21, 23])
+def test_sample_over_several_spans(n, dtype):
+    # 2 and 8 spans of 1024 sample blocks: the outer prefix sums and their
+    # search.
+    rng = np.random.default_rng(n)
+    ss = qsim_amd.StateSpace(dtype)
+    s = random_state(n, rng, dtype)
+    st = upload(s, n, dtype)
+    draws = oracle.generate_random_values(20000, 9, oracle.serial_norm(n, s))
+    np.testing.assert_array_equal(ss.sample_with_draws(st, draws[:-1]),
+                                  oracle.sample_with_draws(n, s, draws))
+    np.testing.assert_array_equal(ss.sample(st, 1000, 5),
+                                  oracle.sample(n, s, 1000, 5))
+
+
+def test_sample_over_more_spans_than_a_workgroup(ss32):
+    # 29 qubits: 512 spans, two rounds of the outer scan.  Uniform amplitudes:
+    # a draw in the middle of amplitude j finds j.
+    n = 29
+    st = ss32.create(n)
+    ss32.set_state_uniform(st)
+    p = float(np.float32(1 / np.sqrt(1 << n))) ** 2
+    j = np.unique(np.random.default_rng(5).integers(0, 1 << n, 20000))
+    j[[0, -1]] = 0, (1 << n) - 1
+    np.testing.assert_array_equal(ss32.sample_with_draws(st, (j + 0.5) * p), j)
+    draws = oracle.generate_random_values(1000, 3, ss32.norm(st))[:-1] / p
+    got = ss32.sample(st, 1000, 3)
+    far = np.abs(draws - np.round(draws)) > 1e-3
+    np.testing.assert_array_equal(got[far], np.floor(draws)[far])
+    assert far.mean() > 0.9
+
+
 def test_sample_draws_past_the_end(ss32):
     # Draws at or beyond the total map to 2^n - 1 (lib/statespace_basic.h:227-229).
     n = 10
@@ -381,6 +430,85 @@ def test_measurement_vs_oracle(dtype):
         ss.collapse(st, mask, bits)
         oracle.collapse(n, s, mask, bits)
         assert rel_l2(st.to_numpy(), s) < TOL[dtype] * 4
+
+
+def test_measurement_of_a_long_range(ss32):
+    # 23 qubits: ranges of 8192 amplitudes, two narrowing steps of eight loads
+    # in flight.  Amplitudes are whole numbers times 2^-22: squares and sums
+    # are exact, so every index is.
+    n, rng = 23, np.random.default_rng(23)
+    s = np.zeros(2 << n, np.float32)
+    s[0::2] = rng.integers(-2000, 2001, 1 << n) * 2.0**-22
+    st = upload(s, n, np.float32)
+    p = (s[0::2] * s[0::2]).astype(np.float64)
+    pn = ss32.partial_norms(st)
+    part = (1 << n) // len(pn)
+    np.testing.assert_array_equal(pn, p.reshape(-1, part).sum(axis=1))
+    for m in (0, 1, 511, 1023):
+        csum = np.cumsum(p[m * part:(m + 1) * part])
+        for r in rng.uniform(0, csum[-1], 50):
+            k = ss32.find_measured_bits(st, m, r, (1 << n) - 1)
+            assert k == m * part + np.searchsorted(csum, r, side="right")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,mask,bits", [
+    (6, 0b111000, 0b101000), (12, 0b1000, 0b1000), (13, 0b1, 0),
+    (13, 0b1000000000100, 0b100), (16, 0b1011000010001000, 0b11000000001000),
+    (16, 0xffff, 0x1234), (16, 0xfff8, 0x1230), (19, 0x60000, 0x20000),
+    (14, 0b11000, 0b100)])
+def test_collapse_masks(n, mask, bits, dtype):
+    # Measured qubits whose zero half is skipped (from qubit 3, complex128 2),
+    # those that are only tested, both, all; the last wants a bit outside the
+    # mask, which no amplitude has.
+    rng = np.random.default_rng(n)
+    ss = qsim_amd.StateSpace(dtype)
+    s = random_state(n, rng, dtype)
+    st = upload(s, n, dtype)
+    ss.collapse(st, mask, bits)
+    if bits & ~mask:
+        assert not st.to_numpy().any()
+    else:
+        oracle.collapse(n, s, mask, bits)
+        assert rel_l2(st.to_numpy(), s) < TOL[dtype] * 4
+
+
+@pytest.mark.parametrize("n", [14, 18])
+def test_states_aligned_to_an_amplitude(n, sim, ss32):
+    # A complex64 state 8 bytes off a 16-byte boundary, as a caller's buffer
+    # may be: the kernels that load 16 bytes give what they give on it.
+    rng = np.random.default_rng(n)
+    s, t = random_state(n, rng), random_state(n, rng)
+    room = [ss32.create(n + 1) for _ in range(2)]
+    assert all(r.ptr % 16 == 0 for r in room)
+    results = []
+    for shift in (0, 8):
+        a, b = (qsim_amd.State(n, np.float32, ptr=r.ptr + shift, owner=False)
+                for r in room)
+        a.from_numpy(s)
+        b.from_numpy(t)
+        rng = np.random.default_rng(1)
+        out = [ss32.norm(a), ss32.inner_product(a, b), ss32.partial_norms(a),
+               ss32.sample(a, 1000, 2)]
+        for tb in (9, 13, 14):
+            tile = list(range(4)) + list(range(n - tb + 4, n))
+            gates = []
+            for k in (1, 2, 3, 4, 4):
+                qs = sorted(rng.choice(tile, k, replace=False).tolist())
+                gates.append((qs, to_interleaved(random_matrix(k, rng),
+                                                 np.float64)))
+            sim.apply_gate_block(tile, gates, a)
+        for k in (1, 2, 3, 4, 5, 6):
+            for qs in (list(range(k)), list(range(n - k, n))):
+                m = to_interleaved(random_matrix(k, rng), np.float32)
+                sim.apply_gate(qs, m, a)
+                out.append(sim.expectation_value(qs, m, a))
+        out.append(a.to_numpy())
+        ss32.collapse(a, 0b1010010, 0b10)
+        out += [a.to_numpy(), b.to_numpy()]
+        results.append(out)
+    for x, y in zip(*results):
+        np.testing.assert_array_equal(x, y)
 
 
 @pytest.mark.parametrize("n,run", [(18, 64), (24, 64), (24, 1024)])

@@ -170,6 +170,85 @@ def random_batch(sizes, tile_bits, rng):
     return b
 
 
+def apply(psi, n, qs, m):
+    """m, row and column bit j on qubit qs[j], over psi in FP64."""
+    k = len(qs)
+    axes = [n - 1 - q for q in reversed(qs)]
+    v = np.moveaxis(psi.reshape((2,) * n), axes, range(k))
+    v = (m @ v.reshape(1 << k, -1)).reshape((2,) * n)
+    return np.moveaxis(v, range(k), axes).reshape(-1)
+
+
+def replay(b):
+    """The batch's streams in FP64 numpy: pair values, choices, states."""
+    mats = np.concatenate(b.mats).astype(np.float64)
+
+    def mat(off, k):
+        m = mats[off:off + (2 << 2 * k)].reshape(1 << k, 1 << k, 2)
+        return m[..., 0] + 1j * m[..., 1]
+
+    zz, dec, states = [], np.full(b.slots, -1, np.int32), []
+    for n, num_pairs, _, begin, end, first_pair, normalise in b.descs:
+        psi = np.zeros(1 << n, np.complex128)
+        psi[0] = 1
+        i = begin
+        while i < end:
+            o = b.ops[i]
+            k = int(o["k"])
+            if o["kind"] == GATE:
+                psi = apply(psi, n, o["q"][:k].tolist(), mat(int(o["moff"]), k))
+            elif o["kind"] == CHANNEL:
+                # lib/qtrajectory.h:330-370: the non-unitary operators in
+                # turn until the draw falls below the running sum.
+                nq = int(o["moff2"])
+                norm = np.vdot(psi, psi).real if o["pad"] & 1 else 1.0
+                cp, best, at, pick = float(o["cp"]), 0.0, 0, -1
+                for j in range(k):
+                    c = b.ops[i + 1 + j]
+                    if c["pad"] & 1:
+                        continue
+                    kk = apply(psi, n, o["q"][:nq].tolist(),
+                               mat(int(c["moff2"]), nq))
+                    prob = np.vdot(psi, kk).real / norm
+                    if prob > best:
+                        best, at = prob, j
+                    cp += prob - float(c["r"])
+                    if o["r"] < cp or j == k - 1:
+                        pick = j if o["r"] < cp else at
+                        break
+                dec[o["slot"]] = pick
+                if pick >= 0 and b.ops[i + 1 + pick]["k"]:
+                    c = b.ops[i + 1 + pick]
+                    ck = int(c["k"])
+                    psi = apply(psi, n, c["q"][:ck].tolist(),
+                                mat(int(c["moff"]), ck))
+                psi = psi / np.sqrt(norm)
+                i += k
+            i += 1
+        p = np.abs(psi) ** 2
+        idx = np.arange(1 << n)
+        for qa, qb in b.pairs[first_pair:first_pair + num_pairs]:
+            sign = 1 - 2 * (((idx >> qa) ^ (idx >> qb)) & 1)
+            zz.append((p * sign).sum() / p.sum())
+        if normalise:
+            psi = psi / np.sqrt(p.sum())
+        states.append(np.stack([psi.real, psi.imag], 1).reshape(-1))
+    return np.array(zz), dec, states
+
+
+@pytest.mark.parametrize("threads", [256, 1024, TILED])
+@pytest.mark.parametrize("tile_bits,sizes", [
+    (14, [17, 14, 9, 4]), (13, [15, 13, 11, 10]), (10, [12, 10, 6])])
+def test_batch_matches_numpy(tile_bits, sizes, threads):
+    b = random_batch(sizes, tile_bits, np.random.default_rng(sum(sizes)))
+    zz, dec, states = replay(b)
+    zt, dt, st = b.run(threads)
+    np.testing.assert_array_equal(dt, dec)
+    np.testing.assert_allclose(zt, zz, atol=1e-5, rtol=0)
+    for n, x, y in zip(sizes, st, states):
+        assert np.linalg.norm(x - y) < 1e-5, n
+
+
 @pytest.mark.parametrize("tile_bits,sizes", [
     (14, [18, 17, 16, 15, 14, 13, 10, 9, 6, 4]),
     (13, [17, 15, 14, 13, 12, 9, 8]),
