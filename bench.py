@@ -85,7 +85,8 @@ SWEEP_PATHS = [f"fp32-k{k}" for k in range(2, 7)]
 
 # HBM bytes per amplitude per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE
 # runs, scaled by what the counters read for a copy of known size (reads x 2,
-# writes x 1); profiles/gate_passes_32q_blocked_vs_fused.md.
+# writes x 1); profiles/gate_passes_32q_blocked_vs_fused.md ("The 14-qubit pass
+# with IO waves" for GateBlockF16IoKernel).
 MEASURED_HBM_BYTES_PER_AMP = {"GateBlockF16IoKernel": 16.00,
                               "GateBlockKernel": 16.04}
 

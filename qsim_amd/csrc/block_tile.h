@@ -689,10 +689,11 @@ struct TileIo {
 // exchange, which nothing overlaps, moves bits unchanged) and on the way out
 // by the stores.
 //
-// Bound by the HBM stream up to 5 ops, then by the ops (about 2.1 ms each:
-// LDS reads and writes of the whole tile, the fp16 split and the MFMA chain
-// in sequence).  32 qubits, tiles of 4 low and 10 random higher qubits, 1 / 3
-// / 5 / 7 ops: 15.4-16.0 / 15.4-15.9 / 16.0-16.2 / 20.3-20.4 ms, against
+// Bound by the HBM stream up to 4 ops; the ops take as long at 5, and each
+// further one 2.1 ms more (LDS reads and writes of the whole tile, the fp16
+// split and the MFMA chain in sequence).  32 qubits, tiles of 4 low and 10
+// random higher qubits, 1 / 3
+// / 5 / 7 ops: 13.3-16.0 / 13.5-16.0 / 16.0-16.6 / 20.3-20.9 ms, against
 // 16.3 / 16.0-17.5 / 18.7-20.1 / 23.2-24.2 with every wave doing both.  The
 // 64 KiB shape has two workgroups a CU, which hide each other's phases, and
 // keeps that structure.

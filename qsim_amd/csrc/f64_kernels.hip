@@ -12,15 +12,18 @@
 // qubits, so runs of 32 or more amplitudes whatever the targets.  A 256-thread
 // workgroup copies a set to LDS; wave w computes 16-row blocks w, w + 4, ...
 // (their rows of A stay in its registers for the whole pass) for every group
-// of the set; the results go back to their slots and the set is copied out,
-// with the next set's loads in flight in registers meanwhile.  Four (k = 5)
-// or two workgroups share a CU.
+// of the set; the results go back to their slots and the set is copied out.
+// The next set is loaded before the product, but the compiler holds it in
+// scratch memory (80 / 144 bytes a lane) and waits for it there, so its latency
+// is one of the phases.  Four (k = 5) or two workgroups share a CU.
 //
 // The vector kernels need a group per thread: 2^k amplitudes of 16 bytes in
 // registers, and half (k = 5) or a quarter (k = 6) of the tile kernel's
 // threads have one.  27 qubits: k = 6 1.65-1.83 ms (10.5 with high targets,
 // 29-34 in tiles; the FP64 MFMA rate allows 0.95), k = 5 1.09-1.38 ms (3.4-3.7
-// in tiles); the phases between a set's barriers bound both.  k = 5 with every
+// in tiles); the phases between a set's barriers bound both.  On 12-28 qubits
+// k = 6 takes 0.03-0.20 of the vector kernels' time, k = 5 with a low target
+// 0.2-0.4.  k = 5 with every
 // target at qubit >= 5 stays on the vector kernel, which keeps a group per
 // thread without LDS there: 0.92-1.08 ms against 1.27-1.38.
 
