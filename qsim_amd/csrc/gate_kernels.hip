@@ -10,8 +10,8 @@
 //    bits by swaps across lanes.  No LDS, no barriers.
 //  * GateRegKernel  -- all targets and controls at qubit >= 5 (not k = 4):
 //    one group per work item, held in registers.
-//  * GateTileKernel -- the rest (k = 5, 6 with a qubit below 5, and small
-//    states).  A workgroup stages a tile of 2^tb amplitudes (the Lc lowest
+//  * GateTileKernel -- the rest (k = 5, 6 with a qubit below 5, small states,
+//    far-apart k = 2 with a low control).  A workgroup stages a tile of 2^tb amplitudes (the Lc lowest
 //    qubits, contiguous in memory, times the high targets) in LDS with
 //    coalesced loads, applies the groups from LDS and streams the tile back.
 //
@@ -380,8 +380,18 @@ int DispatchK(typename Cplx<FP>::T* s, unsigned n, const unsigned* qs,
     // for k = 1.  With controls, complex128 is 2-5 % better on the lanes (27
     // qubits 191-210 : 187-198), and k = 4 too (20 qubits 26 : 16).
     const bool reg = lowest >= 5 && K <= 3 && (nc == 0 || sizeof(FP) == 4);
+    // complex64 k = 2 with a control below a half line and both targets from
+    // qubit 14 up stays on the tile kernel, whose runs are of 2^11 amplitudes,
+    // from 28 qubits: there the lane kernel takes 0.89-1.21 times its time on
+    // random sets, 1.04 on average (27 qubits 0.90-1.14, 0.99; with a target
+    // below 14 0.76-1.02, 0.89).  Not with controls inside the tile's run
+    // that the lane kernel skips (twice the traffic).
+    bool tile = K == 2 && sizeof(FP) == 4 && n >= 28 && nc > 0 &&
+                cqs[0] < 3 && qs[0] >= 14;
+    for (unsigned i = 0; i < nc; ++i)
+      tile = tile && (cqs[i] < 3 || cqs[i] >= 13);
     LaneGeom lg;
-    if (!reg && LaneGeometry<FP>(n, qs, K, cqs, nc, cvals, lg)) {
+    if (!reg && !tile && LaneGeometry<FP>(n, qs, K, cqs, nc, cvals, lg)) {
       if constexpr (byval) return LaunchLane<FP, K>(s, lg, mv);
       else return LaunchLane<FP, K>(s, lg, mp);
     }

@@ -143,8 +143,8 @@ __device__ __forceinline__ void SwapLowTargets(C (&v)[1 << K],
 // Gates without targets in the lanes: k = 4 with members 4 MiB apart or more,
 // and complex64 k = 2 with a control in the lanes.  Random sets of targets on
 // 26-30 qubits, runs of 32 against workgroups in order: complex64 k = 4 2 %
-// less on average, 40 % at most, 6 % more at worst; complex128 k = 4 4 %, 29 %,
-// 8 %; complex64 k = 2 6 %, 27 %, 7 %.  With every set of k = 4 the worst is 16
+// less on average, 38 % at most, 6 % more at worst; complex128 k = 4 3 %, 34 %,
+// 8 %; complex64 k = 2 6 %, 31 %, 7 %.  With every set of k = 4 the worst is 16
 // % more, and complex128 k <= 3 have 20 %.
 template <typename FP, int K>
 inline bool LaneFar(const LaneGeom& g) {

@@ -236,6 +236,27 @@ def test_lane_kernel_far_members(dtype, n, qs, controls, sim):
     assert rel_l2(st.to_numpy(), s) < TOL[dtype]
 
 
+@pytest.mark.parametrize("qs,controls", [([16, 27], [1]), ([17, 24], [0, 2]),
+                                         ([13, 24], [2]), ([14, 27], [2, 20]),
+                                         ([14, 27], [2, 12])])
+def test_two_far_targets_with_a_low_control(qs, controls, sim, ss32):
+    # 28 qubits, both sides of the line between the tile and the lane kernel.
+    # Uniform amplitudes: each target pattern gets its row sum.
+    n, rng = 28, np.random.default_rng(28)
+    u = random_matrix(2, rng, unitary=False)
+    st = ss32.create(n)
+    ss32.set_state_uniform(st)
+    cvals = (1 << len(controls)) - 2
+    sim.apply_controlled_gate(qs, controls, cvals, to_interleaved(u, np.float32),
+                              st)
+    a = float(np.float32(2.0**-14))
+    for i in rng.integers(0, 1 << n, 3000).tolist():
+        want = a
+        if all((i >> c) & 1 == (cvals >> b) & 1 for b, c in enumerate(controls)):
+            want = a * u[((i >> qs[0]) & 1) | ((i >> qs[1]) & 1) << 1].sum()
+        assert abs(ss32.get_ampl(st, i) - want) < 1e-6 * a * 4, i
+
+
 @pytest.mark.parametrize("n", [10, 13, 20, 21])
 def test_four_qubit_gates_around_the_small_state_kernel(n, sim):
     # complex64 k = 4 without a target below qubit 5: up to 20 qubits 32 groups
