@@ -438,7 +438,8 @@ int qsim_hip_traj_prepare(const qsim_hip_traj_desc* trajs, unsigned num_traj,
 /* Runs the whole batch: one launch with `threads` (256, 512 or 1024) per
  * trajectory, or the tiled batch's launches (QSIM_HIP_TRAJ_TILED); with
  * use_graph they are captured once in a hipGraph and replayed after.
- * Waits for completion. */
+ * Streams without tile passes get the tiled batch's launches (and a little
+ * device memory for them) at their first tiled run.  Waits for completion. */
 int qsim_hip_traj_run(void* handle, unsigned threads, int use_graph);
 /* <Z_a Z_b> of every pair (FP64, pair order of the batch) and the decision
  * record (the chosen Kraus operator's index in its channel; -1: none chosen

@@ -11,9 +11,10 @@
 //  * GateRegKernel  -- all targets and controls at qubit >= 5 (not k = 4):
 //    one group per work item, held in registers.
 //  * GateTileKernel -- the rest (k = 5, 6 with a qubit below 5, small states,
-//    far-apart k = 2 with a low control).  A workgroup stages a tile of 2^tb amplitudes (the Lc lowest
-//    qubits, contiguous in memory, times the high targets) in LDS with
-//    coalesced loads, applies the groups from LDS and streams the tile back.
+//    far-apart k = 2 with a low control).  A workgroup stages a tile of 2^tb
+//    amplitudes (the Lc lowest qubits, contiguous in memory, times the high
+//    targets) in LDS with coalesced loads, applies the groups from LDS and
+//    streams the tile back.
 //
 // The gate matrix (row-major, row/column bit j <-> qs[j]) travels by value in
 // the kernel arguments when it fits in 2 KiB (scalar loads, uniform across the
