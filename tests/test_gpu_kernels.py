@@ -5,6 +5,9 @@ circuits) of the oracle's FP32 result, complex128 within 1e-12; sampled
 bitstrings and measured bits identical for identical draws.
 """
 
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -409,6 +412,32 @@ def test_sample_over_more_spans_than_a_workgroup(ss32):
     far = np.abs(draws - np.round(draws)) > 1e-3
     np.testing.assert_array_equal(got[far], np.floor(draws)[far])
     assert far.mean() > 0.9
+
+
+def test_long_sampling_leaves_other_threads_their_turn(ss32):
+    # 30 million draws take about a second of host time; norms on another
+    # thread do not wait for them.
+    n, num = 10, 30_000_000
+    s = random_state(n, np.random.default_rng(6))
+    st = upload(s, n, np.float32)
+    took = []
+
+    def sample():
+        t = time.perf_counter()
+        bits = ss32.sample(st, num, 4)
+        took.append(time.perf_counter() - t)
+        took.append(np.bincount(bits.astype(np.int64), minlength=1 << n))
+    th = threading.Thread(target=sample)
+    th.start()
+    longest = 0.0
+    while th.is_alive():
+        t = time.perf_counter()
+        ss32.norm(st)
+        longest = max(longest, time.perf_counter() - t)
+    th.join()
+    assert longest < 0.5 * took[0], (longest, took[0])
+    p = np.abs(from_interleaved(s)) ** 2
+    assert np.abs(took[1] / num - p / p.sum()).max() < 6 * np.sqrt(p.max() / num)
 
 
 def test_sample_draws_past_the_end(ss32):
